@@ -41,3 +41,51 @@ def test_dense_inverse_tile_edges(ctx, n):
     assert st.converged and st.coarse_unknowns == 2 * n * n
     assert st.iters <= 24
     assert nrel(d, spla.spsolve(H.tocsc(), g)) <= 1e-9
+
+
+def quadratic_chain(d, n, seed=0):
+    """Quadratic elements on the handle pairs (i, i + 1) and (i, i + 5), permuted
+    handles, the last handle in no element; every element Hessian has its
+    spectrum in [1, 3]."""
+    rng = np.random.default_rng(seed)
+    perm = rng.permutation(n)
+    pairs = [(i, i + 1) for i in range(n - 2)] + [(i, i + 5) for i in range(n - 6)]
+    conn = perm[np.array(pairs, dtype=np.int64).reshape(-1, 2)].astype(np.int32)
+    K = 2 * d
+    Q = np.linalg.qr(rng.normal(size=(conn.shape[0], K, K)))[0]
+    A = np.einsum("eik,ek,ejk->eij", Q, rng.uniform(1.0, 3.0, (conn.shape[0], K)), Q)
+    A = 0.5 * (A + A.transpose(0, 2, 1))
+    params = np.concatenate([A.reshape(-1, K * K), np.zeros((conn.shape[0], K + 1))], axis=1)
+    return configs.Problem("quadratic_chain", d, n, [configs.Term(configs.E_QUADRATIC, conn, params)],
+                           rng.normal(size=d * n))
+
+
+# handles around the update kernel's chunks of 64 and the product's groups of
+# 32 rows; aggregates smaller than, equal to and larger than a chunk, and off
+@pytest.mark.parametrize("d", [1, 2, 3])
+@pytest.mark.parametrize("n", [3, 33, 64, 65, 200, 700])
+@pytest.mark.parametrize("agg", [0, 3, 64, 150])
+def test_solver_order_edges(ctx, d, n, agg):
+    """Solves in solver order (aggregates, parts, chunks; a handle without
+    elements; a free-variable mask) against direct solves of w I + H.  The
+    condition number is at most 40 (element spectra in [1, 3], at most four
+    elements per handle, w = 0.3), so a relative residual of 1e-13 bounds the
+    solution error by 4e-12."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as spla
+    fn = tad.ScalarFunction.from_problem(quadratic_chain(d, n), ctx)
+    rng = np.random.default_rng(n)
+    _, _, H = fn.eval_with_derivatives(rng.normal(size=d * n))
+    A = (H + 0.3 * sp.identity(d * n)).tocsc()
+    b = rng.normal(size=d * n)
+    x, st = fn.solve(b, tol=1e-13, w_identity=0.3, coarse_aggregate=agg)
+    assert st.converged and nrel(x, spla.spsolve(A, b)) <= 1e-10
+    free = (rng.random(d * n) < 0.7).astype(np.uint8)
+    free[0] = 1
+    fi = np.nonzero(free)[0]
+    ref = np.zeros(d * n)
+    ref[fi] = np.atleast_1d(spla.spsolve(A[fi][:, fi].tocsc(), b[fi]))
+    x, st = fn.solve(b, free=free, tol=1e-13, w_identity=0.3, coarse_aggregate=agg)
+    assert st.converged and nrel(x, ref) <= 1e-10 and np.all(x[free == 0] == 0.0)
+    x2, st2 = fn.solve(b, free=free, tol=1e-13, w_identity=0.3, coarse_aggregate=agg)
+    assert np.array_equal(x, x2) and st.iters == st2.iters

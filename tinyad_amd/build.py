@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(ROOT, "_build")
 LIB = os.path.join(HERE, "libtinyad_amd.so")
 SOURCES = ["tad_element.hip", "tad_energy.hip", "tad_linalg.hip", "tad_dense.hip", "tad_basis.hip", "tad_adjoint.hip", "tad_api.cpp"]
-HEADERS = ["tad_energies.hpp", "tad_elements.hpp", "tad_internal.hpp"]
+HEADERS = ["tad_energies.hpp", "tad_elements.hpp", "tad_internal.hpp", "tad_wave.hpp"]
 # public headers the library's sources also compile (device code shared with
 # element kernels built from user energies)
 PUBLIC_HEADERS = ["tinyad_amd.h", "tinyad_amd/device/Dual.hpp", "tinyad_amd/device/Projection.hpp",

@@ -218,6 +218,23 @@ struct HostTerm
     }
 };
 
+// An order of the handles for the solver (entry i is handle perm[i]) with the
+// block pattern in that order, the stored lower-triangle blocks and where
+// each comes from in H, and the update kernel's parts (PcgSystem).
+struct SolverOrder
+{
+    bool ready = false;
+    int64_t n_sym = 0;
+    int Gs = 0, Gv = 0, ppa = 1;
+    DevBuf<int32_t> perm, brow_ptr, bcol, sym_ptr, usrc, diag, place, part_ptr;
+    void release()
+    {
+        perm.release(); brow_ptr.release(); bcol.release(); sym_ptr.release(); usrc.release(); diag.release();
+        place.release(); part_ptr.release();
+        ready = false;
+    }
+};
+
 struct tad_fn_s
 {
     tad_ctx ctx = nullptr;
@@ -247,14 +264,11 @@ struct tad_fn_s
     int64_t n_upper = 0;
     DevBuf<int64_t> uslot_ptr;
     DevBuf<int32_t> uplace;        // 4 per upper block
-    // the solver's copy of H: the lower triangle's blocks (diagonal included)
-    // in CSR order, D*D contiguous values each, the triangle the reference's
-    // SimplicialLDLT reads (LinearSolver.hh:14); per CSR block the stored
-    // block it reads (its own ordinal, or ~ordinal of its mirrored lower block)
-    DevBuf<int32_t> sym_full;      // per stored block: its CSR block
-    DevBuf<int32_t> sym_src;       // per CSR block
-    DevBuf<double> sym_H;          // n_sym * D * D
-    int64_t n_sym = 0;
+    // the solver's copy of H (its lower triangle's blocks in solver order, the
+    // triangle the reference's SimplicialLDLT reads, LinearSolver.hh:14) for
+    // solves without a coarse space: handle order
+    SolverOrder natural;
+    DevBuf<double> sym_H;          // stored blocks of the order in use
     int asm_shape = 0;             // Hessian assembly launch shape (tad_fn_autotune)
     std::vector<int32_t> h_brow_ptr, h_bcol;  // host copy of the block pattern (coarse aggregation)
     std::vector<int64_t> h_urow_ptr;          // first upper block of each block row (host)
@@ -275,7 +289,8 @@ struct tad_fn_s
     // line search
     DevBuf<double> ls_f, x_tmp;
     // solver
-    DevBuf<double> Dinv, r, z, p, q, sol;
+    DevBuf<double> Dinv, xs, r, z, p, q, sol;  // xs: the iterate in solver order
+    DevBuf<unsigned char> free_s;              // free-variable mask in solver order
     DevBuf<PcgScalars> scal;
     DevBuf<double> pcg_parts;
     bool h_valid = false;
@@ -292,11 +307,11 @@ struct tad_fn_s
     {
         int requested = 0;            // aggregate size asked for when the pattern was built (0: none)
         int target = 0;               // aggregate size the pattern was built with
-        int64_t n_agg = 0, n_pairs = 0, n_chunks = 0, n_gchunks = 0;
-        int max_agg_chunks = 0;
-        DevBuf<int32_t> agg_of, agg_ptr, agg_vert, pair_blocks, pair_ab, chunk_ptr, agg_chunk, pair_chunk;
+        int64_t n_agg = 0, n_pairs = 0, n_gchunks = 0;
+        SolverOrder ord;              // aggregate after aggregate, members ascending
+        DevBuf<int32_t> agg_of, agg_ptr, pair_blocks, pair_ab, pair_chunk;
         DevBuf<int64_t> gchunk_ptr;
-        DevBuf<double> dvec, Ac, rc, cparts, chunk_part, gpart, inv_work, rowsum;
+        DevBuf<double> dvec, dvec_h, Ac, rpart, cparts, gpart, inv_work, rowsum;
         DevBuf<float> Ainv32;  // the inverse in FP32 with a diagonal shift, read by every CG iteration
         bool use32 = false;    // Ainv32 belongs to the current factor
         DevBuf<int> info;
@@ -308,13 +323,13 @@ struct tad_fn_s
         double f_w = 0.0;
         void release()
         {
-            agg_of.release(); agg_ptr.release(); agg_vert.release(); pair_blocks.release(); pair_ab.release();
-            chunk_ptr.release(); agg_chunk.release(); pair_chunk.release(); gchunk_ptr.release();
-            dvec.release(); Ac.release(); rc.release(); cparts.release(); chunk_part.release();
+            ord.release();
+            agg_of.release(); agg_ptr.release(); pair_blocks.release(); pair_ab.release();
+            pair_chunk.release(); gchunk_ptr.release();
+            dvec.release(); dvec_h.release(); Ac.release(); rpart.release(); cparts.release();
             gpart.release(); inv_work.release(); rowsum.release(); Ainv32.release(); info.release();
             requested = target = 0;
-            n_agg = n_pairs = n_chunks = n_gchunks = 0;
-            max_agg_chunks = 0;
+            n_agg = n_pairs = n_gchunks = 0;
             factor_valid = false;
         }
     } co;
@@ -367,7 +382,7 @@ void free_pattern(tad_fn fn)
     fn->brow_ptr.release(); fn->bcol.release(); fn->block_row.release(); fn->diag_block.release();
     fn->row_ptr.release(); fn->col_idx.release(); fn->hslot_ptr.release(); fn->gslot_ptr.release();
     fn->block_mirror.release(); fn->uslot_ptr.release(); fn->uplace.release();
-    fn->sym_full.release(); fn->sym_src.release(); fn->sym_H.release();
+    fn->natural.release(); fn->sym_H.release();
     fn->co.release();
     fn->h_brow_ptr.clear(); fn->h_bcol.clear(); fn->h_urow_ptr.clear();
     fn->pipe_ready = false;
@@ -557,38 +572,6 @@ tad_status build_pattern(tad_fn fn)
     for (int64_t u = 0; u < nh; ++u)
         for (int32_t k = brow_ptr[u]; k < brow_ptr[u + 1]; ++k)
             mirror[k] = bcol[k] >= u ? k : (int32_t)find_block(bcol[k], (int32_t)u);
-    // the solver's lower-triangle copy: ordinals of the lower blocks, and per
-    // block the stored block it reads, checked against the pattern (mirror
-    // maps each lower block to its upper block; lower_of inverts it)
-    std::vector<int32_t> sym_full, sym_src(nb);
-    {
-        std::vector<int32_t> ord(nb, -1), lower_of(nb, -1);
-        for (int64_t u = 0; u < nh; ++u)
-            for (int32_t k = brow_ptr[u]; k < brow_ptr[u + 1]; ++k)
-                if (bcol[k] <= u)
-                {
-                    ord[k] = (int32_t)sym_full.size();
-                    sym_full.push_back(k);
-                    const int32_t m = mirror[k];
-                    const bool ok = bcol[k] == u ? (m == k)
-                                                 : (m >= 0 && m < nb && block_row[m] == bcol[k] &&
-                                                    bcol[m] == (int32_t)u && lower_of[m] < 0);
-                    if (!ok) return fail(TAD_ERR_UNSUPPORTED, "Hessian mirror map inconsistent");
-                    lower_of[m] = k;
-                }
-        for (int64_t u = 0; u < nh; ++u)
-            for (int32_t k = brow_ptr[u]; k < brow_ptr[u + 1]; ++k)
-            {
-                if (bcol[k] <= u)
-                {
-                    sym_src[k] = ord[k];
-                    continue;
-                }
-                const int32_t l = lower_of[k];
-                if (l < 0 || ord[l] < 0) return fail(TAD_ERR_UNSUPPORTED, "Hessian pattern not symmetric");
-                sym_src[k] = ~ord[l];
-            }
-    }
     std::vector<std::vector<uint32_t>> gpos(nterms), hpos(nterms), gout(nterms);
     {
         std::vector<int64_t> hc(hptr.begin(), hptr.end() - 1), gc(gptr.begin(), gptr.end() - 1);
@@ -716,8 +699,6 @@ tad_status build_pattern(tad_fn fn)
     TAD_HIP(up(fn->block_mirror, mirror));
     TAD_HIP(up(fn->uslot_ptr, uptr));
     TAD_HIP(up(fn->uplace, uplace));
-    TAD_HIP(up(fn->sym_full, sym_full));
-    TAD_HIP(up(fn->sym_src, sym_src));
     for (size_t ti = 0; ti < fn->terms.size(); ++ti)
     {
         TermDev& td = fn->terms[ti];
@@ -754,9 +735,140 @@ tad_status build_pattern(tad_fn fn)
     fn->n_gslots = gptr[nh];
     fn->n_blocks = nb;
     fn->n_upper = (int64_t)uptr.size() - 1;
-    fn->n_sym = (int64_t)sym_full.size();
     fn->nnz = nnz;
     fn->pattern_ready = true;
+    return TAD_OK;
+}
+
+// The solver's pattern and copy map for the handle order `perm` (a
+// permutation of the handles); agg_ptr: entries of each aggregate (empty: no
+// aggregates).  Rows list their columns ascending in solver order; stored
+// blocks are those with column <= row, row after row, and each is taken from
+// H's lower triangle (the transpose of block (v, u) where the order swaps the
+// two handles).
+tad_status build_order(tad_fn fn, const std::vector<int32_t>& perm, const std::vector<int32_t>& agg_ptr,
+                       SolverOrder& od)
+{
+    const int d = fn->d;
+    const int64_t nh = fn->n_handles;
+    // a function without elements has no pattern: empty rows
+    const std::vector<int32_t> none(fn->h_brow_ptr.empty() ? nh + 1 : 0, 0);
+    const std::vector<int32_t>& rp = fn->h_brow_ptr.empty() ? none : fn->h_brow_ptr;
+    const std::vector<int32_t>& cb = fn->h_bcol;
+    const int64_t nb = (int64_t)cb.size();
+    std::vector<int32_t> pos(nh, -1);
+    for (int64_t i = 0; i < nh; ++i) pos[perm[i]] = (int32_t)i;
+    std::vector<int32_t> brow_ptr(nh + 1, 0), bcol(nb), sym_ptr(nh + 1, 0), usrc, diag(nh, -1), place;
+    place.reserve((size_t)(nb + nh));
+    std::vector<std::pair<int32_t, int32_t>> row;  // (column in solver order, CSR block)
+    std::vector<int32_t> next(nh);                 // next upper entry of each row to be matched
+    usrc.reserve((size_t)nb / 2 + 1);
+    int32_t n_sym = 0;
+    for (int64_t i = 0; i < nh; ++i)
+    {
+        const int32_t u = perm[i];
+        row.clear();
+        for (int32_t k = rp[u]; k < rp[u + 1]; ++k) row.emplace_back(pos[cb[k]], k);
+        std::sort(row.begin(), row.end());
+        const int32_t b0 = brow_ptr[i];
+        brow_ptr[i + 1] = b0 + (int32_t)row.size();
+        next[i] = brow_ptr[i + 1];
+        for (size_t m = 0; m < row.size(); ++m)
+        {
+            const int32_t j = row[m].first, b = b0 + (int32_t)m;
+            bcol[b] = j;
+            if (j > i)
+            {
+                next[i] = std::min(next[i], b);
+                usrc.push_back(-1);
+                continue;
+            }
+            // stored block (i, j): H's lower block of the two handles
+            const int32_t v = perm[j];
+            int32_t k = row[m].second, h = u;
+            int flags = 0;
+            if (v > u)
+            {
+                const auto lo = cb.begin() + rp[v], hi = cb.begin() + rp[v + 1];
+                const auto it = std::lower_bound(lo, hi, u);
+                if (it == hi || *it != u) return fail(TAD_ERR_UNSUPPORTED, "Hessian pattern not symmetric");
+                k = (int32_t)(it - cb.begin());
+                h = v;
+                flags = 1;
+            }
+            if (j == i)
+            {
+                flags = 2;
+                diag[i] = n_sym;
+            }
+            else
+            {
+                // its mirror: rows i come in ascending order, so row j's
+                // upper entries are matched one after the other
+                const int32_t t = next[j]++;
+                if (t >= brow_ptr[j + 1] || bcol[t] != (int32_t)i)
+                    return fail(TAD_ERR_UNSUPPORTED, "Hessian pattern not symmetric");
+                // upper entries before it: all entries before it less the
+                // stored ones of its row and the rows above
+                usrc[t - sym_ptr[j + 1]] = n_sym;
+            }
+            ++n_sym;
+            // rows d h .. d h + d - 1 of H are consecutive, d * (blocks of row h) values each
+            const int64_t nbh = rp[h + 1] - rp[h];
+            const int64_t off = (int64_t)d * d * rp[h] + (int64_t)d * (k - rp[h]);
+            const int64_t code = 4 * (int64_t)d * nbh + flags;
+            if (code > INT32_MAX) return fail(TAD_ERR_UNSUPPORTED, "block row too long");
+            place.push_back((int32_t)off);
+            place.push_back((int32_t)code);
+        }
+        sym_ptr[i + 1] = n_sym;
+    }
+    for (int64_t i = 0; i < nh; ++i)
+        if (next[i] != brow_ptr[i + 1]) return fail(TAD_ERR_UNSUPPORTED, "Hessian pattern not symmetric");
+    // update parts: whole chunks of kPcgPartVerts entries without aggregates;
+    // otherwise every aggregate in the same number of nearly equal parts, as
+    // many as fill the chip but none with less than a chunk
+    std::vector<int32_t> part_ptr(1, 0);
+    od.ppa = 1;
+    if (agg_ptr.empty())
+    {
+        const int64_t chunks = std::max<int64_t>(1, (nh + kPcgPartVerts - 1) / kPcgPartVerts);
+        const int64_t per = (chunks + kPcgMaxParts - 1) / kPcgMaxParts * kPcgPartVerts;
+        for (int64_t o = per; o < nh; o += per) part_ptr.push_back((int32_t)o);
+        part_ptr.push_back((int32_t)nh);
+    }
+    else
+    {
+        const int64_t n_agg = (int64_t)agg_ptr.size() - 1;
+        int32_t most = 1;
+        for (int64_t a = 0; a < n_agg; ++a) most = std::max(most, agg_ptr[a + 1] - agg_ptr[a]);
+        od.ppa = (int)std::max<int64_t>(1, std::min<int64_t>((most + kPcgPartVerts - 1) / kPcgPartVerts,
+                                                             kPcgMaxParts / std::max<int64_t>(1, n_agg)));
+        for (int64_t a = 0; a < n_agg; ++a)
+        {
+            const int64_t size = agg_ptr[a + 1] - agg_ptr[a], per = (size + od.ppa - 1) / od.ppa;
+            for (int p = 1; p <= od.ppa; ++p) part_ptr.push_back(agg_ptr[a] + (int32_t)std::min(size, p * per));
+        }
+    }
+    od.Gv = (int)part_ptr.size() - 1;
+    od.Gs = pcg_spmv_groups(nh);
+    od.n_sym = n_sym;
+    hipStream_t s = fn->s();
+    auto up = [&](DevBuf<int32_t>& buf, const std::vector<int32_t>& vec) -> hipError_t {
+        hipError_t e = buf.ensure(vec.size());
+        if (e != hipSuccess || vec.empty()) return e;
+        return hipMemcpyAsync(buf.p, vec.data(), vec.size() * sizeof(vec[0]), hipMemcpyHostToDevice, s);
+    };
+    TAD_HIP(up(od.perm, perm));
+    TAD_HIP(up(od.brow_ptr, brow_ptr));
+    TAD_HIP(up(od.bcol, bcol));
+    TAD_HIP(up(od.sym_ptr, sym_ptr));
+    TAD_HIP(up(od.usrc, usrc));
+    TAD_HIP(up(od.diag, diag));
+    TAD_HIP(up(od.place, place));
+    TAD_HIP(up(od.part_ptr, part_ptr));
+    TAD_HIP(hipStreamSynchronize(s));
+    od.ready = true;
     return TAD_OK;
 }
 
@@ -858,15 +970,7 @@ tad_status build_coarse(tad_fn fn, int target)
         pair_blocks[i] = keyed[i].second;
     }
     pair_ptr.push_back(nb);
-    // chunks of at most kCoarseChunk handles / fine blocks (parallel sums)
-    std::vector<int32_t> chunk_ptr, agg_chunk(nn + 1, 0);
-    for (int32_t a = 0; a < nn; ++a)
-    {
-        agg_chunk[a] = (int32_t)chunk_ptr.size();
-        for (int32_t o = agg_ptr[a]; o < agg_ptr[a + 1]; o += kCoarseChunk) chunk_ptr.push_back(o);
-    }
-    agg_chunk[nn] = (int32_t)chunk_ptr.size();
-    chunk_ptr.push_back((int32_t)nh);
+    // chunks of at most kCoarseChunk fine blocks (parallel sums)
     const int64_t n_pairs = (int64_t)pair_ab.size() / 2;
     std::vector<int64_t> gchunk_ptr;
     std::vector<int32_t> pair_chunk(n_pairs + 1, 0);
@@ -887,21 +991,16 @@ tad_status build_coarse(tad_fn fn, int target)
     };
     TAD_HIP(up(c.agg_of, agg_of));
     TAD_HIP(up(c.agg_ptr, agg_ptr));
-    TAD_HIP(up(c.agg_vert, agg_vert));
     TAD_HIP(up(c.pair_blocks, pair_blocks));
     TAD_HIP(up(c.pair_ab, pair_ab));
-    TAD_HIP(up(c.chunk_ptr, chunk_ptr));
-    TAD_HIP(up(c.agg_chunk, agg_chunk));
     TAD_HIP(up(c.gchunk_ptr, gchunk_ptr));
     TAD_HIP(up(c.pair_chunk, pair_chunk));
     TAD_HIP(hipStreamSynchronize(s));
     c.n_agg = nn;
     c.n_pairs = n_pairs;
-    c.n_chunks = (int64_t)chunk_ptr.size() - 1;
     c.n_gchunks = (int64_t)gchunk_ptr.size() - 1;
-    for (int32_t a = 0; a < nn; ++a) c.max_agg_chunks = std::max(c.max_agg_chunks, agg_chunk[a + 1] - agg_chunk[a]);
     c.target = target;
-    return TAD_OK;
+    return build_order(fn, agg_vert, agg_ptr, c.ord);
 }
 
 // Largest coarse matrix the two-level preconditioner builds (dense FP64 inverse).
@@ -922,7 +1021,7 @@ constexpr double kCoarse32Change = 0.1;
 // positive definite (block-Jacobi alone then).  With o.coarse_reuse the
 // inverse and lever arms of the previous compatible solve are kept (*reused).
 tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o, const unsigned char* free_dev,
-                        CoarseDev* cd, bool* use, bool* reused)
+                        PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused)
 {
     *use = false;
     *reused = false;
@@ -963,30 +1062,21 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     KernelTimer& tm = fn->ctx->timer;
     TAD_HIP(c.dvec.ensure((size_t)nh * d));
     TAD_HIP(c.Ac.ensure((size_t)(nc * nc)));
-    TAD_HIP(c.rc.ensure((size_t)nc));
-    const int Gc = coarse_apply_groups(c.n_agg);
-    TAD_HIP(c.cparts.ensure((size_t)2 * Gc));
+    TAD_HIP(c.dvec_h.ensure((size_t)nh * d));
+    TAD_HIP(c.rpart.ensure((size_t)(c.ord.ppa * nc)));
+    TAD_HIP(c.cparts.ensure((size_t)2 * c.n_agg));
     TAD_HIP(c.info.ensure(2));
-    TAD_HIP(c.chunk_part.ensure((size_t)c.n_chunks * kc));
     TAD_HIP(c.gpart.ensure((size_t)c.n_gchunks * kc * kc));
+    *order = &c.ord;
     cd->kc = kc;
     cd->n_agg = c.n_agg;
     cd->nc = nc;
-    cd->agg_of = c.agg_of.p;
     cd->agg_ptr = c.agg_ptr.p;
-    cd->agg_vert = c.agg_vert.p;
-    cd->n_chunks = c.n_chunks;
-    cd->chunk_ptr = c.chunk_ptr.p;
-    cd->agg_chunk = c.agg_chunk.p;
-    cd->max_agg_chunks = c.max_agg_chunks;
-    cd->chunk_part = c.chunk_part.p;
     cd->dvec = c.dvec.p;
     cd->Ainv = c.Ac.p;
     cd->Ainv32 = c.use32 ? c.Ainv32.p : nullptr;
-    cd->rc = c.rc.p;
+    cd->rpart = c.rpart.p;
     cd->cparts = c.cparts.p;
-    cd->Gc = Gc;
-    cd->free_vars = free_dev;
     if (o.coarse_reuse && c.factor_valid && !free_dev && c.f_kc == kc && c.f_w == o.w_identity)
     {
         *use = true;
@@ -998,12 +1088,13 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     cd->Ainv32 = nullptr;
     tm.begin("coarse_setup", s);
     tm.begin("coarse_galerkin", s);
-    if (rot) TAD_HIP(launch_coarse_dvec(d, nh, fn->x_hess.p, *cd, c.dvec.p, s));
-    else TAD_HIP(launch_fill(c.dvec.p, nh * d, 0.0, s));
+    if (rot)
+        TAD_HIP(launch_coarse_dvec(d, nh, fn->x_hess.p, c.agg_of.p, c.agg_ptr.p, c.ord.perm.p, c.dvec_h.p, c.dvec.p,
+                                   s));
     TAD_HIP(launch_fill(c.Ac.p, nc * nc, 0.0, s));
-    TAD_HIP(launch_coarse_galerkin(d, c.n_pairs, c.n_gchunks, c.gchunk_ptr.p, c.pair_chunk.p, c.pair_blocks.p,
-                                   c.pair_ab.p, fn->block_row.p, fn->brow_ptr.p, fn->bcol.p, fn->row_ptr.p, H_dev,
-                                   o.w_identity, *cd, c.gpart.p, c.Ac.p, s));
+    TAD_HIP(launch_coarse_galerkin(d, kc, nc, c.n_pairs, c.n_gchunks, c.gchunk_ptr.p, c.pair_chunk.p,
+                                   c.pair_blocks.p, c.pair_ab.p, fn->block_row.p, fn->brow_ptr.p, fn->bcol.p,
+                                   fn->row_ptr.p, H_dev, o.w_identity, c.dvec_h.p, free_dev, c.gpart.p, c.Ac.p, s));
     // reduced basis: coarse directions without free variables leave A_c only
     // semidefinite; a relative diagonal shift makes it definite (those
     // directions prolong to zero)
@@ -1024,7 +1115,6 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     if (info[0] != 0)
     {
         tm.end("coarse_setup", s);
-        cd->kc = 0;
         return TAD_OK;  // not positive definite at working precision: block-Jacobi alone
     }
     // The CG iterations read an FP32 copy with the diagonal shift
@@ -1303,25 +1393,17 @@ constexpr int kGraphIters = 8;
 
 // Every operand the recorded CG launches hold: the graph is recorded again
 // when any of them changes.
-std::vector<uint64_t> pcg_graph_key(tad_fn fn, const double* H_dev, const double* sol_dev,
-                                    const unsigned char* free_dev, const CoarseDev* co, double w, hipStream_t s)
+std::vector<uint64_t> pcg_graph_key(int d, const PcgSystem& a, hipStream_t s)
 {
     auto u = [](const void* p) { return (uint64_t)(uintptr_t)p; };
-    uint64_t wbits;
-    std::memcpy(&wbits, &w, sizeof(w));
-    std::vector<uint64_t> k = { (uint64_t)fn->d, (uint64_t)fn->n_handles, u(fn->brow_ptr.p), u(fn->bcol.p),
-                                u(fn->row_ptr.p), u(H_dev), wbits, u(fn->Dinv.p), u(sol_dev), u(fn->r.p),
-                                u(fn->z.p), u(fn->p.p), u(fn->q.p), u(fn->pcg_parts.p), u(fn->scal.p), u(free_dev),
-                                u(s), u(fn->sym_src.p), u(fn->sym_H.p) };
-    if (co)
-    {
-        const uint64_t more[] = { (uint64_t)co->kc, (uint64_t)co->n_agg, (uint64_t)co->nc, u(co->agg_ptr),
-                                  u(co->agg_vert), (uint64_t)co->n_chunks, u(co->chunk_ptr), u(co->agg_chunk),
-                                  (uint64_t)co->max_agg_chunks, u(co->chunk_part), u(co->dvec), u(co->Ainv32),
-                                  u(co->rc), u(co->cparts), (uint64_t)co->Gc, u(co->free_vars) };
-        k.insert(k.end(), std::begin(more), std::end(more));
-    }
-    return k;
+    uint64_t wbits, tbits;
+    std::memcpy(&wbits, &a.w, sizeof(a.w));
+    std::memcpy(&tbits, &a.tol2, sizeof(a.tol2));
+    return { (uint64_t)d, (uint64_t)a.nh, u(a.perm), u(a.brow_ptr), u(a.bcol), u(a.sym_ptr), u(a.usrc), u(a.diag), u(a.Hs),
+             u(a.part_ptr), (uint64_t)a.Gs, (uint64_t)a.Gv, wbits, tbits, (uint64_t)a.max_iters, u(a.b), u(a.sol),
+             u(a.Dinv), u(a.x), u(a.r), u(a.z), u(a.p), u(a.q), u(a.s), u(a.parts), u(a.sc), u(a.free_h), u(a.free_s),
+             (uint64_t)a.kc, (uint64_t)a.ppa, (uint64_t)a.n_agg, (uint64_t)a.nc, u(a.agg_ptr), u(a.dvec), u(a.Ainv),
+             u(a.Ainv32), u(a.rpart), u(a.cparts), u(s) };
 }
 
 tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev,
@@ -1332,37 +1414,63 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     hipStream_t s = fn->s();
     KernelTimer& tm = fn->ctx->timer;
     TAD_HIP(fn->Dinv.ensure((size_t)nh * d * (d + 1) / 2));  // packed symmetric blocks
+    TAD_HIP(fn->xs.ensure(n));
     TAD_HIP(fn->r.ensure(n));
     TAD_HIP(fn->z.ensure(n));
     TAD_HIP(fn->p.ensure(2 * n));
     TAD_HIP(fn->q.ensure(n));
     TAD_HIP(fn->scal.ensure(1));
-    TAD_HIP(fn->pcg_parts.ensure((size_t)pcg_parts_size(d, nh)));
     if (o.max_iters <= 0) return fail(TAD_ERR_INVALID, "max_iters must be positive");
-    tm.begin("pcg_setup", s);
-    TAD_HIP(launch_pcg_setup(d, nh, fn->brow_ptr.p, fn->diag_block.p, fn->row_ptr.p, H_dev, o.w_identity, free_dev,
-                             fn->Dinv.p, s));
-    tm.end("pcg_setup", s);
-    TAD_HIP(fn->sym_H.ensure((size_t)fn->n_sym * d * d));
-    tm.begin("sym_pack", s);
-    TAD_HIP(launch_sym_pack(d, fn->n_sym, fn->sym_full.p, fn->block_row.p, fn->brow_ptr.p, fn->bcol.p,
-                            fn->row_ptr.p, H_dev, fn->sym_H.p, s));
-    tm.end("sym_pack", s);
-    CoarseDev cd;
+    PcgSystem sys;
+    const SolverOrder* od = &fn->natural;
     bool use_coarse = false, coarse_reused = false;
-    TAD_TRY(setup_coarse(fn, H_dev, o, free_dev, &cd, &use_coarse, &coarse_reused));
-    const CoarseDev* co = use_coarse ? &cd : nullptr;
-    PcgScalars hs;
-    std::memset(&hs, 0, sizeof(hs));
-    hs.tol2 = o.tol * o.tol;
-    hs.max_iters = o.max_iters;
-    PcgScalars* pin = (PcgScalars*)(fn->ctx->pinned + 56);
-    std::memcpy(pin, &hs, sizeof(hs));
-    TAD_HIP(hipMemcpyAsync(fn->scal.p, pin, sizeof(hs), hipMemcpyHostToDevice, s));
+    TAD_TRY(setup_coarse(fn, H_dev, o, free_dev, &sys, &od, &use_coarse, &coarse_reused));
+    if (od == &fn->natural && !od->ready)
+    {
+        std::vector<int32_t> id(nh);
+        for (int64_t i = 0; i < nh; ++i) id[i] = (int32_t)i;
+        TAD_TRY(build_order(fn, id, {}, fn->natural));
+    }
+    if (free_dev) TAD_HIP(fn->free_s.ensure(n));
+    TAD_HIP(fn->pcg_parts.ensure((size_t)pcg_parts_size(od->Gs, od->Gv)));
+    TAD_HIP(fn->sym_H.ensure((size_t)od->n_sym * d * d));
+    if (!use_coarse) sys.kc = 0;
+    sys.nh = nh;
+    sys.perm = od->perm.p;
+    sys.brow_ptr = od->brow_ptr.p;
+    sys.bcol = od->bcol.p;
+    sys.sym_ptr = od->sym_ptr.p;
+    sys.usrc = od->usrc.p;
+    sys.diag = od->diag.p;
+    sys.Hs = fn->sym_H.p;
+    sys.part_ptr = od->part_ptr.p;
+    sys.Gs = od->Gs;
+    sys.Gv = od->Gv;
+    sys.ppa = od->ppa;
+    sys.w = o.w_identity;
+    sys.tol2 = o.tol * o.tol;
+    sys.max_iters = o.max_iters;
+    sys.b = rhs_dev;
+    sys.sol = sol_dev;
+    sys.Dinv = fn->Dinv.p;
+    sys.x = fn->xs.p;
+    sys.r = fn->r.p;
+    sys.z = fn->z.p;
+    sys.p = fn->p.p;
+    sys.s = fn->p.p + n;
+    sys.q = fn->q.p;
+    sys.parts = fn->pcg_parts.p;
+    sys.sc = fn->scal.p;
+    sys.free_h = free_dev;
+    sys.free_s = free_dev ? fn->free_s.p : nullptr;
+    tm.begin("sym_pack", s);
+    TAD_HIP(launch_sym_pack(d, od->n_sym, od->place.p, H_dev, fn->sym_H.p, s));
+    tm.end("sym_pack", s);
     tm.begin("pcg_init", s);
-    TAD_HIP(launch_pcg_init(d, nh, rhs_dev, free_dev, fn->Dinv.p, sol_dev, fn->r.p, fn->z.p, fn->pcg_parts.p,
-                            fn->scal.p, co, s));
+    TAD_HIP(launch_pcg_init(d, sys, s));
     tm.end("pcg_init", s);
+    PcgScalars hs;
+    PcgScalars* pin = (PcgScalars*)(fn->ctx->pinned + 56);
     const int every = std::max(1, o.check_every);
     Timer* timer = fn->ctx->timer.enabled ? &fn->ctx->timer : nullptr;
     // iterations are launched in chunks; every kernel returns at once after
@@ -1385,16 +1493,13 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
         auto launch_chunk = [&]() -> hipError_t {
             for (int c = 0; c < kGraphIters; ++c)
             {
-                hipError_t e = launch_pcg_iteration(d, nh, fn->brow_ptr.p, fn->bcol.p, fn->sym_src.p,
-                                                    fn->sym_H.p, o.w_identity, fn->Dinv.p, sol_dev,
-                                                    fn->r.p, fn->z.p, fn->p.p, fn->q.p, fn->pcg_parts.p, fn->scal.p,
-                                                    0, true, free_dev, co, s, nullptr, true);
+                hipError_t e = launch_pcg_iteration(d, sys, 0, true, s, nullptr, true);
                 if (e == hipSuccess) e = launch_pcg_advance(fn->scal.p, s);
                 if (e != hipSuccess) return e;
             }
             return hipSuccess;
         };
-        std::vector<uint64_t> key = pcg_graph_key(fn, H_dev, sol_dev, free_dev, co, o.w_identity, s);
+        std::vector<uint64_t> key = pcg_graph_key(d, sys, s);
         if (fn->pcg_graph && fn->pcg_graph_key == key)
             gexec = fn->pcg_graph;
         else
@@ -1436,10 +1541,7 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
         else
         {
             for (int c = 0; c < chunk && k <= o.max_iters; ++c, ++k)
-                TAD_HIP(launch_pcg_iteration(d, nh, fn->brow_ptr.p, fn->bcol.p, fn->sym_src.p, fn->sym_H.p,
-                                             o.w_identity,
-                                             fn->Dinv.p, sol_dev, fn->r.p, fn->z.p, fn->p.p, fn->q.p, fn->pcg_parts.p,
-                                             fn->scal.p, k, k < o.max_iters, free_dev, co, s, timer));
+                TAD_HIP(launch_pcg_iteration(d, sys, k, k < o.max_iters, s, timer));
         }
         TAD_HIP(hipMemcpyAsync(pin, fn->scal.p, sizeof(hs), hipMemcpyDeviceToHost, s));
         TAD_HIP(hipStreamSynchronize(s));
@@ -1451,12 +1553,17 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     fn->last_solve_iters = hs.iters;
     fn->solves_since_rebuild = coarse_reused ? fn->solves_since_rebuild + 1 : 0;
     const double rel = hs.bb > 0 ? std::sqrt(hs.rr / hs.bb) : 0.0;
+    if (hs.breakdown)  // no product wrote the solution: the last iterate
+    {
+        TAD_HIP(launch_pcg_solution(d, sys, s));
+        TAD_HIP(hipStreamSynchronize(s));
+    }
     if (st)
     {
         st->iters = hs.iters;
         st->rel_residual = rel;
-        st->converged = (!hs.breakdown && hs.rr <= hs.tol2 * hs.bb) ? 1 : 0;
-        st->coarse_unknowns = use_coarse ? (int)cd.nc : 0;
+        st->converged = (!hs.breakdown && hs.rr <= sys.tol2 * hs.bb) ? 1 : 0;
+        st->coarse_unknowns = use_coarse ? (int)sys.nc : 0;
         st->coarse_reused = coarse_reused ? 1 : 0;
     }
     if (hs.breakdown) return fail(TAD_ERR_SOLVE, "Linear solve failed: matrix not positive definite");

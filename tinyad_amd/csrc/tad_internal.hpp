@@ -61,9 +61,10 @@ constexpr int kGroupMaxBlocks = 224;  // 4 waves x 224 x 9 doubles < 64 KiB of L
 // Solver bookkeeping written by block 0 of the PCG kernels (see tad_linalg.hip).
 struct PcgScalars
 {
-    double bb, rr, tol2;
+    double bb, rr;
     double rho_hist[2], alpha_hist[2];  // rho_k and alpha_k, slot k & 1
-    int iters, max_iters, done, breakdown;
+    int iters, breakdown;
+    int done;  // 0; k + 1 when iteration k's product found the end; -1 after a breakdown
     int k;  // iteration index for launches that read it from here (graph replays)
 };
 
@@ -157,53 +158,72 @@ hipError_t launch_axpy_point(const double* x0, const double* dir, const double* 
 hipError_t launch_dot(const double* a, const double* b, int64_t n, double* partials, double* out, hipStream_t s);
 
 // --- PCG -------------------------------------------------------------------
+// Operands of the CG kernels.  Vectors, matrix copy and preconditioner are in
+// solver order: solver entry i belongs to handle perm[i], and with a coarse
+// space the members of an aggregate are consecutive.
 // Coarse space of the two-level preconditioner (additive correction
-// z += P A_c^-1 P^T r on top of block-Jacobi).  P maps kc unknowns per
+// z += P A_c^-1 P^T r on top of block-Jacobi): P maps kc unknowns per
 // aggregate to its handles: d translations and, when kc > d, the rotations
-// about the aggregate's first handle (lever arms dvec[v] = x_v - x_root).
-struct CoarseDev
+// about the aggregate's first handle (lever arms dvec[i] = x_i - x_root).
+struct PcgSystem
 {
-    int kc = 0;                      // unknowns per aggregate; 0: no coarse correction
-    int64_t n_agg = 0, nc = 0;       // aggregates, coarse unknowns (kc * n_agg)
-    const int32_t* agg_of = nullptr; // [n_handles]
-    const int32_t* agg_ptr = nullptr;  // [n_agg + 1] members agg_vert[agg_ptr[a] .. agg_ptr[a+1]), ascending
-    const int32_t* agg_vert = nullptr; // [n_handles]
-    // member lists cut into chunks of at most kCoarseChunk handles, chunks of
-    // one aggregate consecutive: chunk ch covers agg_vert[chunk_ptr[ch] ..
-    // chunk_ptr[ch+1]); aggregate a owns chunks agg_chunk[a] .. agg_chunk[a+1]
-    int64_t n_chunks = 0;
-    const int32_t* chunk_ptr = nullptr;  // [n_chunks + 1]
-    const int32_t* agg_chunk = nullptr;  // [n_agg + 1]
-    int max_agg_chunks = 0;              // most chunks of one aggregate
-    double* chunk_part = nullptr;        // [n_chunks * kc] restriction partials
-    const double* dvec = nullptr;    // [n_handles * d]
-    const double* Ainv = nullptr;    // [nc * nc] inverse Galerkin matrix (symmetric, both triangles)
-    const float* Ainv32 = nullptr;   // [nc * nc] its FP32 copy for the CG iterations (launch_coarse_to32), or null
-    double* rc = nullptr;            // [nc] restricted residual
-    double* cparts = nullptr;        // [2 * Gc] partials of r_c . A_c^-1 r_c, slot k & 1
-    int Gc = 0;                      // workgroups of the coarse product
-    const unsigned char* free_vars = nullptr;  // [n_vars] reduced basis (null: every variable free)
+    int64_t nh = 0;
+    const int32_t* perm = nullptr;      // [nh] handle of each solver entry
+    const int32_t* brow_ptr = nullptr;  // [nh + 1] block rows
+    const int32_t* bcol = nullptr;      // columns (solver order), ascending in each row
+    const int32_t* sym_ptr = nullptr;   // [nh + 1] stored blocks (column <= row) of each row
+    const int32_t* usrc = nullptr;      // per upper block, row after row: the stored block it is the transpose of
+    const int32_t* diag = nullptr;      // [nh] stored diagonal block, -1: none
+    const double* Hs = nullptr;         // stored blocks (launch_sym_pack)
+    // the update kernel's blocks: block b owns entries [part_ptr[b], part_ptr[b + 1])
+    const int32_t* part_ptr = nullptr;  // [Gv + 1]
+    int Gs = 0, Gv = 0;                 // workgroups of the product and the update
+    double w = 0.0, tol2 = 0.0;
+    int max_iters = 0;
+    const double* b = nullptr;          // right-hand side, handle order
+    double* sol = nullptr;              // solution, handle order
+    double *Dinv = nullptr, *x = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *s = nullptr;
+    double* parts = nullptr;            // pcg_parts_size(Gs, Gv) partial sums
+    PcgScalars* sc = nullptr;
+    // reduced basis (CG on the free variables only, the reduced basis of
+    // newton_direction_reduced_basis, NewtonDirection.hh:76-105, for a basis B
+    // that selects variables): mask in handle order (null: every variable
+    // free) and its copy in solver order
+    const unsigned char* free_h = nullptr;
+    unsigned char* free_s = nullptr;
+    // coarse space
+    int kc = 0;                         // unknowns per aggregate; 0: no coarse correction
+    int ppa = 1;                        // update blocks per aggregate (Gv = n_agg * ppa)
+    int64_t n_agg = 0, nc = 0;          // aggregates, coarse unknowns (kc * n_agg)
+    const int32_t* agg_ptr = nullptr;   // [n_agg + 1] entries of each aggregate
+    const double* dvec = nullptr;       // [nh * d]
+    const double* Ainv = nullptr;       // [nc * nc] inverse Galerkin matrix (symmetric, both triangles)
+    const float* Ainv32 = nullptr;      // [nc * nc] its FP32 copy for the CG iterations (launch_coarse_to32), or null
+    double* rpart = nullptr;            // [ppa * nc] restricted residual, one row per part of an aggregate
+    double* cparts = nullptr;           // [2 * n_agg] partials of r_c . A_c^-1 r_c, slot k & 1
 };
 
-constexpr int kCoarseChunk = 256;  // handles per restriction chunk, fine blocks per Galerkin chunk
+constexpr int kCoarseChunk = 256;  // fine blocks per Galerkin chunk
+constexpr int kPcgPartVerts = 64;  // entries the update kernel handles at a time
+constexpr int kPcgMaxParts = 1024;  // update blocks asked for (more only when there are more aggregates)
 
-// Workgroups of the coarse product (one per aggregate), i.e. the r_c . y_c
-// partials it writes per CG iteration.
-int coarse_apply_groups(int64_t n_agg);
-
-// Lever arms dvec[v] = x_v - x_(first member of v's aggregate).
-hipError_t launch_coarse_dvec(int d, int64_t nh, const double* x, const CoarseDev& c, double* dvec, hipStream_t s);
+// Lever arms x_v - x_(first member of v's aggregate) in handle order and in
+// solver order.
+hipError_t launch_coarse_dvec(int d, int64_t nh, const double* x, const int32_t* agg_of, const int32_t* agg_ptr,
+                              const int32_t* perm, double* dvec_h, double* dvec, hipStream_t s);
 
 // A_c (column-major nc x nc, zeroed by the caller) = P^T (w I + H) P.  The
 // fine CSR blocks of each coarse block pair (a, b) (pair_blocks, CSR order)
 // are cut into chunks of at most kCoarseChunk blocks (gchunk_ptr; the chunks
 // of pair p are pair_chunk[p] .. pair_chunk[p+1]); one wave sums a chunk,
 // then each pair sums its chunk partials (gpart, n_gchunks * kc^2) in order.
-hipError_t launch_coarse_galerkin(int d, int64_t n_pairs, int64_t n_gchunks, const int64_t* gchunk_ptr,
-                                  const int32_t* pair_chunk, const int32_t* pair_blocks, const int32_t* pair_ab,
-                                  const int32_t* block_row, const int32_t* brow_ptr, const int32_t* bcol,
-                                  const int32_t* row_ptr, const double* H, double w, const CoarseDev& c,
-                                  double* gpart, double* Ac, hipStream_t s);
+// dvec_h, free_vars: handle order.
+hipError_t launch_coarse_galerkin(int d, int kc, int64_t nc, int64_t n_pairs, int64_t n_gchunks,
+                                  const int64_t* gchunk_ptr, const int32_t* pair_chunk, const int32_t* pair_blocks,
+                                  const int32_t* pair_ab, const int32_t* block_row, const int32_t* brow_ptr,
+                                  const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
+                                  const double* dvec_h, const unsigned char* free_vars, double* gpart, double* Ac,
+                                  hipStream_t s);
 
 // A (n x n, column-major, symmetric positive definite) <- A^-1 (symmetric),
 // by blocked Gauss-Jordan sweeps with FP64 MFMA products.  work:
@@ -223,50 +243,33 @@ hipError_t launch_abs_rowmax(int64_t n, const double* A, double* rowsum, double*
 // positive definite and so is A32.
 hipError_t launch_coarse_to32(int64_t n, const double* A, double delta, float* A32, hipStream_t s);
 
-// Copies the lower triangle of the column-major n x n matrix A to the upper.
-hipError_t launch_symmetrize_lower(int64_t n, double* A, hipStream_t s);
+// The solver's copy of H: the n_sym blocks of its lower triangle in solver
+// order (diagonal included), d*d contiguous row-major values each; place: two
+// int32 per stored block, its offset in H and 4 * row stride + flags (1: read
+// transposed, 2: diagonal, symmetrized from its lower entries): the solve uses
+// H's scalar lower triangle, as SimplicialLDLT does.
+hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* place, const double* H, double* sym_H, hipStream_t s);
 
-// z += P A_c^-1 P^T r (the restriction r_c = P^T r, then the coarse product
-// and the prolongation in one launch, with the partials of r_c . A_c^-1 r_c
-// into slot `slot`); every kernel returns at once once the solve has
-// terminated.
-// kdev (optional): the slot is (*kdev) & 1, read on the device.
-hipError_t launch_coarse_correction(int d, int64_t nh, const CoarseDev& c, const double* r, double* z, int slot,
-                                    PcgScalars* sc, hipStream_t s, Timer* timer, const int* kdev = nullptr);
-// free_vars (optional, n bytes, 0 = fixed): CG on the free variables only, the
-// reduced basis of newton_direction_reduced_basis (NewtonDirection.hh:76-105)
-// for a basis B that selects variables; fixed variables of the solution are 0.
-// Dinv: the block-Jacobi inverse, per handle the upper triangle of its
-// symmetric d x d block (d (d + 1) / 2 doubles, row by row).
-hipError_t launch_pcg_setup(int d, int64_t n_handles, const int32_t* brow_ptr, const int32_t* diag_block,
-                            const int32_t* row_ptr, const double* H, double w, const unsigned char* free_vars,
-                            double* Dinv, hipStream_t s);
+// Workgroups of the product for nh block rows.
+int pcg_spmv_groups(int64_t nh);
+// Size (doubles) of the partial-sum buffer of the CG kernels.
+int64_t pcg_parts_size(int64_t Gs, int64_t Gv);
 
-hipError_t launch_pcg_init(int d, int64_t n_handles, const double* b, const unsigned char* free_vars,
-                           const double* Dinv, double* x, double* r, double* z, double* partials, PcgScalars* sc,
-                           const CoarseDev* coarse, hipStream_t s);
+// Before iteration 0: the block-Jacobi inverse (per entry the upper triangle
+// of its symmetric d x d block, d (d + 1) / 2 doubles, row by row), x = 0,
+// r = b, z = M^-1 r, cleared bookkeeping.
+hipError_t launch_pcg_init(int d, const PcgSystem& a, hipStream_t s);
 
-// The solver's copy of H: the n_sym blocks of its lower triangle (diagonal
-// included) in CSR order, d*d contiguous row-major values each (sym_full: CSR
-// block of each stored block), diagonal blocks symmetrized from their lower
-// entries: the solve uses H's scalar lower triangle, as SimplicialLDLT does.
-hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* sym_full, const int32_t* block_row,
-                           const int32_t* brow_ptr, const int32_t* bcol, const int32_t* row_ptr, const double* H,
-                           double* sym_H, hipStream_t s);
-
-// One CG iteration k: SpMV on z with the termination test, then (with_update)
-// the scalar recurrences and the p / q / x / r / z update, and the coarse
-// correction of z when `coarse` has kc > 0.  pbuf holds 2 * n values (p, then
-// s = (w I + H) z).  read_k: the kernels take k from sc->k on the device
-// instead of the argument (launches recorded once and replayed, with
-// launch_pcg_advance after each iteration).  The SpMV reads H from sym_H
-// (packed by launch_sym_pack): CSR block b reads stored block sym_src[b], or
-// the transpose of ~sym_src[b] when negative.
-hipError_t launch_pcg_iteration(int d, int64_t n_handles, const int32_t* brow_ptr, const int32_t* bcol,
-                                const int32_t* sym_src, const double* sym_H, double w, const double* Dinv, double* x,
-                                double* r, double* z, double* pbuf, double* q, double* partials, PcgScalars* sc, int k,
-                                bool with_update, const unsigned char* free_vars, const CoarseDev* coarse,
-                                hipStream_t s, Timer* timer, bool read_k = false);
+// One CG iteration k: SpMV on z with the termination test (on termination
+// that launch writes the solution), then (with_update) the scalar recurrences
+// and the p / q / x / r / z update, and the coarse correction of z.  read_k:
+// the kernels take k from sc->k on the device instead of the argument
+// (launches recorded once and replayed, with launch_pcg_advance after each
+// iteration).
+hipError_t launch_pcg_iteration(int d, const PcgSystem& a, int k, bool with_update, hipStream_t s, Timer* timer,
+                                bool read_k = false);
+// The current iterate in handle order (a solve that broke down).
+hipError_t launch_pcg_solution(int d, const PcgSystem& a, hipStream_t s);
 // sc->k += 1 (one lane)
 hipError_t launch_pcg_advance(PcgScalars* sc, hipStream_t s);
 
@@ -283,9 +286,6 @@ hipError_t launch_basis_scale(int64_t m, const double* r, const double* dinv, do
 hipError_t launch_basis_step(int64_t m, double alpha, const double* p, const double* q, double* y, double* r,
                              hipStream_t s);
 hipError_t launch_basis_direction(int64_t m, const double* z, double beta, double* p, hipStream_t s);
-
-// Size (doubles) of the partial-sum buffer the PCG kernels need.
-int64_t pcg_parts_size(int d, int64_t n_handles);
 
 // Per-segment energies: ranges[(t * n_seg + s) * 2 + {0,1}] is the element
 // range of segment s in term t (absolute indices into elem_f).

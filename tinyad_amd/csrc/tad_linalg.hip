@@ -12,6 +12,7 @@
 #include <cstdint>
 #include <algorithm>
 #include "tad_internal.hpp"
+#include "tad_wave.hpp"
 #include "tad_energies.hpp"
 #include "tad_elements.hpp"
 
@@ -33,22 +34,6 @@ __device__ __forceinline__ double block_sum(double v, double* sh)
     double r = sh[0];
 #pragma unroll
     for (int w = 1; w < kBlock / 64; ++w) r += sh[w];
-    return r;
-}
-
-// Same fixed-order reduction for a block of NT threads (NT a multiple of 64).
-template <int NT>
-__device__ __forceinline__ double block_sum_n(double v, double* sh)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    const int wave = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh[wave] = v;
-    __syncthreads();
-    double r = sh[0];
-#pragma unroll
-    for (int w = 1; w < NT / 64; ++w) r += sh[w];
     return r;
 }
 
@@ -448,37 +433,14 @@ hipError_t launch_assemble_gradient(int d, int precision, int64_t nh, const int6
 // another block of the same kernel writes.  Block 0 records bookkeeping
 // (iteration count, residual, termination) for later kernels and the host.
 //
-// Partial buffer layout (doubles): [pq: Gs][rz: 2 x Gv][rr: 2 x Gv][rr0: Gv]
-
-// Block-uniform read of the termination flag: block 0 of the same kernel may
-// set it while other blocks start, so one thread reads it for the whole block
-// and every thread then takes the same branch around the barriers below.
-__device__ __forceinline__ bool block_done(const PcgScalars* sc)
-{
-    __shared__ int flag;
-    if (threadIdx.x == 0) flag = sc->done;
-    __syncthreads();
-    return flag != 0;
-}
-
-// Every block re-sums all n partials: thread t adds parts[t], parts[t + NT],
-// ... in index order (four loads in flight), then the fixed block tree.
-template <int NT = kBlock>
-__device__ __forceinline__ double sum_parts(const double* __restrict__ parts, int n, double* sh)
-{
-    double acc = 0.0;
-    int i = threadIdx.x;
-    for (; i + 3 * NT < n; i += 4 * NT)
-    {
-        const double a0 = parts[i], a1 = parts[i + NT], a2 = parts[i + 2 * NT], a3 = parts[i + 3 * NT];
-        acc += a0;
-        acc += a1;
-        acc += a2;
-        acc += a3;
-    }
-    for (; i < n; i += NT) acc += parts[i];
-    return block_sum_n<NT>(acc, sh);
-}
+// Partial buffer layout (doubles): [pq: Gs][rz: 2 x Gv][rr: 2 x Gv]
+//
+// The solver's vectors, matrix copy and preconditioner are in solver order
+// (PcgSystem::perm): the members of an aggregate are consecutive, so that the
+// update kernel, whose blocks own a part of one aggregate each, also sums the
+// aggregate's restricted residual, the coarse correction adds to consecutive
+// entries, and the rows a block of the product takes share most of the
+// entries of z they gather.
 
 // The block-Jacobi inverse keeps the upper triangle of each symmetric D x D
 // block, row by row: (0,0) (0,1) .. (0,D-1) (1,1) .. (D-1,D-1).
@@ -519,107 +481,6 @@ __device__ __forceinline__ void invert_block(const double* B, double* o)
     }
 }
 
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_pcg_setup(int64_t nh, const int32_t* __restrict__ brow_ptr,
-                                                      const int32_t* __restrict__ diag_block,
-                                                      const int32_t* __restrict__ row_ptr,
-                                                      const double* __restrict__ H, double w,
-                                                      const unsigned char* __restrict__ free_vars,
-                                                      double* __restrict__ Dinv)
-{
-    const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= nh) return;
-    const int nbu = brow_ptr[u + 1] - brow_ptr[u];
-    const int k = diag_block[u];
-    const int64_t base = row_ptr[D * u];
-    // reduced basis: a fixed component takes a unit row / column here and a
-    // zero row / column in the inverse (the free sub-block's inverse)
-    bool fr[D];
-#pragma unroll
-    for (int i = 0; i < D; ++i) fr[i] = free_vars ? free_vars[u * D + i] != 0 : true;
-    double B[D * D], o[D * D];
-    if (k < 0)
-    {
-        // handle used by no element: its rows are empty, (w I + H) is w I there
-#pragma unroll
-        for (int i = 0; i < D; ++i)
-#pragma unroll
-            for (int j = i; j < D; ++j)
-                Dinv[u * PackedBlock<D>::n + PackedBlock<D>::at(i, j)] =
-                    (i == j && fr[i]) ? (w > 0.0 ? 1.0 / w : 1.0) : 0.0;
-        return;
-    }
-    // the block's lower entries (the solve uses H's scalar lower triangle)
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-#pragma unroll
-        for (int j = 0; j < D; ++j)
-        {
-            const int il = i > j ? i : j, jl = i > j ? j : i;
-            B[i * D + j] = (fr[i] && fr[j]) ? H[base + (int64_t)il * D * nbu + D * k + jl] + (i == j ? w : 0.0)
-                                            : (i == j ? 1.0 : 0.0);
-        }
-    invert_block<D>(B, o);
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-#pragma unroll
-        for (int j = 0; j < D; ++j)
-            if (!(fr[i] && fr[j])) o[i * D + j] = 0.0;
-    // the upper triangle: the inverse of a symmetric block is symmetric (the
-    // cofactor products above commute), and the stored preconditioner is
-    // symmetric exactly even where H's block is so only up to rounding
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-#pragma unroll
-        for (int j = i; j < D; ++j) Dinv[u * PackedBlock<D>::n + PackedBlock<D>::at(i, j)] = o[i * D + j];
-}
-
-// x = 0, r = b, z = M^-1 r; partials rho_0 = r.z (slot 1) and ||b||^2 (rr0)
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_pcg_init(int64_t nh, const double* __restrict__ b,
-                                                     const unsigned char* __restrict__ free_vars,
-                                                     const double* __restrict__ Dinv, double* __restrict__ x,
-                                                     double* __restrict__ r, double* __restrict__ z,
-                                                     double* __restrict__ parts, int Gs, int Gv, PcgScalars* sc)
-{
-    __shared__ double sh[kBlock];
-    double rz = 0.0, rr = 0.0;
-    for (int64_t u = (int64_t)blockIdx.x * kBlock + threadIdx.x; u < nh; u += (int64_t)gridDim.x * kBlock)
-    {
-        double rv[D];
-#pragma unroll
-        for (int i = 0; i < D; ++i)
-        {
-            rv[i] = (free_vars && !free_vars[u * D + i]) ? 0.0 : b[u * D + i];
-            x[u * D + i] = 0.0;
-            r[u * D + i] = rv[i];
-        }
-#pragma unroll
-        for (int i = 0; i < D; ++i)
-        {
-            double zi = 0.0;
-#pragma unroll
-            for (int j = 0; j < D; ++j) zi += Dinv[u * PackedBlock<D>::n + PackedBlock<D>::at(i, j)] * rv[j];
-            z[u * D + i] = zi;
-            rz += rv[i] * zi;
-            rr += rv[i] * rv[i];
-        }
-    }
-    const double srz = block_sum(rz, sh);
-    const double srr = block_sum(rr, sh);
-    if (threadIdx.x == 0)
-    {
-        parts[Gs + Gv + blockIdx.x] = srz;      // rho_0 in slot 1
-        parts[Gs + 4 * Gv + blockIdx.x] = srr;  // rr0
-        if (blockIdx.x == 0)
-        {
-            sc->iters = 0;
-            sc->done = 0;
-            sc->breakdown = 0;
-        }
-    }
-}
-
 // Chronopoulos-Gear form of preconditioned CG (the iterates of standard PCG
 // in exact arithmetic, one reduction point per iteration):
 //   s_k = A z_k,  delta_k = z_k.s_k,  rho_k = r_k.z_k
@@ -629,16 +490,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_init(int64_t nh, const double* _
 //   x += alpha p,  r -= alpha q,  z = M^-1 r
 // so the SpMV gathers only z, which is complete when it runs.
 
-// The solver's copy of H (the lower triangle's blocks, diagonal included, in
-// CSR order; D*D contiguous row-major values each), one thread per value.
-// A diagonal block takes its upper entries from its lower ones, so the copy
-// is the symmetric matrix of H's scalar lower triangle.
+// The solver's copy of H: its lower triangle's blocks in solver order
+// (diagonal included), D*D contiguous row-major values each, one thread per
+// value.  place[l] is stored block l's offset in H and 4 * row stride + flags
+// (1: take the transpose of the block there; 2: diagonal, take the upper
+// entries from the lower ones), so that the copy is the symmetric matrix of
+// H's scalar lower triangle.
 template <int D>
-__global__ __launch_bounds__(kBlock) void k_sym_pack(int64_t n_sym, const int32_t* __restrict__ sym_full,
-                                                     const int32_t* __restrict__ block_row,
-                                                     const int32_t* __restrict__ brow_ptr,
-                                                     const int32_t* __restrict__ bcol,
-                                                     const int32_t* __restrict__ row_ptr,
+__global__ __launch_bounds__(kBlock) void k_sym_pack(int64_t n_sym, const int2* __restrict__ place,
                                                      const double* __restrict__ H, double* __restrict__ Hs)
 {
     constexpr int DD = D * D;
@@ -647,54 +506,70 @@ __global__ __launch_bounds__(kBlock) void k_sym_pack(int64_t n_sym, const int32_
     const int64_t l = id / DD;
     const int m = (int)(id - l * DD);
     int i = m / D, j = m - i * D;
-    const int32_t b = sym_full[l];
-    const int32_t u = block_row[b];
-    if (bcol[b] == u && i < j)
+    const int2 pl = place[l];
+    if ((pl.y & 1) || ((pl.y & 2) && i < j))
     {
         const int t = i;
         i = j;
         j = t;
     }
-    const int32_t b0 = brow_ptr[u];
-    const int64_t nbu = brow_ptr[u + 1] - b0;
-    Hs[id] = H[(int64_t)row_ptr[D * u] + i * D * nbu + (int64_t)D * (b - b0) + j];
+    Hs[id] = H[(int64_t)pl.x + (int64_t)i * (pl.y >> 2) + j];
+}
+
+// sol = x in handle order (solver entry i belongs to handle perm[i])
+template <int D>
+__device__ __forceinline__ void unpermute(int64_t nh, const int32_t* __restrict__ perm, const double* __restrict__ x,
+                                          double* __restrict__ sol)
+{
+    for (int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; id < nh * D;
+         id += (int64_t)gridDim.x * blockDim.x)
+    {
+        const int64_t i = id / D;
+        sol[(int64_t)perm[i] * D + (id - i * D)] = x[id];
+    }
+}
+
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_unpermute(int64_t nh, const int32_t* __restrict__ perm,
+                                                      const double* __restrict__ x, double* __restrict__ sol)
+{
+    unpermute<D>(nh, perm, x, sol);
 }
 
 // CG iteration k, first half: termination test on rr_k = ||r_k||^2 (k = 0:
-// ||b||^2, recorded), then s = (w I + H) z and partial z.s.  The termination
-// flag, the residual partials and the first row group's block data are all
-// requested before the test, so their memory latencies overlap.  LPB lanes
-// per block row, lane k takes blocks k, k + LPB, ... of the row, then a
-// shuffle tree.  H comes from the solver's copy: block b of row u is stored
-// block src[b], or the transpose of stored block ~src[b] (the lower block
-// (v, u) it mirrors), so every stored off-diagonal block is read twice per
-// product.  XCD: the workgroups of one XCD (blockIdx % 8, the dispatch order
+// ||b||^2, recorded), then s = (w I + H) z and partial z.s.  On termination
+// the launch that finds it writes the solution in handle order instead (every
+// block decides alike; done = k + 1 marks that launch, so that a block that
+// starts late and already reads the flag still writes its share).  The
+// termination flag, the residual partials and the first row group's data are
+// all requested before the test, so their memory latencies overlap.  LPB
+// lanes per block row, lane k takes blocks k, k + LPB, ... of the row, then a
+// fixed tree.  H comes from the solver's copy: a row's columns ascend, so its
+// blocks up to the diagonal are the stored blocks of the row in order, and an
+// upper block is the transpose of stored block usrc (the lower block (v, u)
+// it mirrors); every stored off-diagonal block is read twice per product.  XCD: the workgroups of one XCD (blockIdx % 8, the dispatch order
 // across the eight XCDs) take a contiguous eighth of the row groups in
 // order, so the block an upper block reads belongs to a row that the same
 // XCD streams shortly after, and the second read can hit in that XCD's L2.
-// Requires gridDim.x % 8 == 0 for XCD.
+// Requires gridDim.x % 8 == 0 for XCD.  60^3 cube: 160 MB in 36 us (4.4 TB/s);
+// the upper blocks' 72-byte pieces are separate cache lines for every lane.
 template <int D, int LPB, bool XCD>
-__global__ __launch_bounds__(kBlock) void k_spmv_sym(int64_t nh, const int32_t* __restrict__ brow_ptr,
-                                                     const int32_t* __restrict__ bcol,
-                                                     const int32_t* __restrict__ src, const double* __restrict__ Hs,
-                                                     double w, const double* __restrict__ z,
-                                                     double* __restrict__ sv, double* __restrict__ parts, int Gs,
-                                                     int Gv, int k, const int* __restrict__ kdev, PcgScalars* sc)
+__global__ __launch_bounds__(kBlock) void k_spmv_sym(PcgSystem a, int Gs, int Gv, int k, const int* __restrict__ kdev)
 {
-    static_assert(kBlock * 4 >= 1024, "the residual partials (at most 1024) are read four per thread");
     constexpr int DD = D * D;
+    const int64_t nh = a.nh;
+    const int32_t* __restrict__ bcol = a.bcol;
+    const int32_t* __restrict__ usrc = a.usrc;
+    const double* __restrict__ Hs = a.Hs;
+    const double* __restrict__ z = a.z;
+    PcgScalars* sc = a.sc;
     if (kdev) k = *kdev;
-    __shared__ double sh[kBlock];
+    __shared__ double sh[kBlock / 64][1], sh2[kBlock / 64][1];
     __shared__ int flag;
     const int done_v = threadIdx.x == 0 ? sc->done : 0;
-    const double* rparts = k == 0 ? parts + Gs + 4 * Gv : parts + Gs + 2 * Gv + ((k + 1) & 1) * Gv;
-    double pa[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-    {
-        const int i = threadIdx.x + q * kBlock;
-        pa[q] = i < Gv ? rparts[i] : 0.0;
-    }
+    const double* rparts = a.parts + Gs + 2 * Gv + ((k + 1) & 1) * Gv;
+    double rv[4];
+    strided_fetch<kBlock, 4>(rparts, Gv, rv);
     const int lane = threadIdx.x % LPB;
     constexpr int rows_per_block = kBlock / LPB;
     const int64_t n_groups = (nh + rows_per_block - 1) / rows_per_block;
@@ -713,63 +588,68 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sym(int64_t nh, const int32_t* 
         gstep = gridDim.x;
         gend = n_groups;
     }
-    auto load_block = [&](int64_t b, double* h) {
-        const int32_t si = src[b];
-        const double* __restrict__ hb = Hs + (int64_t)(si < 0 ? ~si : si) * DD;
-        double t[DD];
+    // the row's first two blocks of this lane: everything they need is loaded
+    // before anything is used, so 16 blocks per row are in flight at once
+    struct Two
+    {
+        double h[2][DD], z[2][D];
+        bool tr[2];
+    };
+    int b0, nbu, s0, nlow;  // first block of the row, blocks, first stored block, stored blocks
+    auto row_head = [&](int64_t u) {
+        b0 = a.brow_ptr[u];
+        nbu = a.brow_ptr[u + 1] - b0;
+        s0 = a.sym_ptr[u];
+        nlow = a.sym_ptr[u + 1] - s0;
+    };
+    auto load_block = [&](int kk, double* h, double* zv, bool& tr) {
+        const int64_t v = bcol[b0 + kk];
+        tr = kk >= nlow;
+        const int us = usrc[max(0, b0 - s0 + kk - nlow)];  // (read by every lane: no branch before the block's loads)
+        const int64_t si = tr ? us : s0 + kk;
+        const double* __restrict__ hb = Hs + si * DD;
 #pragma unroll
-        for (int m = 0; m < DD; ++m) t[m] = hb[m];
+        for (int m = 0; m < DD; ++m) h[m] = hb[m];
+#pragma unroll
+        for (int j = 0; j < D; ++j) zv[j] = z[v * D + j];
+    };
+    auto add_block = [&](const double* h, const double* zv, bool tr, double* acc) {
 #pragma unroll
         for (int i = 0; i < D; ++i)
 #pragma unroll
-            for (int j = 0; j < D; ++j) h[i * D + j] = si < 0 ? t[j * D + i] : t[i * D + j];
+            for (int j = 0; j < D; ++j) acc[i] += (tr ? h[j * D + i] : h[i * D + j]) * zv[j];
     };
-    int f_nbu = 0, f_b0 = 0;
-    int64_t f_v = 0;
-    double f_h[DD];
-    if (g0 < gend)
+    Two t2;
+    auto load_two = [&](int64_t u) {
+        row_head(u);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            if (lane + m * LPB < nbu) load_block(lane + m * LPB, t2.h[m], t2.z[m], t2.tr[m]);
+    };
     {
         const int64_t u = g0 * rows_per_block + threadIdx.x / LPB;
-        if (u < nh)
-        {
-            f_b0 = brow_ptr[u];
-            f_nbu = brow_ptr[u + 1] - f_b0;
-            if (lane < f_nbu)
-            {
-                f_v = bcol[f_b0 + lane];
-                load_block(f_b0 + lane, f_h);
-            }
-        }
+        if (g0 < gend && u < nh) load_two(u);
     }
     if (threadIdx.x == 0) flag = done_v;
-    __syncthreads();
-    if (flag) return;
-    double racc = 0.0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        if ((int)threadIdx.x + q * kBlock < Gv) racc += pa[q];
-    const double rsum = block_sum_n<kBlock>(racc, sh);
-    double rr, bb;
-    if (k == 0)
-    {
-        bb = rsum;
-        rr = bb;
-    }
-    else
-    {
-        rr = rsum;
-        bb = sc->bb;
-    }
-    const bool stop = rr <= sc->tol2 * bb || k >= sc->max_iters;
+    double racc[1] = { strided_rest<kBlock, 4>(rparts, Gv, rv) };
+    block_totals<kBlock, 1>(racc, sh);  // its barrier publishes the flag
+    if (flag != 0 && flag != k + 1) return;
+    const double rr = racc[0];
+    const double bb = k == 0 ? rr : sc->bb;
+    const bool stop = rr <= a.tol2 * bb || k >= a.max_iters;
     if (blockIdx.x == 0 && threadIdx.x == 0)
     {
         if (k == 0) sc->bb = bb;
         sc->rr = rr;
         sc->iters = k;
-        if (stop) sc->done = 1;
+        if (stop) sc->done = k + 1;
     }
-    if (stop) return;
-    double zs = 0.0;
+    if (stop)
+    {
+        unpermute<D>(nh, a.perm, a.x, a.sol);
+        return;
+    }
+    double zs[1] = { 0.0 };
     bool first = true;
     for (int64_t g = g0; g < gend; g += gstep)
     {
@@ -779,197 +659,39 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sym(int64_t nh, const int32_t* 
         for (int i = 0; i < D; ++i) acc[i] = 0.0;
         if (u < nh)
         {
-            int b0, nbu, kk0;
-            if (first)
+            if (!first) load_two(u);
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                if (lane + m * LPB < nbu) add_block(t2.h[m], t2.z[m], t2.tr[m], acc);
+            for (int kk = lane + 2 * LPB; kk < nbu; kk += LPB)
             {
-                b0 = f_b0;
-                nbu = f_nbu;
-                if (lane < nbu)
-                {
-                    double zv[D];
-#pragma unroll
-                    for (int j = 0; j < D; ++j) zv[j] = z[f_v * D + j];
-#pragma unroll
-                    for (int i = 0; i < D; ++i)
-#pragma unroll
-                        for (int j = 0; j < D; ++j) acc[i] += f_h[i * D + j] * zv[j];
-                }
-                kk0 = lane + LPB;
-            }
-            else
-            {
-                b0 = brow_ptr[u];
-                nbu = brow_ptr[u + 1] - b0;
-                kk0 = lane;
-            }
-            for (int kk = kk0; kk < nbu; kk += LPB)
-            {
-                const int64_t v = bcol[b0 + kk];
-                double h[DD];
-                load_block(b0 + kk, h);
-                double zv[D];
-#pragma unroll
-                for (int j = 0; j < D; ++j) zv[j] = z[v * D + j];
-#pragma unroll
-                for (int i = 0; i < D; ++i)
-#pragma unroll
-                    for (int j = 0; j < D; ++j) acc[i] += h[i * D + j] * zv[j];
+                load_block(kk, t2.h[0], t2.z[0], t2.tr[0]);
+                add_block(t2.h[0], t2.z[0], t2.tr[0], acc);
             }
         }
         first = false;
+        static_assert(LPB == 8, "the sum over a row's lanes: quads, then 8 lanes");
 #pragma unroll
-        for (int off = LPB / 2; off > 0; off >>= 1)
-#pragma unroll
-            for (int i = 0; i < D; ++i) acc[i] += __shfl_xor(acc[i], off, LPB);
+        for (int i = 0; i < D; ++i)
+        {
+            acc[i] += dpp_move<0xB1>(acc[i]);   // quad_perm 1 0 3 2
+            acc[i] += dpp_move<0x4E>(acc[i]);   // quad_perm 2 3 0 1
+            acc[i] += dpp_move<0x141>(acc[i]);  // row_half_mirror
+        }
         if (u < nh && lane == 0)
         {
 #pragma unroll
             for (int i = 0; i < D; ++i)
             {
                 const double zi = z[u * D + i];
-                const double si = acc[i] + w * zi;
-                sv[u * D + i] = si;
-                zs += zi * si;
+                const double si = acc[i] + a.w * zi;
+                a.s[u * D + i] = si;
+                zs[0] += zi * si;
             }
         }
     }
-    const double tot = block_sum(zs, sh);
-    if (threadIdx.x == 0) parts[blockIdx.x] = tot;
-}
-
-// CG iteration k, second half: scalars, direction recurrences, x / r / z
-// update; partials of rho_{k+1} = r.z and ||r||^2 into slot k & 1.  alpha and
-// rho of iteration k are kept (slot k & 1 of sc) for iteration k + 1.
-// A block of 64 D threads owns 64 consecutive vertices per step: thread t
-// updates variable t of the chunk (every vector access is a contiguous run),
-// and the D x D preconditioner blocks and the new residual pass through LDS
-// for z = M^-1 r.
-constexpr int kUpdVerts = 64;
-
-template <int D>
-__global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(int64_t nh, const double* __restrict__ Dinv,
-                                                              double* __restrict__ x, double* __restrict__ r,
-                                                              double* __restrict__ z, double* __restrict__ p,
-                                                              double* __restrict__ q,
-                                                              const double* __restrict__ sv,
-                                                              double* __restrict__ parts, int Gs, int Gv, int k,
-                                                              const int* __restrict__ kdev,
-                                                              const double* __restrict__ cparts, int Gc,
-                                                              const unsigned char* __restrict__ free_vars,
-                                                              PcgScalars* sc)
-{
-    if (kdev) k = *kdev;
-    constexpr int NT = kUpdVerts * D;
-    constexpr int PB = PackedBlock<D>::n;
-    constexpr int ND = (kUpdVerts * PB + NT - 1) / NT;  // packed block entries per thread and chunk
-    if (block_done(sc)) return;
-    __shared__ double sh[NT];
-    __shared__ double sD[ND * NT];
-    __shared__ double sR[NT];
-    const int64_t n = nh * D;
-    const int64_t dn = nh * PB;
-    const int t = threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * kUpdVerts;
-    // operands of one chunk: this thread's variable and its share of the
-    // chunk's packed preconditioner blocks
-    double zc = 0.0, pc = 0.0, qc = 0.0, sc_ = 0.0, xc = 0.0, rc = 0.0, dc[ND];
-    auto load = [&](int64_t c0) {
-        const int64_t iv = c0 * D + t;
-        if (iv < n)
-        {
-            zc = z[iv];
-            pc = p[iv];
-            qc = q[iv];
-            sc_ = sv[iv];
-            xc = x[iv];
-            rc = r[iv];
-        }
-#pragma unroll
-        for (int m = 0; m < ND; ++m)
-        {
-            const int64_t id = c0 * PB + t + (int64_t)m * NT;
-            dc[m] = (t + m * NT < kUpdVerts * PB && id < dn) ? Dinv[id] : 0.0;
-        }
-    };
-    int64_t c0 = (int64_t)blockIdx.x * kUpdVerts;
-    if (c0 < nh) load(c0);  // in flight during the scalar re-sums
-    const double delta = sum_parts<NT>(parts, Gs, sh);
-    double rho = sum_parts<NT>(parts + Gs + ((k + 1) & 1) * Gv, Gv, sh);
-    // r.z with the coarse correction: r.(D^-1 r) + (P^T r).(A_c^-1 P^T r)
-    if (Gc > 0) rho += sum_parts<NT>(cparts + ((k + 1) & 1) * Gc, Gc, sh);
-    double beta = 0.0, den = delta;
-    if (k > 0)
-    {
-        const double rho_prev = sc->rho_hist[(k + 1) & 1];
-        const double alpha_prev = sc->alpha_hist[(k + 1) & 1];
-        beta = rho / rho_prev;
-        den = delta - beta * rho / alpha_prev;
-        // p.Ap from the recurrence can cancel to <= 0 near convergence even
-        // for a positive definite matrix: restart along z (beta = 0, p = z,
-        // p.Ap = z.Az) instead of reporting a breakdown
-        if (!(den > 0.0))
-        {
-            beta = 0.0;
-            den = delta;
-        }
-    }
-    if (!(den > 0.0))
-    {
-        // not positive definite along z: the same decision in every block
-        if (blockIdx.x == 0 && threadIdx.x == 0)
-        {
-            sc->breakdown = 1;
-            sc->done = 1;
-            sc->iters = k;
-        }
-        return;
-    }
-    const double alpha = rho / den;
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-    {
-        sc->rho_hist[k & 1] = rho;
-        sc->alpha_hist[k & 1] = alpha;
-    }
-    double rz = 0.0, rr = 0.0;
-    for (; c0 < nh; c0 += stride)
-    {
-        const int64_t iv = c0 * D + t;
-        double rv = 0.0;
-        if (iv < n)
-        {
-            const double pi = k > 0 ? fma(beta, pc, zc) : zc;
-            const double qi = k > 0 ? fma(beta, qc, sc_) : sc_;
-            p[iv] = pi;
-            q[iv] = qi;
-            x[iv] = xc + alpha * pi;
-            rv = rc - alpha * qi;
-            if (free_vars && !free_vars[iv]) rv = 0.0;  // reduced basis: no residual on fixed variables
-            r[iv] = rv;
-        }
-        __syncthreads();  // the previous chunk's LDS reads are complete
-        sR[t] = rv;
-#pragma unroll
-        for (int m = 0; m < ND; ++m) sD[t + m * NT] = dc[m];
-        __syncthreads();
-        if (c0 + stride < nh) load(c0 + stride);  // next chunk in flight during this one's z
-        if (iv < n)
-        {
-            const int vl = t / D, i = t - vl * D;
-            double zi = 0.0;
-#pragma unroll
-            for (int j = 0; j < D; ++j) zi += sD[vl * PB + PackedBlock<D>::at(i, j)] * sR[vl * D + j];
-            z[iv] = zi;
-            rz += rv * zi;
-            rr += rv * rv;
-        }
-    }
-    const double srz = block_sum_n<NT>(rz, sh);
-    const double srr = block_sum_n<NT>(rr, sh);
-    if (threadIdx.x == 0)
-    {
-        parts[Gs + (k & 1) * Gv + blockIdx.x] = srz;
-        parts[Gs + 2 * Gv + (k & 1) * Gv + blockIdx.x] = srr;
-    }
+    block_totals<kBlock, 1>(zs, sh2);
+    if (threadIdx.x == 0) a.parts[blockIdx.x] = zs[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -980,7 +702,7 @@ __global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(int64_t nh, const 
 // translations and, for KC > D, the rotations omega about the aggregate's
 // first handle, delta x_v = omega x dv (D = 3) or omega (-dv_1, dv_0) (D = 2).
 // Every sum below runs in a fixed order (fixed lane assignment and a fixed
-// shuffle tree), so the correction is bitwise reproducible.
+// tree), so the correction is bitwise reproducible.
 template <int D, int KC>
 __device__ __forceinline__ void coarse_rows(const double* __restrict__ dv, double R[D][KC])
 {
@@ -1007,27 +729,308 @@ __device__ __forceinline__ void coarse_rows(const double* __restrict__ dv, doubl
     }
 }
 
+// CG iteration k, second half: scalars, direction recurrences, x / r / z
+// update; partials of rho_{k+1} = r.z and ||r||^2 into slot k & 1.  alpha and
+// rho of iteration k are kept (slot k & 1 of sc) for iteration k + 1.
+// Block b owns the handles [part_ptr[b], part_ptr[b + 1]) of solver order, a
+// part of one aggregate, in chunks of 64: thread t updates variable t of the
+// chunk (every vector access is a contiguous run), the D x D preconditioner
+// blocks, the new residual and the lever arms pass through LDS for
+// z = M^-1 r and (KC > 0) the first wave's sums R_v^T r_v of the restricted
+// residual: block b = aggregate * ppa + p writes its KC sums to row p of
+// rpart, so r_c is the sum of ppa rows and needs no kernel of its own.  At 10K
+// handles the kernel is a chain of memory latencies, so the operands of the
+// first chunk and all partials of the three scalars are requested before any
+// is used: 100 x 100 grid update 6.5 us + restriction 3.2 -> 4.8 us in all;
+// 30^3 tet cube 6.7 + 4.2 -> 6.6; 60^3, bound by 78 MB of vectors, 16.0 + 6.4
+// -> 14.6 (5.3 TB/s).
+//
+// INIT (before iteration 0, k = -1): the block-Jacobi inverse from the
+// solver's copy of H, x = 0, r = b, z = M^-1 r and the same partials.
+constexpr int kUpdVerts = 64;
+
+template <int D, int KC, bool INIT>
+__global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(PcgSystem a, int Gs, int Gv, int k,
+                                                              const int* __restrict__ kdev)
+{
+    constexpr int NT = kUpdVerts * D;
+    constexpr int NW = D;  // waves
+    constexpr int PB = PackedBlock<D>::n;
+    constexpr int ND = (kUpdVerts * PB + NT - 1) / NT;  // packed block entries per thread and chunk
+    constexpr bool ROT = KC > D;
+    __shared__ double sh[NW][3], sh2[NW][2];
+    __shared__ double sD[ND * NT];
+    __shared__ double sR[NT];
+    __shared__ double sV[ROT ? NT : 1];
+    __shared__ int flag;
+    PcgScalars* sc = a.sc;
+    const int t = threadIdx.x;
+    const int blk = blockIdx.x;
+    if (INIT) k = -1;
+    else if (kdev) k = *kdev;
+    const int64_t lo = a.part_ptr[blk], hi = a.part_ptr[blk + 1];
+    // operands of one chunk: this thread's variable and its share of the
+    // chunk's packed preconditioner blocks
+    double zc = 0.0, pc = 0.0, qc = 0.0, sc_ = 0.0, xc = 0.0, rc = 0.0, vc = 0.0, dc[ND];
+    auto load = [&](int64_t c0) {
+        const int64_t iv = c0 * D + t;
+        if (iv < hi * D)
+        {
+            if constexpr (INIT)
+                rc = a.b[(int64_t)a.perm[iv / D] * D + iv % D];
+            else
+            {
+                zc = a.z[iv];
+                pc = a.p[iv];
+                qc = a.q[iv];
+                sc_ = a.s[iv];
+                xc = a.x[iv];
+                rc = a.r[iv];
+            }
+            if constexpr (ROT) vc = a.dvec[iv];
+        }
+        if constexpr (!INIT)
+        {
+#pragma unroll
+            for (int m = 0; m < ND; ++m)
+            {
+                const int64_t id = c0 * PB + t + (int64_t)m * NT;
+                dc[m] = (t + m * NT < kUpdVerts * PB && id < hi * PB) ? a.Dinv[id] : 0.0;
+            }
+        }
+    };
+    double alpha = 0.0, beta = 0.0;
+    if constexpr (INIT)
+    {
+        if (lo < hi) load(lo);
+        if (blk == 0 && t == 0)
+        {
+            sc->iters = 0;
+            sc->done = 0;
+            sc->breakdown = 0;
+            sc->k = 0;
+        }
+    }
+    else
+    {
+        const int done_v = t == 0 ? sc->done : 0;
+        const double rho_prev = k > 0 ? sc->rho_hist[(k + 1) & 1] : 1.0;
+        const double alpha_prev = k > 0 ? sc->alpha_hist[(k + 1) & 1] : 1.0;
+        // delta, r.(D^-1 r), (P^T r).(A_c^-1 P^T r): thread t adds the
+        // partials t, t + NT, ... in order
+        const double* __restrict__ pd = a.parts;
+        const double* __restrict__ pr = a.parts + Gs + ((k + 1) & 1) * Gv;
+        const double* __restrict__ pk = KC > 0 ? a.cparts + ((k + 1) & 1) * a.n_agg : nullptr;
+        double vd[6], vr[6], vk[3];
+        strided_fetch<NT, 6>(pd, Gs, vd);
+        strided_fetch<NT, 6>(pr, Gv, vr);
+        if constexpr (KC > 0) strided_fetch<NT, 3>(pk, a.n_agg, vk);
+        if (lo < hi) load(lo);  // in flight during the sums
+        if (t == 0) flag = done_v;
+        double tot[3] = { strided_rest<NT, 6>(pd, Gs, vd), strided_rest<NT, 6>(pr, Gv, vr), 0.0 };
+        if constexpr (KC > 0) tot[2] = strided_rest<NT, 3>(pk, a.n_agg, vk);
+        if constexpr (NT == 64) __syncthreads();
+        block_totals<NT, 3>(tot, sh);
+        if (flag) return;
+        const double delta = tot[0], rho = tot[1] + tot[2];
+        double den = delta;
+        if (k > 0)
+        {
+            beta = rho / rho_prev;
+            den = delta - beta * rho / alpha_prev;
+            // p.Ap from the recurrence can cancel to <= 0 near convergence even
+            // for a positive definite matrix: restart along z (beta = 0, p = z,
+            // p.Ap = z.Az) instead of reporting a breakdown
+            if (!(den > 0.0))
+            {
+                beta = 0.0;
+                den = delta;
+            }
+        }
+        if (!(den > 0.0))
+        {
+            // not positive definite along z: the same decision in every block
+            if (blk == 0 && t == 0)
+            {
+                sc->breakdown = 1;
+                sc->done = -1;
+                sc->iters = k;
+            }
+            return;
+        }
+        alpha = rho / den;
+        if (blk == 0 && t == 0)
+        {
+            sc->rho_hist[k & 1] = rho;
+            sc->alpha_hist[k & 1] = alpha;
+        }
+    }
+    double part[2] = { 0.0, 0.0 };  // r.z, ||r||^2
+    double cr[KC > 0 ? KC : 1];
+#pragma unroll
+    for (int c = 0; c < (KC > 0 ? KC : 1); ++c) cr[c] = 0.0;
+    for (int64_t c0 = lo; c0 < hi; c0 += kUpdVerts)
+    {
+        const int64_t iv = c0 * D + t;
+        const bool in = iv < hi * D;
+        double rv = 0.0;
+        if constexpr (INIT)
+        {
+            if (c0 > lo) __syncthreads();  // the previous chunk's LDS reads are complete
+            // inverse diagonal blocks of this chunk (threads 0 .. 63)
+            if (t < kUpdVerts)
+            {
+                const int64_t v = c0 + t;
+                double B[D * D], o[D * D];
+                bool fr[D];
+#pragma unroll
+                for (int i = 0; i < D; ++i) fr[i] = false;
+#pragma unroll
+                for (int m = 0; m < D * D; ++m) o[m] = 0.0;
+                if (v < hi)
+                {
+                    const int64_t h0 = (int64_t)a.perm[v] * D;
+                    const int32_t dg = a.diag[v];
+#pragma unroll
+                    for (int i = 0; i < D; ++i)
+                    {
+                        fr[i] = a.free_h ? a.free_h[h0 + i] != 0 : true;
+                        if (a.free_h) a.free_s[v * D + i] = fr[i] ? 1 : 0;
+                    }
+                    // reduced basis: a fixed component takes a unit row /
+                    // column here and a zero row / column in the inverse (the
+                    // free sub-block's inverse); a handle used by no element
+                    // has no block: (w I + H) is w I there
+#pragma unroll
+                    for (int i = 0; i < D; ++i)
+#pragma unroll
+                        for (int j = 0; j < D; ++j)
+                        {
+                            const double hb = dg < 0 ? 0.0 : a.Hs[(int64_t)dg * (D * D) + i * D + j];
+                            const double e = hb + (i == j ? (dg < 0 && !(a.w > 0.0) ? 1.0 : a.w) : 0.0);
+                            B[i * D + j] = (fr[i] && fr[j]) ? e : (i == j ? 1.0 : 0.0);
+                        }
+                    invert_block<D>(B, o);
+                }
+                // the upper triangle: the inverse of a symmetric block is
+                // symmetric (the cofactor products commute)
+#pragma unroll
+                for (int i = 0; i < D; ++i)
+#pragma unroll
+                    for (int j = i; j < D; ++j)
+                    {
+                        const double e = (fr[i] && fr[j]) ? o[i * D + j] : 0.0;
+                        sD[t * PB + PackedBlock<D>::at(i, j)] = e;
+                        if (v < hi) a.Dinv[v * PB + PackedBlock<D>::at(i, j)] = e;
+                    }
+            }
+            if (in)
+            {
+                rv = (a.free_h && !a.free_h[(int64_t)a.perm[iv / D] * D + iv % D]) ? 0.0 : rc;
+                a.x[iv] = 0.0;
+                a.r[iv] = rv;
+            }
+        }
+        else if (in)
+        {
+            const double pi = k > 0 ? fma(beta, pc, zc) : zc;
+            const double qi = k > 0 ? fma(beta, qc, sc_) : sc_;
+            a.p[iv] = pi;
+            a.q[iv] = qi;
+            a.x[iv] = xc + alpha * pi;
+            rv = rc - alpha * qi;
+            if (a.free_h && !a.free_s[iv]) rv = 0.0;  // reduced basis: no residual on fixed variables
+            a.r[iv] = rv;
+        }
+        if (!INIT && c0 > lo) __syncthreads();  // the previous chunk's LDS reads are complete
+        sR[t] = rv;
+        if constexpr (ROT) sV[t] = vc;
+        if constexpr (!INIT)
+        {
+#pragma unroll
+            for (int m = 0; m < ND; ++m) sD[t + m * NT] = dc[m];
+        }
+        __syncthreads();
+        if (c0 + kUpdVerts < hi) load(c0 + kUpdVerts);  // next chunk in flight during this one's z
+        if (in)
+        {
+            const int vl = t / D, i = t - vl * D;
+            double zi = 0.0;
+#pragma unroll
+            for (int j = 0; j < D; ++j) zi += sD[vl * PB + PackedBlock<D>::at(i, j)] * sR[vl * D + j];
+            a.z[iv] = zi;
+            part[0] += rv * zi;
+            part[1] += rv * rv;
+        }
+        if constexpr (KC > 0)
+        {
+            if (t < kUpdVerts)  // sR is 0 past the part's end
+            {
+                double dv[D], R[D][KC];
+#pragma unroll
+                for (int i = 0; i < D; ++i) dv[i] = ROT ? sV[ROT ? t * D + i : 0] : 0.0;
+                if (c0 + t >= hi)
+                {
+#pragma unroll
+                    for (int i = 0; i < D; ++i) dv[i] = 0.0;
+                }
+                coarse_rows<D, KC>(dv, R);
+#pragma unroll
+                for (int i = 0; i < D; ++i)
+#pragma unroll
+                    for (int c = 0; c < KC; ++c) cr[c] += R[i][c] * sR[t * D + i];
+            }
+        }
+    }
+    if constexpr (KC > 0)
+    {
+        if (t < 64)
+        {
+#pragma unroll
+            for (int c = 0; c < KC; ++c) cr[c] = wave_total(cr[c]);
+            double v = cr[0];
+#pragma unroll
+            for (int c = 1; c < KC; ++c) v = t == c ? cr[c] : v;
+            const int64_t ag = blk / a.ppa, p = blk - ag * a.ppa;
+            if (t < KC) a.rpart[p * a.nc + ag * KC + t] = v;
+        }
+    }
+    block_totals<NT, 2>(part, sh2);
+    if (t == 0)
+    {
+        a.parts[Gs + (k & 1) * Gv + blk] = part[0];
+        a.parts[Gs + 2 * Gv + (k & 1) * Gv + blk] = part[1];
+    }
+}
+
 // sum over the 64 lanes of a wave, fixed xor tree (every lane gets the total)
 template <int L>
 __device__ __forceinline__ void wave_sum(double* v)
 {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-        for (int m = 0; m < L; ++m) v[m] += __shfl_xor(v[m], off, 64);
+    for (int m = 0; m < L; ++m) v[m] = wave_total(v[m]);
 }
 
+// Lever arms dv_v = x_v - x_(first member of v's aggregate), in handle order
+// (Galerkin sums) and in solver order (CG iterations).
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_coarse_dvec(int64_t nh, const double* __restrict__ x,
                                                         const int32_t* __restrict__ agg_of,
                                                         const int32_t* __restrict__ agg_ptr,
-                                                        const int32_t* __restrict__ agg_vert, double* __restrict__ dvec)
+                                                        const int32_t* __restrict__ perm, double* __restrict__ dvec_h,
+                                                        double* __restrict__ dvec)
 {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nh) return;
-    const int64_t root = agg_vert[agg_ptr[agg_of[v]]];
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i0 >= nh) return;
+    const int64_t v = perm[i0];
+    const int64_t root = perm[agg_ptr[agg_of[v]]];
 #pragma unroll
-    for (int i = 0; i < D; ++i) dvec[v * D + i] = x[v * D + i] - x[root * D + i];
+    for (int i = 0; i < D; ++i)
+    {
+        const double e = x[v * D + i] - x[root * D + i];
+        dvec_h[v * D + i] = e;
+        dvec[i0 * D + i] = e;
+    }
 }
 
 // one wave per chunk of a coarse block pair's fine blocks (u, v): sum of
@@ -1136,208 +1139,124 @@ __global__ __launch_bounds__(kBlock) void k_shift_diagonal(int64_t n, double* __
     A[j + j * n] = a == 0.0 ? 1.0 : a * (1.0 + rel);
 }
 
-__global__ __launch_bounds__(kBlock) void k_symmetrize_lower(int64_t n, double* __restrict__ A)
-{
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n * n) return;
-    const int64_t i = id % n, j = id / n;  // entry (i, j), column-major
-    if (i < j) A[i + j * n] = A[j + i * n];
-}
+// Coarse product and prolongation in one launch, one workgroup of
+// kCoarseBlock threads per aggregate a: r_c = the ppa rows of restriction
+// partials, y_a = rows a KC .. a KC + KC - 1 of A_c^-1 r_c (row i of the
+// symmetric inverse is its contiguous column i; thread t takes the entries t,
+// t + kCoarseBlock, ..., then a fixed wave tree and the waves' partials in
+// order), one partial r_c[a] . y_a, then z_v += R_v y_a for every member v of
+// the aggregate.  The first loads of every kind are issued before the
+// termination flag is looked at (100 x 100 grid 5.7 -> 4.0 us, 60^3 cube 12.8
+// -> 10.5 us, of which 30 MB are the FP32 inverse).  60^3 cube, 459
+// aggregates, per CG iteration: 512 and 256 lanes alike, 1,024 2 us slower.
+constexpr int kCoarseBlock = 512;
 
-// r_c = P^T r: one wave per chunk of an aggregate's handles, then one
-// thread per coarse unknown sums its aggregate's chunk partials in order
-template <int D, int KC>
-__global__ __launch_bounds__(kBlock) void k_coarse_restrict_chunk(int64_t n_chunks,
-                                                                  const int32_t* __restrict__ chunk_ptr,
-                                                                  const int32_t* __restrict__ agg_vert,
-                                                                  const double* __restrict__ dvec,
-                                                                  const double* __restrict__ r,
-                                                                  double* __restrict__ part, PcgScalars* sc)
+template <int D, int KC, class TA>
+__global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem a, const TA* __restrict__ Ainv, int k,
+                                                                       const int* __restrict__ kdev)
 {
-    if (block_done(sc)) return;
-    const int lane = threadIdx.x & 63;
-    const int64_t ch = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (ch >= n_chunks) return;
+    constexpr int NW = kCoarseBlock / 64;
+    __shared__ double wpart[NW][KC];
+    __shared__ double y[KC], ry[KC];
+    __shared__ int flag;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int done_v = t == 0 ? a.sc->done : 0;
+    const int slot = (kdev ? *kdev : k) & 1;
+    const int64_t ag = blockIdx.x, nc = a.nc;
+    const TA* __restrict__ col = Ainv + ag * KC * nc;
+    const double* __restrict__ rpart = a.rpart;
+    const int ppa = a.ppa;
+    auto rc = [&](int64_t j) {
+        double v[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[p] = p < ppa ? rpart[p * nc + j] : 0.0;
+        double e = ((v[0] + v[1]) + v[2]) + v[3];
+        for (int p = 4; p < ppa; ++p) e += rpart[p * nc + j];
+        return e;
+    };
     double acc[KC];
 #pragma unroll
     for (int c = 0; c < KC; ++c) acc[c] = 0.0;
-    const int64_t m1 = chunk_ptr[ch + 1];
-    for (int64_t m = chunk_ptr[ch] + lane; m < m1; m += 64)
+    int64_t j = t;
+    if (j < nc)
     {
-        const int64_t v = agg_vert[m];
-        double R[D][KC];
-        coarse_rows<D, KC>(dvec + v * D, R);
+        const double rj = rc(j);
+#pragma unroll
+        for (int c = 0; c < KC; ++c) acc[c] = (double)col[c * nc + j] * rj;
+    }
+    const double rown = t < KC ? rc(ag * KC + t) : 0.0;
+    // this thread's first member
+    const int64_t m0 = a.agg_ptr[ag], m1 = a.agg_ptr[ag + 1];
+    double zv[D], dv[D];
+    auto member = [&](int64_t v) {
 #pragma unroll
         for (int i = 0; i < D; ++i)
         {
-            const double ri = r[v * D + i];
-#pragma unroll
-            for (int c = 0; c < KC; ++c) acc[c] += R[i][c] * ri;
+            zv[i] = a.z[v * D + i];
+            dv[i] = KC > D ? a.dvec[v * D + i] : 0.0;
         }
-    }
-    wave_sum<KC>(acc);
-#pragma unroll
-    for (int c = 0; c < KC; ++c)
-        if (lane == c) part[ch * KC + c] = acc[c];
-}
-
-template <int KC>
-__global__ __launch_bounds__(kBlock) void k_coarse_restrict_sum(int64_t n_agg, const int32_t* __restrict__ agg_chunk,
-                                                                const double* __restrict__ part,
-                                                                double* __restrict__ rc, PcgScalars* sc)
-{
-    if (block_done(sc)) return;
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n_agg * KC) return;
-    const int64_t a = id / KC;
-    const int c = (int)(id % KC);
-    double t = 0.0;
-    for (int32_t ch = agg_chunk[a]; ch < agg_chunk[a + 1]; ++ch) t += part[(int64_t)ch * KC + c];
-    rc[id] = t;
-}
-
-// Both restriction stages in one launch: one workgroup of kCoarseBlock
-// threads per aggregate, its waves take the aggregate's chunks in turn (each
-// chunk reduced exactly as by k_coarse_restrict_chunk), the chunk partials go
-// to LDS and are summed in chunk order as by k_coarse_restrict_sum, so r_c
-// has the same bits.  For aggregates of at most kRestrictMaxChunks chunks.
-constexpr int kRestrictMaxChunks = 64;
-// lanes per aggregate in the restriction and the coarse product (60^3 tet
-// cube, 459 aggregates: 512 and 256 22.4 us per CG iteration for both
-// kernels, 1,024 24.2 us)
-constexpr int kCoarseBlock = 512;
-
-template <int D, int KC>
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_restrict(const int32_t* __restrict__ agg_chunk,
-                                                            const int32_t* __restrict__ chunk_ptr,
-                                                            const int32_t* __restrict__ agg_vert,
-                                                            const double* __restrict__ dvec,
-                                                            const double* __restrict__ r, double* __restrict__ rc,
-                                                            PcgScalars* sc)
-{
-    if (block_done(sc)) return;
-    __shared__ double cpart[kRestrictMaxChunks * KC];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t a = blockIdx.x;
-    const int32_t c0 = agg_chunk[a], c1 = agg_chunk[a + 1];
-    for (int32_t ch = c0 + wv; ch < c1; ch += kCoarseBlock / 64)
-    {
-        double acc[KC];
-#pragma unroll
-        for (int c = 0; c < KC; ++c) acc[c] = 0.0;
-        const int64_t m1 = chunk_ptr[ch + 1];
-        for (int64_t m = chunk_ptr[ch] + lane; m < m1; m += 64)
-        {
-            const int64_t v = agg_vert[m];
-            double R[D][KC];
-            coarse_rows<D, KC>(dvec + v * D, R);
-#pragma unroll
-            for (int i = 0; i < D; ++i)
-            {
-                const double ri = r[v * D + i];
-#pragma unroll
-                for (int c = 0; c < KC; ++c) acc[c] += R[i][c] * ri;
-            }
-        }
-        wave_sum<KC>(acc);
-#pragma unroll
-        for (int c = 0; c < KC; ++c)
-            if (lane == c) cpart[(ch - c0) * KC + c] = acc[c];
-    }
+    };
+    if (m0 + t < m1) member(m0 + t);
+    if (t == 0) flag = done_v;
     __syncthreads();
-    if (threadIdx.x < KC)
+    if (flag) return;
+    for (j += kCoarseBlock; j < nc; j += kCoarseBlock)
     {
-        double t = 0.0;
-        for (int32_t k = 0; k < c1 - c0; ++k) t += cpart[k * KC + threadIdx.x];
-        rc[a * KC + threadIdx.x] = t;
-    }
-}
-
-// Coarse product and prolongation in one launch, one workgroup of
-// kCoarseBlock threads per aggregate a: y_a = rows a KC .. a KC + KC - 1 of
-// A_c^-1 r_c (row i of the symmetric inverse is its contiguous column i;
-// thread t takes the entries t, t + kCoarseBlock, ..., then a fixed wave tree
-// and the waves' partials in order), one partial r_c[a] . y_a, then
-// z_v += R_v y_a for every member v of the aggregate.
-template <int D, int KC, class TA>
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(int64_t nc, const TA* __restrict__ Ainv,
-                                                                       const double* __restrict__ rc,
-                                                                       const int32_t* __restrict__ agg_ptr,
-                                                                       const int32_t* __restrict__ agg_vert,
-                                                                       const double* __restrict__ dvec,
-                                                                       const unsigned char* __restrict__ free_vars,
-                                                                       double* __restrict__ z,
-                                                                       double* __restrict__ cparts_all, int slot,
-                                                                       int Gc, const int* __restrict__ kdev,
-                                                                       PcgScalars* sc)
-{
-    if (block_done(sc)) return;
-    double* __restrict__ cparts = cparts_all + (int64_t)(kdev ? (*kdev & 1) : slot) * Gc;
-    constexpr int NW = kCoarseBlock / 64;
-    __shared__ double wpart[NW][KC];
-    __shared__ double y[KC];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t a = blockIdx.x;
-    const TA* __restrict__ col = Ainv + a * KC * nc;
-    double acc[KC];
-#pragma unroll
-    for (int c = 0; c < KC; ++c) acc[c] = 0.0;
-    for (int64_t j = threadIdx.x; j < nc; j += kCoarseBlock)
-    {
-        const double rj = rc[j];
+        const double rj = rc(j);
 #pragma unroll
         for (int c = 0; c < KC; ++c) acc[c] += (double)col[c * nc + j] * rj;
     }
     wave_sum<KC>(acc);
-#pragma unroll
-    for (int c = 0; c < KC; ++c)
-        if (lane == c) wpart[wv][c] = acc[c];
-    __syncthreads();
-    if (threadIdx.x < KC)
+    if (lane == 0)
     {
-        double t = 0.0;
 #pragma unroll
-        for (int k = 0; k < NW; ++k) t += wpart[k][threadIdx.x];
-        y[threadIdx.x] = t;
+        for (int c = 0; c < KC; ++c) wpart[wv][c] = acc[c];
     }
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (t < KC)
     {
-        double t = 0.0;
+        double v = 0.0;
 #pragma unroll
-        for (int c = 0; c < KC; ++c) t += rc[a * KC + c] * y[c];
-        cparts[a] = t;
+        for (int w = 0; w < NW; ++w) v += wpart[w][t];
+        y[t] = v;
+        ry[t] = rown * v;
+    }
+    __syncthreads();
+    if (t == 0)
+    {
+        double v = 0.0;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) v += ry[c];
+        a.cparts[slot * a.n_agg + ag] = v;
     }
     double ya[KC];
 #pragma unroll
     for (int c = 0; c < KC; ++c) ya[c] = y[c];
-    const int32_t m1 = agg_ptr[a + 1];
-    for (int32_t m = agg_ptr[a] + threadIdx.x; m < m1; m += kCoarseBlock)
+    for (int64_t v = m0 + t; v < m1; v += kCoarseBlock)
     {
-        const int64_t v = agg_vert[m];
+        if (v != m0 + t) member(v);
         double R[D][KC];
-        coarse_rows<D, KC>(dvec + v * D, R);
+        coarse_rows<D, KC>(dv, R);
 #pragma unroll
         for (int i = 0; i < D; ++i)
         {
-            if (free_vars && !free_vars[v * D + i]) continue;
-            double t = z[v * D + i];
+            if (a.free_h && !a.free_s[v * D + i]) continue;
+            double e = zv[i];
 #pragma unroll
-            for (int c = 0; c < KC; ++c) t += R[i][c] * ya[c];
-            z[v * D + i] = t;
+            for (int c = 0; c < KC; ++c) e += R[i][c] * ya[c];
+            a.z[v * D + i] = e;
         }
     }
 }
 
-int coarse_apply_groups(int64_t n_agg) { return (int)std::max<int64_t>(1, n_agg); }
-
-hipError_t launch_coarse_dvec(int d, int64_t nh, const double* x, const CoarseDev& c, double* dvec, hipStream_t s)
+hipError_t launch_coarse_dvec(int d, int64_t nh, const double* x, const int32_t* agg_of, const int32_t* agg_ptr,
+                              const int32_t* perm, double* dvec_h, double* dvec, hipStream_t s)
 {
     if (nh == 0) return hipSuccess;
     const unsigned g = (unsigned)((nh + kBlock - 1) / kBlock);
-    if (d == 1) k_coarse_dvec<1><<<g, kBlock, 0, s>>>(nh, x, c.agg_of, c.agg_ptr, c.agg_vert, dvec);
-    else if (d == 2) k_coarse_dvec<2><<<g, kBlock, 0, s>>>(nh, x, c.agg_of, c.agg_ptr, c.agg_vert, dvec);
-    else k_coarse_dvec<3><<<g, kBlock, 0, s>>>(nh, x, c.agg_of, c.agg_ptr, c.agg_vert, dvec);
+    if (d == 1) k_coarse_dvec<1><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
+    else if (d == 2) k_coarse_dvec<2><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
+    else k_coarse_dvec<3><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
     return hipGetLastError();
 }
 
@@ -1345,29 +1264,32 @@ template <int D, int KC>
 static void galerkin_t(int64_t n_pairs, int64_t n_gchunks, const int64_t* gchunk_ptr, const int32_t* pair_chunk,
                        const int32_t* pair_blocks, const int32_t* pair_ab, const int32_t* block_row,
                        const int32_t* brow_ptr, const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
-                       const CoarseDev& c, double* gpart, double* Ac, hipStream_t s)
+                       const double* dvec_h, const unsigned char* free_vars, int64_t nc, double* gpart, double* Ac,
+                       hipStream_t s)
 {
     const unsigned g1 = (unsigned)((n_gchunks * 64 + kBlock - 1) / kBlock);
     k_coarse_galerkin_chunk<D, KC><<<g1, kBlock, 0, s>>>(n_gchunks, gchunk_ptr, pair_blocks, block_row, brow_ptr,
-                                                          bcol, row_ptr, H, w, c.dvec, c.free_vars, gpart);
+                                                          bcol, row_ptr, H, w, dvec_h, free_vars, gpart);
     const unsigned g2 = (unsigned)((n_pairs * KC * KC + kBlock - 1) / kBlock);
-    k_coarse_galerkin_pairs<KC><<<g2, kBlock, 0, s>>>(n_pairs, pair_chunk, pair_ab, gpart, c.nc, Ac);
+    k_coarse_galerkin_pairs<KC><<<g2, kBlock, 0, s>>>(n_pairs, pair_chunk, pair_ab, gpart, nc, Ac);
 }
 
-hipError_t launch_coarse_galerkin(int d, int64_t n_pairs, int64_t n_gchunks, const int64_t* gchunk_ptr,
-                                  const int32_t* pair_chunk, const int32_t* pair_blocks, const int32_t* pair_ab,
-                                  const int32_t* block_row, const int32_t* brow_ptr, const int32_t* bcol,
-                                  const int32_t* row_ptr, const double* H, double w, const CoarseDev& c,
-                                  double* gpart, double* Ac, hipStream_t s)
+hipError_t launch_coarse_galerkin(int d, int kc, int64_t nc, int64_t n_pairs, int64_t n_gchunks,
+                                  const int64_t* gchunk_ptr, const int32_t* pair_chunk, const int32_t* pair_blocks,
+                                  const int32_t* pair_ab, const int32_t* block_row, const int32_t* brow_ptr,
+                                  const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
+                                  const double* dvec_h, const unsigned char* free_vars, double* gpart, double* Ac,
+                                  hipStream_t s)
 {
     if (n_pairs == 0) return hipSuccess;
 #define TAD_GALERKIN(DD, KK) galerkin_t<DD, KK>(n_pairs, n_gchunks, gchunk_ptr, pair_chunk, pair_blocks, pair_ab, \
-                                                 block_row, brow_ptr, bcol, row_ptr, H, w, c, gpart, Ac, s)
-    if (d == 3 && c.kc == 6) TAD_GALERKIN(3, 6);
-    else if (d == 3 && c.kc == 3) TAD_GALERKIN(3, 3);
-    else if (d == 2 && c.kc == 3) TAD_GALERKIN(2, 3);
-    else if (d == 2 && c.kc == 2) TAD_GALERKIN(2, 2);
-    else if (d == 1 && c.kc == 1) TAD_GALERKIN(1, 1);
+                                                 block_row, brow_ptr, bcol, row_ptr, H, w, dvec_h, free_vars, nc, \
+                                                 gpart, Ac, s)
+    if (d == 3 && kc == 6) TAD_GALERKIN(3, 6);
+    else if (d == 3 && kc == 3) TAD_GALERKIN(3, 3);
+    else if (d == 2 && kc == 3) TAD_GALERKIN(2, 3);
+    else if (d == 2 && kc == 2) TAD_GALERKIN(2, 2);
+    else if (d == 1 && kc == 1) TAD_GALERKIN(1, 1);
     else return hipErrorInvalidValue;
 #undef TAD_GALERKIN
     return hipGetLastError();
@@ -1434,177 +1356,114 @@ hipError_t launch_coarse_to32(int64_t n, const double* A, double delta, float* A
     return hipGetLastError();
 }
 
-hipError_t launch_symmetrize_lower(int64_t n, double* A, hipStream_t s)
+constexpr int kSpmvLanes = 8;
+
+int pcg_spmv_groups(int64_t nh)
 {
-    if (n == 0) return hipSuccess;
-    k_symmetrize_lower<<<(unsigned)((n * n + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, A);
+    // SpMV: kSpmvLanes lanes per block row, at most 1,024 workgroups (60^3
+    // tet cube, 227K block rows: 8 lanes and 1,024 workgroups 40.7 us per
+    // product against 42.1 with 768, 49.4 with 512, 43.1 with 1,536 and 44.8
+    // with 2,048; 16 lanes with 2,048 workgroups 47.3, 4 lanes with 1,536
+    // 50.1), a multiple of 8 (the XCDs) from 8 on
+    const int64_t rows_per_block = kBlock / kSpmvLanes;
+    const int64_t gs = std::max<int64_t>(1, std::min<int64_t>((nh + rows_per_block - 1) / rows_per_block, 1024));
+    return (int)(gs < 8 ? gs : (gs + 7) / 8 * 8);
+}
+
+int64_t pcg_parts_size(int64_t Gs, int64_t Gv) { return Gs + 4 * Gv; }
+
+hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* place, const double* H, double* sym_H, hipStream_t s)
+{
+    if (n_sym == 0) return hipSuccess;
+    const unsigned grid = (unsigned)((n_sym * d * d + kBlock - 1) / kBlock);
+    const int2* pl = reinterpret_cast<const int2*>(place);
+    if (d == 1) k_sym_pack<1><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
+    else if (d == 2) k_sym_pack<2><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
+    else k_sym_pack<3><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
+    return hipGetLastError();
+}
+
+template <int D>
+static void spmv_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
+{
+    if (a.Gs % 8 == 0) k_spmv_sym<D, kSpmvLanes, true><<<a.Gs, kBlock, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+    else k_spmv_sym<D, kSpmvLanes, false><<<a.Gs, kBlock, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+}
+
+template <int D, int KC>
+static void update_t(const PcgSystem& a, int k, const int* kdev, bool init, hipStream_t s)
+{
+    if (init) k_pcg_update<D, KC, true><<<a.Gv, kUpdVerts * D, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+    else k_pcg_update<D, KC, false><<<a.Gv, kUpdVerts * D, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+}
+
+static hipError_t update_any(int d, const PcgSystem& a, int k, const int* kdev, bool init, hipStream_t s)
+{
+    if (d == 3 && a.kc == 6) update_t<3, 6>(a, k, kdev, init, s);
+    else if (d == 3 && a.kc == 3) update_t<3, 3>(a, k, kdev, init, s);
+    else if (d == 3 && a.kc == 0) update_t<3, 0>(a, k, kdev, init, s);
+    else if (d == 2 && a.kc == 3) update_t<2, 3>(a, k, kdev, init, s);
+    else if (d == 2 && a.kc == 2) update_t<2, 2>(a, k, kdev, init, s);
+    else if (d == 2 && a.kc == 0) update_t<2, 0>(a, k, kdev, init, s);
+    else if (d == 1 && a.kc == 1) update_t<1, 1>(a, k, kdev, init, s);
+    else if (d == 1 && a.kc == 0) update_t<1, 0>(a, k, kdev, init, s);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
 template <int D, int KC>
-static void coarse_correction_t(int64_t nh, const CoarseDev& c, const double* r, double* z, int slot, PcgScalars* sc,
-                                hipStream_t s, const int* kdev)
+static void coarse_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
 {
-    if (c.max_agg_chunks <= kRestrictMaxChunks)
-    {
-        k_coarse_restrict<D, KC><<<(unsigned)c.n_agg, kCoarseBlock, 0, s>>>(c.agg_chunk, c.chunk_ptr, c.agg_vert,
-                                                                            c.dvec, r, c.rc, sc);
-    }
+    if (a.Ainv32)
+        k_coarse_apply_prolong<D, KC, float><<<(unsigned)a.n_agg, kCoarseBlock, 0, s>>>(a, a.Ainv32, k, kdev);
     else
-    {
-        const unsigned gch = (unsigned)((c.n_chunks * 64 + kBlock - 1) / kBlock);
-        k_coarse_restrict_chunk<D, KC><<<gch, kBlock, 0, s>>>(c.n_chunks, c.chunk_ptr, c.agg_vert, c.dvec, r,
-                                                               c.chunk_part, sc);
-        const unsigned gs = (unsigned)((c.n_agg * KC + kBlock - 1) / kBlock);
-        k_coarse_restrict_sum<KC><<<gs, kBlock, 0, s>>>(c.n_agg, c.agg_chunk, c.chunk_part, c.rc, sc);
-    }
-    if (c.Ainv32)
-        k_coarse_apply_prolong<D, KC, float><<<(unsigned)c.n_agg, kCoarseBlock, 0, s>>>(
-            c.nc, c.Ainv32, c.rc, c.agg_ptr, c.agg_vert, c.dvec, c.free_vars, z, c.cparts, slot, c.Gc, kdev, sc);
-    else
-        k_coarse_apply_prolong<D, KC, double><<<(unsigned)c.n_agg, kCoarseBlock, 0, s>>>(
-            c.nc, c.Ainv, c.rc, c.agg_ptr, c.agg_vert, c.dvec, c.free_vars, z, c.cparts, slot, c.Gc, kdev, sc);
+        k_coarse_apply_prolong<D, KC, double><<<(unsigned)a.n_agg, kCoarseBlock, 0, s>>>(a, a.Ainv, k, kdev);
 }
 
-hipError_t launch_coarse_correction(int d, int64_t nh, const CoarseDev& c, const double* r, double* z, int slot,
-                                    PcgScalars* sc, hipStream_t s, Timer* timer, const int* kdev)
+// z += P A_c^-1 P^T r with the restricted residual's parts of the last update
+static hipError_t coarse_any(int d, const PcgSystem& a, int k, const int* kdev, hipStream_t s, Timer* timer)
 {
-    if (c.kc == 0 || c.n_agg == 0) return hipSuccess;
+    if (a.kc == 0) return hipSuccess;
     if (timer) timer->begin("pcg_coarse", s);
-    if (d == 3 && c.kc == 6) coarse_correction_t<3, 6>(nh, c, r, z, slot, sc, s, kdev);
-    else if (d == 3 && c.kc == 3) coarse_correction_t<3, 3>(nh, c, r, z, slot, sc, s, kdev);
-    else if (d == 2 && c.kc == 3) coarse_correction_t<2, 3>(nh, c, r, z, slot, sc, s, kdev);
-    else if (d == 2 && c.kc == 2) coarse_correction_t<2, 2>(nh, c, r, z, slot, sc, s, kdev);
-    else if (d == 1 && c.kc == 1) coarse_correction_t<1, 1>(nh, c, r, z, slot, sc, s, kdev);
+    if (d == 3 && a.kc == 6) coarse_t<3, 6>(a, k, kdev, s);
+    else if (d == 3 && a.kc == 3) coarse_t<3, 3>(a, k, kdev, s);
+    else if (d == 2 && a.kc == 3) coarse_t<2, 3>(a, k, kdev, s);
+    else if (d == 2 && a.kc == 2) coarse_t<2, 2>(a, k, kdev, s);
+    else if (d == 1 && a.kc == 1) coarse_t<1, 1>(a, k, kdev, s);
     else return hipErrorInvalidValue;
     if (timer) timer->end("pcg_coarse", s);
     return hipGetLastError();
 }
 
-constexpr int kSpmvLanes = 8;
-
-void pcg_grids(int d, int64_t nh, int* Gs, int* Gv)
+hipError_t launch_pcg_init(int d, const PcgSystem& a, hipStream_t s)
 {
-    // SpMV: kSpmvLanes lanes per block row, at most 1,024 workgroups (60^3
-    // tet cube, 227K block rows: 8 lanes and 1,024 workgroups 40.7 us per
-    // product against 42.1 with 768, 49.4 with 512, 43.1 with 1,536 and 44.8
-    // with 2,048; 16 lanes with 2,048 workgroups 47.3, 4 lanes with 1,536 50.1)
-    (void)d;
-    const int64_t rows_per_block = kBlock / kSpmvLanes;
-    const int64_t gs = (nh + rows_per_block - 1) / rows_per_block;
-    const int64_t gv = (nh + kUpdVerts - 1) / kUpdVerts;
-    *Gs = (int)std::max<int64_t>(1, std::min<int64_t>(gs, 1024));
-    *Gv = (int)std::max<int64_t>(1, std::min<int64_t>(gv, 1024));
+    const hipError_t e = update_any(d, a, -1, nullptr, true, s);
+    return e != hipSuccess ? e : coarse_any(d, a, -1, nullptr, s, nullptr);
 }
 
-int64_t pcg_parts_size(int d, int64_t nh)
+hipError_t launch_pcg_iteration(int d, const PcgSystem& a, int k, bool with_update, hipStream_t s, Timer* timer,
+                                bool read_k)
 {
-    int Gs, Gv;
-    pcg_grids(d, nh, &Gs, &Gv);
-    return Gs + 5 * (int64_t)Gv;
-}
-
-hipError_t launch_pcg_setup(int d, int64_t nh, const int32_t* brow_ptr, const int32_t* diag_block,
-                            const int32_t* row_ptr, const double* H, double w, const unsigned char* free_vars,
-                            double* Dinv, hipStream_t s)
-{
-    const unsigned grid = (unsigned)((nh + kBlock - 1) / kBlock);
-    if (d == 1) k_pcg_setup<1><<<grid, kBlock, 0, s>>>(nh, brow_ptr, diag_block, row_ptr, H, w, free_vars, Dinv);
-    else if (d == 2) k_pcg_setup<2><<<grid, kBlock, 0, s>>>(nh, brow_ptr, diag_block, row_ptr, H, w, free_vars, Dinv);
-    else k_pcg_setup<3><<<grid, kBlock, 0, s>>>(nh, brow_ptr, diag_block, row_ptr, H, w, free_vars, Dinv);
-    return hipGetLastError();
-}
-
-hipError_t launch_pcg_init(int d, int64_t nh, const double* b, const unsigned char* free_vars, const double* Dinv,
-                           double* x, double* r, double* z, double* parts, PcgScalars* sc, const CoarseDev* co,
-                           hipStream_t s)
-{
-    int Gs, Gv;
-    pcg_grids(d, nh, &Gs, &Gv);
-    if (d == 1) k_pcg_init<1><<<Gv, kBlock, 0, s>>>(nh, b, free_vars, Dinv, x, r, z, parts, Gs, Gv, sc);
-    else if (d == 2) k_pcg_init<2><<<Gv, kBlock, 0, s>>>(nh, b, free_vars, Dinv, x, r, z, parts, Gs, Gv, sc);
-    else k_pcg_init<3><<<Gv, kBlock, 0, s>>>(nh, b, free_vars, Dinv, x, r, z, parts, Gs, Gv, sc);
-    // z_0 gets the coarse correction; its r.z partials join rho_0 in slot 1
-    if (co && co->kc > 0 && co->n_agg > 0)
-    {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        return launch_coarse_correction(d, nh, *co, r, z, 1, sc, s, nullptr);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* sym_full, const int32_t* block_row,
-                           const int32_t* brow_ptr, const int32_t* bcol, const int32_t* row_ptr, const double* H,
-                           double* sym_H, hipStream_t s)
-{
-    if (n_sym == 0) return hipSuccess;
-    const unsigned grid = (unsigned)((n_sym * d * d + kBlock - 1) / kBlock);
-    if (d == 1)
-        k_sym_pack<1><<<grid, kBlock, 0, s>>>(n_sym, sym_full, block_row, brow_ptr, bcol, row_ptr, H, sym_H);
-    else if (d == 2)
-        k_sym_pack<2><<<grid, kBlock, 0, s>>>(n_sym, sym_full, block_row, brow_ptr, bcol, row_ptr, H, sym_H);
-    else
-        k_sym_pack<3><<<grid, kBlock, 0, s>>>(n_sym, sym_full, block_row, brow_ptr, bcol, row_ptr, H, sym_H);
-    return hipGetLastError();
-}
-
-template <int D, int LPB>
-static void spmv_sym_t(int64_t nh, const int32_t* brow_ptr, const int32_t* bcol, const int32_t* src,
-                       const double* Hs, double w, const double* z, double* sv, double* parts, int Gs, int Gv, int k,
-                       const int* kdev, PcgScalars* sc, hipStream_t s)
-{
-    if (Gs % 8 == 0)
-        k_spmv_sym<D, LPB, true><<<Gs, kBlock, 0, s>>>(nh, brow_ptr, bcol, src, Hs, w, z, sv, parts, Gs, Gv, k,
-                                                        kdev, sc);
-    else
-        k_spmv_sym<D, LPB, false><<<Gs, kBlock, 0, s>>>(nh, brow_ptr, bcol, src, Hs, w, z, sv, parts, Gs, Gv, k,
-                                                         kdev, sc);
-}
-
-hipError_t launch_pcg_iteration(int d, int64_t nh, const int32_t* brow_ptr, const int32_t* bcol,
-                                const int32_t* sym_src, const double* sym_H, double w, const double* Dinv, double* x,
-                                double* r, double* z, double* pbuf, double* q, double* parts, PcgScalars* sc, int k,
-                                bool with_update, const unsigned char* free_vars, const CoarseDev* co, hipStream_t s,
-                                Timer* timer, bool read_k)
-{
-    const int* kdev = read_k ? &sc->k : nullptr;
-    const bool coarse = co && co->kc > 0 && co->n_agg > 0;
-    const double* cparts = coarse ? co->cparts : nullptr;
-    const int Gc = coarse ? co->Gc : 0;
-    int Gs, Gv;
-    pcg_grids(d, nh, &Gs, &Gv);
-    double* p = pbuf;
-    double* sv = pbuf + nh * d;
-    if (!sym_H || !sym_src) return hipErrorInvalidValue;
+    const int* kdev = read_k ? &a.sc->k : nullptr;
     if (timer) timer->begin("spmv", s);
-    if (d == 1)
-        spmv_sym_t<1, kSpmvLanes>(nh, brow_ptr, bcol, sym_src, sym_H, w, z, sv, parts, Gs, Gv, k, kdev, sc, s);
-    else if (d == 2)
-        spmv_sym_t<2, kSpmvLanes>(nh, brow_ptr, bcol, sym_src, sym_H, w, z, sv, parts, Gs, Gv, k, kdev, sc, s);
-    else
-        spmv_sym_t<3, kSpmvLanes>(nh, brow_ptr, bcol, sym_src, sym_H, w, z, sv, parts, Gs, Gv, k, kdev, sc, s);
+    if (d == 1) spmv_t<1>(a, k, kdev, s);
+    else if (d == 2) spmv_t<2>(a, k, kdev, s);
+    else spmv_t<3>(a, k, kdev, s);
     if (timer) timer->end("spmv", s);
-    if (!with_update) return hipGetLastError();
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !with_update) return e;
     if (timer) timer->begin("pcg_update", s);
-    if (d == 1)
-        k_pcg_update<1><<<Gv, kUpdVerts, 0, s>>>(nh, Dinv, x, r, z, p, q, sv, parts, Gs, Gv, k, kdev, cparts, Gc,
-                                                  free_vars, sc);
-    else if (d == 2)
-        k_pcg_update<2><<<Gv, 2 * kUpdVerts, 0, s>>>(nh, Dinv, x, r, z, p, q, sv, parts, Gs, Gv, k, kdev, cparts, Gc,
-                                                      free_vars, sc);
-    else
-        k_pcg_update<3><<<Gv, 3 * kUpdVerts, 0, s>>>(nh, Dinv, x, r, z, p, q, sv, parts, Gs, Gv, k, kdev, cparts, Gc,
-                                                      free_vars, sc);
+    e = update_any(d, a, k, kdev, false, s);
     if (timer) timer->end("pcg_update", s);
-    // z of iteration k + 1 gets the coarse correction; its r.z partials go to
-    // slot k & 1 next to the update's
-    if (coarse)
-    {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        return launch_coarse_correction(d, nh, *co, r, z, k & 1, sc, s, timer, kdev);
-    }
+    return e != hipSuccess ? e : coarse_any(d, a, k, kdev, s, timer);
+}
+
+hipError_t launch_pcg_solution(int d, const PcgSystem& a, hipStream_t s)
+{
+    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((a.nh * d + kBlock - 1) / kBlock, 1024));
+    if (d == 1) k_unpermute<1><<<grid, kBlock, 0, s>>>(a.nh, a.perm, a.x, a.sol);
+    else if (d == 2) k_unpermute<2><<<grid, kBlock, 0, s>>>(a.nh, a.perm, a.x, a.sol);
+    else k_unpermute<3><<<grid, kBlock, 0, s>>>(a.nh, a.perm, a.x, a.sol);
     return hipGetLastError();
 }
 
