@@ -89,3 +89,40 @@ def test_solver_order_edges(ctx, d, n, agg):
     assert st.converged and nrel(x, ref) <= 1e-10 and np.all(x[free == 0] == 0.0)
     x2, st2 = fn.solve(b, free=free, tol=1e-13, w_identity=0.3, coarse_aggregate=agg)
     assert np.array_equal(x, x2) and st.iters == st2.iters
+
+
+# one pivot tile and less, a tile boundary, several tiles, and the largest
+# sizes the dense preconditioner takes (2,400 variables, 1,536 in 3D)
+@pytest.mark.parametrize("kind,n", [("grid", 3), ("grid", 8), ("grid", 17), ("grid", 34), ("cube", 2), ("cube", 3),
+                                    ("cube", 7)])
+def test_small_systems_dense_preconditioner(ctx, kind, n):
+    """Automatic solves of small systems: the dense inverse makes the
+    preconditioned matrix the identity to rounding (condition numbers below
+    1e6), so two CG iterations reach 1e-12; against direct solves, with a
+    free-variable mask, with w, and with a reused inverse of another Hessian
+    (whose preconditioned spectrum is a few percent wide here)."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as spla
+    P = pinned_grid(n) if kind == "grid" else configs.twist_cube(m=n, seed=2)
+    fn = tad.ScalarFunction.from_problem(P, ctx)
+    f, g, H = fn.eval_with_hessian_proj(P.x0)
+    nv = g.size
+    for w in (0.0, 0.3):
+        d, st = fn.solve(g, tol=1e-12, w_identity=w)
+        assert st.converged and st.coarse_unknowns == nv and st.iters <= 2
+        assert nrel(d, spla.spsolve((H + w * sp.identity(nv)).tocsc(), g)) <= 1e-9
+    free = np.ones(nv, dtype=np.uint8)
+    free[: nv // 3] = 0
+    fi = np.nonzero(free)[0]
+    d, st = fn.solve(g, free=free, tol=1e-12)
+    ref = np.zeros(nv)
+    ref[fi] = spla.spsolve(H.tocsr()[fi][:, fi].tocsc(), g[fi])
+    assert st.converged and st.iters <= 2 and nrel(d, ref) <= 1e-9 and np.all(d[free == 0] == 0.0)
+    fn.solve(g, tol=1e-12)
+    scale = 1.0 + 0.05 * np.cos(np.arange(nv))
+    S = sp.diags(scale)
+    H2 = (S @ H @ S).tocsr()  # same pattern, still positive definite
+    H2.sort_indices()
+    d, st = fn.solve(g, H=H2.data, tol=1e-12, coarse_reuse=1)
+    assert st.converged and st.coarse_reused == 1
+    assert nrel(d, spla.spsolve(H2.tocsc(), g)) <= 1e-9

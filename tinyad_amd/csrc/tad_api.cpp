@@ -321,6 +321,11 @@ struct tad_fn_s
         bool factor_valid = false;
         int f_kc = 0;
         double f_w = 0.0;
+        // small systems: the inverse of w I + H (a later solve that asks for
+        // reuse may keep it)
+        DevBuf<double> dense_inv, dense_parts;
+        bool dense_valid = false;
+        double dense_w = 0.0;
         void release()
         {
             ord.release();
@@ -328,6 +333,8 @@ struct tad_fn_s
             pair_chunk.release(); gchunk_ptr.release();
             dvec.release(); dvec_h.release(); Ac.release(); rpart.release(); cparts.release();
             gpart.release(); inv_work.release(); rowsum.release(); Ainv32.release(); info.release();
+            dense_inv.release(); dense_parts.release();
+            dense_valid = false;
             requested = target = 0;
             n_agg = n_pairs = n_gchunks = 0;
             factor_valid = false;
@@ -342,6 +349,7 @@ struct tad_fn_s
     DevBuf<double> bas_v, bas_tv, bas_vec;
     bool x_hess_valid = false;
     int last_solve_iters = 0;  // iterations of the previous solve (first poll of the next one)
+    int last_dense_iters = 1;  // the same with the dense preconditioner
     // CG iterations recorded as a HIP graph (tad_fn_set_solve_graphs): the
     // executable graph and the operands it was recorded with
     int solve_graphs = 0;      // 1 on, 0 off
@@ -1005,12 +1013,29 @@ tad_status build_coarse(tad_fn fn, int target)
 
 // Largest coarse matrix the two-level preconditioner builds (dense FP64 inverse).
 constexpr int64_t kMaxCoarse = 8192;
-// Automatic aggregate size (tad_solve_opts.coarse_aggregate < 0): about
-// kAutoCoarse coarse unknowns up to kAutoHandles handles, growing with the
-// cube root of the handle count above, to at most 2 kAutoCoarse.
-constexpr int64_t kAutoCoarse = 1400;
-constexpr double kAutoHandles = 30000.0;
-constexpr int64_t kAutoMinAggregate = 32;
+// Automatic number of coarse unknowns (tad_solve_opts.coarse_aggregate < 0): a
+// larger coarse space saves CG iterations and costs its inverse once per
+// rebuild.  Rebuilt in every solve, Newton step in ms at (unknowns):
+// pinned grids, 1,600 handles 1.45 (1,200), 1.38 (603), 1.54 (300), 1.92
+// (150); 3,600 1.77 (1,353), 1.75 (675), 1.91 (342); 10,000 2.58 (1,875),
+// 2.37 (945), 2.57 (630); 19,600 3.21 (1,839), 3.14 (1,233), 3.15 (921), 3.71
+// (612); twisted cubes, 3,375 handles 1.66 (1,272), 1.51 (636), 1.73 (324);
+// 9,261 2.18 (1,404), 1.89 (870), 1.82 (438); 29,791 3.02 (1,404), 2.76 (702),
+// 3.06 (468); 97,336 6.36 (2,286), 6.06 (1,530), 6.42 (1,146); 226,981 12.6
+// (2,658), 12.5 (1,776), 12.8 (1,332).  A Newton loop that rebuilds it only
+// every few steps (lagged) pays a fraction of the inverse per step, and takes
+// about twice as many unknowns below 100K handles (1,404 up to 30K, the
+// optimum measured with a rebuild in every 5th step).  In 3D aggregates hold
+// at least 32 handles: the leftovers of smaller ones are often collinear,
+// their rotations dependent and A_c singular.
+constexpr int64_t kAutoMinAggregate2 = 8, kAutoMinAggregate = 32;
+double auto_coarse_unknowns(int d, int64_t nh, bool lagged)
+{
+    const double h = (double)nh;
+    const double most = std::min(2800.0, 1400.0 * std::cbrt(std::max(1.0, h / 30000.0)));
+    if (lagged) return most;
+    return std::min(most, d == 3 ? 700.0 * std::pow(std::max(1.0, h / 30000.0), 0.68) : 700.0 * std::cbrt(h / 4000.0));
+}
 // Largest relative change of the coarse correction accepted from its FP32 copy.
 constexpr double kCoarse32Change = 0.1;
 
@@ -1021,7 +1046,7 @@ constexpr double kCoarse32Change = 0.1;
 // positive definite (block-Jacobi alone then).  With o.coarse_reuse the
 // inverse and lever arms of the previous compatible solve are kept (*reused).
 tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o, const unsigned char* free_dev,
-                        PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused)
+                        PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused, bool lagged)
 {
     *use = false;
     *reused = false;
@@ -1030,15 +1055,11 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     if (o.coarse_aggregate == 0 || nh == 0 || fn->n_blocks == 0) return TAD_OK;
     const bool rot = fn->x_hess_valid && d >= 2;
     const int kc = rot ? (d == 3 ? 6 : 3) : d;
-    // automatic size (measured optimum, ms per Newton iteration with the
-    // coarse inverse rebuilt every 5th: 30^3 cube 1,404 unknowns 3.95 against
-    // 2,790 4.47; 40^3 1,380 7.25 against 2,778 7.41; 60^3 1,404 20.7,
-    // 2,526 19.4, 2,808 19.0, 3,186 21.0), at least 32 handles per aggregate
-    const double nc_auto = std::min(2.0 * kAutoCoarse,
-                                    kAutoCoarse * std::cbrt(std::max(1.0, (double)nh / kAutoHandles)));
     const int64_t agg = o.coarse_aggregate > 0
                             ? o.coarse_aggregate
-                            : std::max<int64_t>(kAutoMinAggregate, (int64_t)std::ceil((double)(nh * kc) / nc_auto));
+                            : std::max<int64_t>(lagged || d == 3 ? kAutoMinAggregate : kAutoMinAggregate2,
+                                                (int64_t)std::ceil((double)(nh * kc) /
+                                                                   auto_coarse_unknowns(d, nh, lagged)));
     // keep the dense coarse matrix bounded: larger aggregates for large meshes
     // (grown further while breadth-first aggregates come out too small)
     const int want = (int)std::max<int64_t>(agg, (nh * kc + kMaxCoarse - 1) / kMaxCoarse);
@@ -1402,12 +1423,29 @@ std::vector<uint64_t> pcg_graph_key(int d, const PcgSystem& a, hipStream_t s)
     return { (uint64_t)d, (uint64_t)a.nh, u(a.perm), u(a.brow_ptr), u(a.bcol), u(a.sym_ptr), u(a.usrc), u(a.diag), u(a.Hs),
              u(a.part_ptr), (uint64_t)a.Gs, (uint64_t)a.Gv, wbits, tbits, (uint64_t)a.max_iters, u(a.b), u(a.sol),
              u(a.Dinv), u(a.x), u(a.r), u(a.z), u(a.p), u(a.q), u(a.s), u(a.parts), u(a.sc), u(a.free_h), u(a.free_s),
-             (uint64_t)a.kc, (uint64_t)a.ppa, (uint64_t)a.n_agg, (uint64_t)a.nc, u(a.agg_ptr), u(a.dvec), u(a.Ainv),
+             (uint64_t)a.kc, (uint64_t)a.dense, (uint64_t)a.ppa, (uint64_t)a.n_agg, (uint64_t)a.nc, u(a.agg_ptr), u(a.dvec), u(a.Ainv),
              u(a.Ainv32), u(a.rpart), u(a.cparts), u(s) };
 }
 
-tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev,
-                      const tad_solve_opts& o, tad_solve_stats* st, const unsigned char* free_dev = nullptr)
+// Systems of at most this many variables are solved with the dense inverse of
+// w I + H as the preconditioner (automatic coarse size only): one or two CG
+// iterations on an FP64 inverse instead of 35 .. 100 of three launches each;
+// the inverse costs about 28 us per 64 variables.  Newton step, dense against
+// two-level: pinned grids 128 variables 0.28 / 1.08 ms, 512 0.44 / 1.50,
+// 1,152 0.72 / 1.68, 2,048 1.33 / 1.74, 2,592 1.70 / 1.72; twisted cubes 192
+// 0.36 / 0.91 ms, 1,029 0.76 / 1.12, 1,536 1.08 / 1.16, 2,187 1.54 / 1.26
+// (fewer iterations in 3D).
+constexpr int64_t kDenseVars2 = 2400, kDenseVars3 = 1536;
+// Iterations the dense preconditioner gets before the solve starts over with
+// the two-level one (a matrix so close to singular that its inverse is
+// useless), with a rebuilt and with a reused inverse.
+constexpr int kDenseIters = 32, kDenseReuseIters = 200;
+
+// One solve.  lagged: the coarse space serves several solves.  dense: with the dense preconditioner; *again = true when that
+// one is not usable or did not converge within its iterations (nothing is
+// returned then).
+tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev, const tad_solve_opts& o,
+                      tad_solve_stats* st, const unsigned char* free_dev, bool lagged, bool dense, bool* again)
 {
     const int d = fn->d;
     const int64_t nh = fn->n_handles, n = fn->n_vars;
@@ -1420,11 +1458,10 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     TAD_HIP(fn->p.ensure(2 * n));
     TAD_HIP(fn->q.ensure(n));
     TAD_HIP(fn->scal.ensure(1));
-    if (o.max_iters <= 0) return fail(TAD_ERR_INVALID, "max_iters must be positive");
     PcgSystem sys;
     const SolverOrder* od = &fn->natural;
     bool use_coarse = false, coarse_reused = false;
-    TAD_TRY(setup_coarse(fn, H_dev, o, free_dev, &sys, &od, &use_coarse, &coarse_reused));
+    if (!dense) TAD_TRY(setup_coarse(fn, H_dev, o, free_dev, &sys, &od, &use_coarse, &coarse_reused, lagged));
     if (od == &fn->natural && !od->ready)
     {
         std::vector<int32_t> id(nh);
@@ -1434,7 +1471,11 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     if (free_dev) TAD_HIP(fn->free_s.ensure(n));
     TAD_HIP(fn->pcg_parts.ensure((size_t)pcg_parts_size(od->Gs, od->Gv)));
     TAD_HIP(fn->sym_H.ensure((size_t)od->n_sym * d * d));
-    if (!use_coarse) sys.kc = 0;
+    if (!use_coarse)
+    {
+        sys.kc = 0;
+        sys.n_agg = 0;
+    }
     sys.nh = nh;
     sys.perm = od->perm.p;
     sys.brow_ptr = od->brow_ptr.p;
@@ -1466,6 +1507,32 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     tm.begin("sym_pack", s);
     TAD_HIP(launch_sym_pack(d, od->n_sym, od->place.p, H_dev, fn->sym_H.p, s));
     tm.end("sym_pack", s);
+    if (dense)
+    {
+        auto& c = fn->co;
+        use_coarse = true;
+        coarse_reused = o.coarse_reuse && c.dense_valid && !free_dev && c.dense_w == o.w_identity;
+        sys.max_iters = std::min(o.max_iters, coarse_reused ? kDenseReuseIters : kDenseIters);
+        sys.dense = 1;
+        sys.nc = n;
+        sys.n_agg = dense_apply_groups(n);
+        TAD_HIP(c.dense_inv.ensure((size_t)(n * n)));
+        TAD_HIP(c.dense_parts.ensure((size_t)2 * sys.n_agg));
+        sys.Ainv = c.dense_inv.p;
+        sys.cparts = c.dense_parts.p;
+        if (!coarse_reused)
+        {
+            c.dense_valid = false;
+            tm.begin("coarse_setup", s);
+            TAD_HIP(c.info.ensure(2));
+            TAD_HIP(c.inv_work.ensure((size_t)spd_inverse_work(n)));
+            TAD_HIP(launch_dense_fill(d, sys, c.dense_inv.p, s));
+            tm.begin("coarse_inverse", s);
+            TAD_HIP(launch_spd_inverse(n, c.dense_inv.p, c.inv_work.p, c.info.p, s));
+            tm.end("coarse_inverse", s);
+            tm.end("coarse_setup", s);
+        }
+    }
     tm.begin("pcg_init", s);
     TAD_HIP(launch_pcg_init(d, sys, s));
     tm.end("pcg_init", s);
@@ -1481,7 +1548,7 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     // (Newton steps need similar counts), later ones come every `every`:
     // each poll stalls the device for a host round trip.
     int k = 0;
-    int chunk = std::max(every, fn->last_solve_iters * 3 / 4);
+    int chunk = dense ? fn->last_dense_iters + 1 : std::max(every, fn->last_solve_iters * 3 / 4);
     // recorded launches: kGraphIters iterations, each followed by the
     // device-side iteration counter's advance, replayed until termination
     // (every kernel returns at once after it, and iteration max_iters stops
@@ -1531,26 +1598,46 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
             }
         }
     }
-    while (k <= o.max_iters)
+    while (k <= sys.max_iters)
     {
         if (gexec)
         {
-            for (int c = 0; c < chunk && k <= o.max_iters; c += kGraphIters, k += kGraphIters)
+            for (int c = 0; c < chunk && k <= sys.max_iters; c += kGraphIters, k += kGraphIters)
                 TAD_HIP(hipGraphLaunch(gexec, s));
         }
         else
         {
-            for (int c = 0; c < chunk && k <= o.max_iters; ++c, ++k)
-                TAD_HIP(launch_pcg_iteration(d, sys, k, k < o.max_iters, s, timer));
+            for (int c = 0; c < chunk && k <= sys.max_iters; ++c, ++k)
+                TAD_HIP(launch_pcg_iteration(d, sys, k, k < sys.max_iters, s, timer));
         }
+        int* info = reinterpret_cast<int*>(fn->ctx->pinned + 96);
+        info[0] = 0;
+        if (dense && !coarse_reused) TAD_HIP(hipMemcpyAsync(info, fn->co.info.p, sizeof(int), hipMemcpyDeviceToHost, s));
         TAD_HIP(hipMemcpyAsync(pin, fn->scal.p, sizeof(hs), hipMemcpyDeviceToHost, s));
         TAD_HIP(hipStreamSynchronize(s));
+        if (info[0] != 0)  // a pivot was not positive: not the preconditioner for this matrix
+        {
+            *again = true;
+            return TAD_OK;
+        }
         if (pin->done) break;
-        chunk = every;
+        chunk = dense ? 2 : every;
     }
     if (!pin->done) return fail(TAD_ERR_SOLVE, "PCG did not report termination");
     std::memcpy(&hs, pin, sizeof(hs));
-    fn->last_solve_iters = hs.iters;
+    if (dense && sys.max_iters < o.max_iters && !(hs.rr <= sys.tol2 * hs.bb))
+    {
+        *again = true;
+        return TAD_OK;
+    }
+    if (dense)
+    {
+        fn->co.dense_valid = !free_dev && !hs.breakdown;
+        fn->co.dense_w = o.w_identity;
+        fn->last_dense_iters = hs.iters;
+    }
+    else
+        fn->last_solve_iters = hs.iters;
     fn->solves_since_rebuild = coarse_reused ? fn->solves_since_rebuild + 1 : 0;
     const double rel = hs.bb > 0 ? std::sqrt(hs.rr / hs.bb) : 0.0;
     if (hs.breakdown)  // no product wrote the solution: the last iterate
@@ -1569,6 +1656,21 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     if (hs.breakdown) return fail(TAD_ERR_SOLVE, "Linear solve failed: matrix not positive definite");
     if (!std::isfinite(rel)) return fail(TAD_ERR_SOLVE, "Linear solve failed: non-finite residual");
     return TAD_OK;
+}
+
+tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev,
+                      const tad_solve_opts& o, tad_solve_stats* st, const unsigned char* free_dev = nullptr,
+                      bool lagged = false)
+{
+    if (o.max_iters <= 0) return fail(TAD_ERR_INVALID, "max_iters must be positive");
+    if (o.coarse_aggregate < 0 && fn->n_blocks > 0 && fn->n_vars <= (fn->d == 3 ? kDenseVars3 : kDenseVars2))
+    {
+        bool again = false;
+        const tad_status r = solve_once(fn, H_dev, rhs_dev, sol_dev, o, st, free_dev, lagged, true, &again);
+        if (!again) return r;
+        fn->co.dense_valid = false;
+    }
+    return solve_once(fn, H_dev, rhs_dev, sol_dev, o, st, free_dev, lagged, false, nullptr);
 }
 
 // Armijo backtracking on device data (LineSearch.hh:26-65).  The direction is
@@ -2636,7 +2738,7 @@ tad_status tad_newton_step(tad_fn fn, double* x, tad_mem mem, const tad_newton_o
     std::memset(&ss, 0, sizeof(ss));
     tad_solve_opts sopt = o.solve;
     if (o.coarse_refresh > 1 && fn->solves_since_rebuild + 1 < o.coarse_refresh) sopt.coarse_reuse = 1;
-    TAD_TRY(solve_core(fn, fn->H_buf.p, fn->g_buf.p, fn->sol.p, sopt, &ss));
+    TAD_TRY(solve_core(fn, fn->H_buf.p, fn->g_buf.p, fn->sol.p, sopt, &ss, nullptr, o.coarse_refresh > 1));
     st.cg_iters = ss.iters;
     st.solve_converged = ss.converged;
     st.coarse_unknowns = ss.coarse_unknowns;

@@ -201,6 +201,9 @@ struct PcgSystem
     const float* Ainv32 = nullptr;      // [nc * nc] its FP32 copy for the CG iterations (launch_coarse_to32), or null
     double* rpart = nullptr;            // [ppa * nc] restricted residual, one row per part of an aggregate
     double* cparts = nullptr;           // [2 * n_agg] partials of r_c . A_c^-1 r_c, slot k & 1
+    // small systems: z = A^-1 r with A = w I + H inverted densely (Ainv, handle
+    // order, kc = 0, n_agg = dense_apply_groups(nh * d)), no block-Jacobi part
+    int dense = 0;
 };
 
 constexpr int kCoarseChunk = 256;  // fine blocks per Galerkin chunk
@@ -254,6 +257,12 @@ hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* place, const dou
 int pcg_spmv_groups(int64_t nh);
 // Size (doubles) of the partial-sum buffer of the CG kernels.
 int64_t pcg_parts_size(int64_t Gs, int64_t Gv);
+
+// The dense preconditioner's matrix w I + H (column-major, lower triangle)
+// from the solver's copy in handle order, and the workgroups (partials) of its
+// product.
+hipError_t launch_dense_fill(int d, const PcgSystem& a, double* A, hipStream_t s);
+int64_t dense_apply_groups(int64_t n);
 
 // Before iteration 0: the block-Jacobi inverse (per entry the upper triangle
 // of its symmetric d x d block, d (d + 1) / 2 doubles, row by row), x = 0,

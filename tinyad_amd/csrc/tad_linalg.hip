@@ -820,15 +820,15 @@ __global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(PcgSystem a, int G
         // partials t, t + NT, ... in order
         const double* __restrict__ pd = a.parts;
         const double* __restrict__ pr = a.parts + Gs + ((k + 1) & 1) * Gv;
-        const double* __restrict__ pk = KC > 0 ? a.cparts + ((k + 1) & 1) * a.n_agg : nullptr;
+        const double* __restrict__ pk = a.cparts + ((k + 1) & 1) * a.n_agg;  // n_agg: 0 without a correction
         double vd[6], vr[6], vk[3];
         strided_fetch<NT, 6>(pd, Gs, vd);
         strided_fetch<NT, 6>(pr, Gv, vr);
-        if constexpr (KC > 0) strided_fetch<NT, 3>(pk, a.n_agg, vk);
+        strided_fetch<NT, 3>(pk, a.n_agg, vk);
         if (lo < hi) load(lo);  // in flight during the sums
         if (t == 0) flag = done_v;
-        double tot[3] = { strided_rest<NT, 6>(pd, Gs, vd), strided_rest<NT, 6>(pr, Gv, vr), 0.0 };
-        if constexpr (KC > 0) tot[2] = strided_rest<NT, 3>(pk, a.n_agg, vk);
+        double tot[3] = { strided_rest<NT, 6>(pd, Gs, vd), strided_rest<NT, 6>(pr, Gv, vr),
+                          strided_rest<NT, 3>(pk, a.n_agg, vk) };
         if constexpr (NT == 64) __syncthreads();
         block_totals<NT, 3>(tot, sh);
         if (flag) return;
@@ -919,7 +919,7 @@ __global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(PcgSystem a, int G
 #pragma unroll
                     for (int j = i; j < D; ++j)
                     {
-                        const double e = (fr[i] && fr[j]) ? o[i * D + j] : 0.0;
+                        const double e = (fr[i] && fr[j] && !a.dense) ? o[i * D + j] : 0.0;
                         sD[t * PB + PackedBlock<D>::at(i, j)] = e;
                         if (v < hi) a.Dinv[v * PB + PackedBlock<D>::at(i, j)] = e;
                     }
@@ -1411,6 +1411,100 @@ static hipError_t update_any(int d, const PcgSystem& a, int k, const int* kdev, 
     return hipGetLastError();
 }
 
+// A small system's dense preconditioner: A = w I + H in FP64 (column-major
+// n x n, lower triangle, zeroed by the caller) from the solver's copy in
+// handle order, one thread per row of A; rows and columns of fixed variables
+// (and rows no element has, for w = 0) are the identity's.
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_dense_fill(PcgSystem a, double* __restrict__ A)
+{
+    const int64_t n = a.nh * D;
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n) return;
+    const int64_t u = r / D;
+    const int i = (int)(r - u * D);
+    const bool fr = a.free_h ? a.free_h[r] != 0 : true;
+    const int32_t s0 = a.sym_ptr[u], s1 = a.sym_ptr[u + 1], b0 = a.brow_ptr[u];
+    for (int32_t l = s0; l < s1; ++l)
+    {
+        const int64_t v = a.bcol[b0 + (l - s0)];
+#pragma unroll
+        for (int j = 0; j < D; ++j)
+        {
+            const int64_t c = v * D + j;
+            if (c >= r || !fr || (a.free_h && !a.free_h[c])) continue;
+            A[r + c * n] = a.Hs[(int64_t)l * (D * D) + i * D + j];
+        }
+    }
+    const int32_t dg = a.diag[u];
+    const double h = dg < 0 ? 0.0 : a.Hs[(int64_t)dg * (D * D) + i * D + i];
+    A[r + r * n] = !fr ? 1.0 : h + (dg < 0 && !(a.w > 0.0) ? 1.0 : a.w);
+}
+
+// z = A^-1 r for the dense preconditioner, one wave per row (four per
+// workgroup), with the workgroup's partial of r.z.
+__global__ __launch_bounds__(kBlock) void k_dense_apply(PcgSystem a, int64_t n, int k, const int* __restrict__ kdev)
+{
+    constexpr int NW = kBlock / 64;
+    __shared__ double sh[NW];
+    __shared__ int flag;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int done_v = t == 0 ? a.sc->done : 0;
+    const int slot = (kdev ? *kdev : k) & 1;
+    const int64_t row = (int64_t)blockIdx.x * NW + wv;
+    double acc = 0.0;
+    if (row < n)
+    {
+        const double* __restrict__ m = a.Ainv + row * n;
+        const double* __restrict__ r = a.r;
+        int64_t j = lane;
+        for (; j + 7 * 64 < n; j += 8 * 64)
+        {
+            double mv[8], rv[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+            {
+                mv[q] = m[j + 64 * q];
+                rv[q] = r[j + 64 * q];
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc = fma(mv[q], rv[q], acc);
+        }
+        for (; j < n; j += 64) acc = fma(m[j], r[j], acc);
+    }
+    if (t == 0) flag = done_v;
+    acc = wave_total(acc);
+    __syncthreads();
+    if (flag) return;
+    if (lane == 0)
+    {
+        if (row < n) a.z[row] = acc;
+        sh[wv] = row < n ? acc * a.r[row] : 0.0;
+    }
+    __syncthreads();
+    if (t == 0)
+    {
+        double v = sh[0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += sh[w];
+        a.cparts[slot * a.n_agg + blockIdx.x] = v;
+    }
+}
+
+hipError_t launch_dense_fill(int d, const PcgSystem& a, double* A, hipStream_t s)
+{
+    const int64_t n = a.nh * d;
+    hipError_t e = launch_fill(A, n * n, 0.0, s);
+    if (e != hipSuccess) return e;
+    const unsigned grid = (unsigned)((n + kBlock - 1) / kBlock);
+    if (d == 1) k_dense_fill<1><<<grid, kBlock, 0, s>>>(a, A);
+    else if (d == 2) k_dense_fill<2><<<grid, kBlock, 0, s>>>(a, A);
+    else k_dense_fill<3><<<grid, kBlock, 0, s>>>(a, A);
+    return hipGetLastError();
+}
+
+int64_t dense_apply_groups(int64_t n) { return (n + kBlock / 64 - 1) / (kBlock / 64); }
+
 template <int D, int KC>
 static void coarse_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
 {
@@ -1420,12 +1514,14 @@ static void coarse_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
         k_coarse_apply_prolong<D, KC, double><<<(unsigned)a.n_agg, kCoarseBlock, 0, s>>>(a, a.Ainv, k, kdev);
 }
 
-// z += P A_c^-1 P^T r with the restricted residual's parts of the last update
+// z += P A_c^-1 P^T r with the restricted residual's parts of the last update,
+// or z = A^-1 r (dense)
 static hipError_t coarse_any(int d, const PcgSystem& a, int k, const int* kdev, hipStream_t s, Timer* timer)
 {
-    if (a.kc == 0) return hipSuccess;
+    if (a.kc == 0 && !a.dense) return hipSuccess;
     if (timer) timer->begin("pcg_coarse", s);
-    if (d == 3 && a.kc == 6) coarse_t<3, 6>(a, k, kdev, s);
+    if (a.dense) k_dense_apply<<<(unsigned)a.n_agg, kBlock, 0, s>>>(a, a.nh * d, k, kdev);
+    else if (d == 3 && a.kc == 6) coarse_t<3, 6>(a, k, kdev, s);
     else if (d == 3 && a.kc == 3) coarse_t<3, 3>(a, k, kdev, s);
     else if (d == 2 && a.kc == 3) coarse_t<2, 3>(a, k, kdev, s);
     else if (d == 2 && a.kc == 2) coarse_t<2, 2>(a, k, kdev, s);
