@@ -115,8 +115,8 @@ def kernel_table(ctx, names):
     return {k: ctx.kernel_stats(k) for k in names}
 
 
-EVAL_KERNELS = ["element", "assemble_gradient", "assemble_hessian", "energy_sum"]
-NEWTON_KERNELS = EVAL_KERNELS + ["spmv", "pcg_update", "pcg_coarse", "pcg_setup", "coarse_setup", "coarse_galerkin",
+EVAL_KERNELS = ["element", "assemble_hessian", "assemble"]  # "assemble": gradient, sums, H for shape 0
+NEWTON_KERNELS = EVAL_KERNELS + ["spmv", "pcg_update", "pcg_coarse", "sym_pack", "coarse_setup", "coarse_galerkin",
                                  "coarse_inverse", "pcg_init", "energy"]
 
 

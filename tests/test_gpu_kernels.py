@@ -126,3 +126,44 @@ def test_small_systems_dense_preconditioner(ctx, kind, n):
     d, st = fn.solve(g, H=H2.data, tol=1e-12, coarse_reuse=1)
     assert st.converged and st.coarse_reused == 1
     assert nrel(d, spla.spsolve(H2.tocsc(), g)) <= 1e-9
+
+
+def star_quadratic(d, n, seed=0):
+    """Quadratic pairs (0, i): handle 0's block row holds n blocks."""
+    rng = np.random.default_rng(seed)
+    conn = np.stack([np.zeros(n - 1, dtype=np.int32), np.arange(1, n, dtype=np.int32)], axis=1)
+    K = 2 * d
+    A = rng.normal(size=(n - 1, K, K))
+    A = A + A.transpose(0, 2, 1)
+    params = np.concatenate([A.reshape(-1, K * K), rng.normal(size=(n - 1, K + 1))], axis=1)
+    return configs.Problem("star", d, n, [configs.Term(configs.E_QUADRATIC, conn, params)], rng.normal(size=d * n))
+
+
+# block rows below, at and above a tile of 256 blocks, and tiles that end in
+# the middle of the chip's eight-fold split
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("d", [1, 2, 3])
+@pytest.mark.parametrize("n", [2, 255, 256, 257, 300, 2000])
+def test_assembly_tiles(ctx, d, n, precision):
+    """Assembly by tiles of rows against one thread per block (the same sums in
+    the same order: identical bits) and against the sum of the element
+    matrices; the second term interleaves short rows."""
+    P = star_quadratic(d, n)
+    Q = quadratic_chain(d, max(n, 8), seed=1)
+    P = configs.Problem("both", d, max(n, 8), P.terms + Q.terms, Q.x0)
+    fn = tad.ScalarFunction.from_problem(P, ctx, precision)
+    x = P.x0
+    out = []
+    for shape in (0, 1):
+        fn.assembly_shape = shape
+        f, g, H = fn.eval_with_derivatives(x)
+        out.append((f, g, H.toarray()))
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
+    ref = np.zeros((x.size, x.size))
+    for t in P.terms:
+        K = t.valence * d
+        A = t.params[:, : K * K].reshape(-1, K, K)
+        idx = (t.conn[:, :, None] * d + np.arange(d)).reshape(-1, K)
+        np.add.at(ref, (idx[:, :, None], idx[:, None, :]), A)
+    # FP64: sums of at most 2,000 terms; mixed: FP32 contributions, FP64 sums
+    assert np.abs(out[0][2] - ref).max() <= (1e-12 if precision == "fp64" else 1e-6) * np.abs(ref).max()

@@ -264,6 +264,10 @@ struct tad_fn_s
     int64_t n_upper = 0;
     DevBuf<int64_t> uslot_ptr;
     DevBuf<int32_t> uplace;        // 4 per upper block
+    // tiles of whole block rows for the assembly (EvalTail)
+    int64_t n_tiles = 0;
+    DevBuf<int32_t> tile_ptr;
+    DevBuf<uint32_t> arun, alen, apos;
     // the solver's copy of H (its lower triangle's blocks in solver order, the
     // triangle the reference's SimplicialLDLT reads, LinearSolver.hh:14) for
     // solves without a coarse space: handle order
@@ -284,8 +288,9 @@ struct tad_fn_s
 
     // evaluation buffers
     DevBuf<unsigned char> gc_buf, hc_buf;  // contributions (FP64 or FP32 by precision)
-    DevBuf<double> elem_f, x_buf, g_buf, H_buf, partials, results, steps;
+    DevBuf<double> elem_f, x_buf, g_buf, H_buf, partials, steps;
     DevBuf<int> err;
+    bool err_clear = false;  // the flag in err is 0 (the last kernel of an evaluation clears it)
     // line search
     DevBuf<double> ls_f, x_tmp;
     // solver
@@ -390,6 +395,7 @@ void free_pattern(tad_fn fn)
     fn->brow_ptr.release(); fn->bcol.release(); fn->block_row.release(); fn->diag_block.release();
     fn->row_ptr.release(); fn->col_idx.release(); fn->hslot_ptr.release(); fn->gslot_ptr.release();
     fn->block_mirror.release(); fn->uslot_ptr.release(); fn->uplace.release();
+    fn->tile_ptr.release(); fn->arun.release(); fn->alen.release(); fn->apos.release();
     fn->natural.release(); fn->sym_H.release();
     fn->co.release();
     fn->h_brow_ptr.clear(); fn->h_bcol.clear(); fn->h_urow_ptr.clear();
@@ -689,6 +695,27 @@ tad_status build_pattern(tad_fn fn)
         for (size_t i = 0; i + 1 < uptr.size(); ++i)
             if (uptr[i] > uptr[i + 1]) return fail(TAD_ERR_UNSUPPORTED, "upper runs out of order");
     }
+    // 5. assembly tiles: whole block rows, at most kAsmTileBlocks blocks unless
+    //    one row alone has more
+    std::vector<int32_t> tile_ptr(1, 0);
+    std::vector<uint32_t> arun(nb), alen(nb), apos(nb, 0);
+    for (int64_t u = 0; u < nh; ++u)
+    {
+        const int32_t nbu = brow_ptr[u + 1] - brow_ptr[u];
+        if (nbu == 0) continue;
+        if (brow_ptr[u] > tile_ptr.back() && brow_ptr[u + 1] - tile_ptr.back() > kAsmTileBlocks)
+            tile_ptr.push_back(brow_ptr[u]);
+        for (int32_t k = brow_ptr[u]; k < brow_ptr[u + 1]; ++k)
+        {
+            const int32_t m = mirror[k];
+            arun[k] = (uint32_t)hptr[m] | (m != k ? 0x80000000u : 0u);
+            alen[k] = (uint32_t)(hptr[m + 1] - hptr[m]);
+            if (nbu <= kAsmTileBlocks)
+                apos[k] = (uint32_t)(d * d * (brow_ptr[u] - tile_ptr.back()) + d * (k - brow_ptr[u])) |
+                          (uint32_t)(d * nbu) << 16;
+        }
+    }
+    if (nb > 0) tile_ptr.push_back((int32_t)nb);
     hipStream_t s = fn->s();
     auto up = [&](auto& buf, const auto& vec) -> hipError_t {
         hipError_t e = buf.ensure(vec.size());
@@ -707,6 +734,10 @@ tad_status build_pattern(tad_fn fn)
     TAD_HIP(up(fn->block_mirror, mirror));
     TAD_HIP(up(fn->uslot_ptr, uptr));
     TAD_HIP(up(fn->uplace, uplace));
+    TAD_HIP(up(fn->tile_ptr, tile_ptr));
+    TAD_HIP(up(fn->arun, arun));
+    TAD_HIP(up(fn->alen, alen));
+    TAD_HIP(up(fn->apos, apos));
     for (size_t ti = 0; ti < fn->terms.size(); ++ti)
     {
         TermDev& td = fn->terms[ti];
@@ -742,6 +773,7 @@ tad_status build_pattern(tad_fn fn)
     fn->n_hslots = hptr[nb];
     fn->n_gslots = gptr[nh];
     fn->n_blocks = nb;
+    fn->n_tiles = (int64_t)tile_ptr.size() - 1;
     fn->n_upper = (int64_t)uptr.size() - 1;
     fn->nnz = nnz;
     fn->pattern_ready = true;
@@ -1176,7 +1208,6 @@ tad_status ensure_ready(tad_fn fn)
     TAD_HIP(fn->g_buf.ensure((size_t)fn->n_vars));
     TAD_HIP(fn->H_buf.ensure((size_t)fn->nnz));
     TAD_HIP(fn->partials.ensure(8 * kReduceBlocks + 4096));
-    TAD_HIP(fn->results.ensure(16));
     TAD_HIP(fn->steps.ensure(16));
     TAD_HIP(fn->err.ensure(1));
     return TAD_OK;
@@ -1259,11 +1290,39 @@ tad_status ensure_aux(tad_ctx ctx, int n_events)
     return TAD_OK;
 }
 
+// The assembly shape in use: as set or tuned; for 0 (the default) the tiles of
+// launch_eval_tail, except for large 3D patterns, where one launch of its own
+// is faster: whole evaluations in us by shape 0 tiles / 1 / 2 / 3, 60^3 cube
+// (3.3 M blocks) FP64 1,251 / 1,226 / 1,219 / 1,229, mixed 751 / 716 / 753 /
+// 733; 30^3 (424K) 226 / 224 / 217 / 217, 140 / 141 / 138 / 138; 10^3 107 / 110
+// / 109 / 111; triangles: 700 x 700 grid FP64 254 / 257 / 264 / 265, mixed 177
+// / 188 / 202 / 197, 256 disks mixed 562 / 572 / 648 / 665.
+constexpr int64_t kTileBlocks3 = 200000;
+int assembly_shape(tad_fn fn)
+{
+    if (fn->asm_shape != 0 || fn->d < 3 || fn->n_blocks < kTileBlocks3) return fn->asm_shape;
+    return fn->precision == TAD_PREC_FP64 ? 2 : 1;
+}
+
+// H's assembly by tiles in `tail`
+void set_tiles(tad_fn fn, EvalTail& tail, double* H_dev)
+{
+    tail.n_tiles = fn->n_tiles;
+    tail.tile_ptr = fn->tile_ptr.p;
+    tail.arun = fn->arun.p;
+    tail.alen = fn->alen.p;
+    tail.apos = fn->apos.p;
+    tail.Hc = fn->hc_buf.p;
+    tail.H = H_dev;
+}
+
 tad_status eval_core(tad_fn fn, const double* x_dev, int mode, double eps, double* g_dev, double* H_dev, double* f)
 {
     hipStream_t s = fn->s();
     KernelTimer& tm = fn->ctx->timer;
-    TAD_HIP(hipMemsetAsync(fn->err.p, 0, sizeof(int), s));
+    // the flag is cleared by the previous evaluation's last kernel
+    if (!fn->err_clear) TAD_HIP(hipMemsetAsync(fn->err.p, 0, sizeof(int), s));
+    fn->err_clear = false;
     if (!fn->pipe_ready) plan_pipeline(fn);
     const bool pipe = fn->pipe_used > 1 && H_dev && mode >= MODE_HESS && fn->n_blocks > 0;
     if (pipe)
@@ -1314,37 +1373,45 @@ tad_status eval_core(tad_fn fn, const double* x_dev, int mode, double eps, doubl
             TAD_HIP(launch_element(t, fn->d, fn->precision, mode, x_dev, eps, fn->elem_f.p, fn->gc_buf.p, fn->hc_buf.p,
                                    fn->err.p, s));
         tm.end("element", s);
-        if (g_dev)
-        {
-            tm.begin("assemble_gradient", s);
-            TAD_HIP(launch_assemble_gradient(fn->d, fn->precision, fn->n_handles, fn->gslot_ptr.p, fn->gc_buf.p, g_dev,
-                                             s));
-            tm.end("assemble_gradient", s);
-        }
     }
-    if (H_dev && mode >= MODE_HESS)
+    EvalTail tail;
+    tail.n_handles = fn->n_handles;
+    const bool hess = H_dev && mode >= MODE_HESS;
+    const int shape = assembly_shape(fn);
+    if (hess && !pipe && shape != 0)
     {
-        if (!pipe)
-        {
-            tm.begin("assemble_hessian", s);
-            TAD_HIP(launch_assemble_hessian(fn->d, fn->precision, fn->asm_shape, fn->hess_asm(), fn->hc_buf.p, H_dev,
-                                            s));
-            tm.end("assemble_hessian", s);
-        }
+        tm.begin("assemble_hessian", s);
+        TAD_HIP(launch_assemble_hessian(fn->d, fn->precision, shape, fn->hess_asm(), fn->hc_buf.p, H_dev, s));
+        tm.end("assemble_hessian", s);
+    }
+    if (hess)
+    {
+        if (!pipe && shape == 0 && fn->n_blocks > 0) set_tiles(fn, tail, H_dev);
         // positions of this Hessian: lever arms of the coarse space's rotations
         TAD_HIP(fn->x_hess.ensure((size_t)fn->n_vars));
-        TAD_HIP(hipMemcpyAsync(fn->x_hess.p, x_dev, fn->n_vars * sizeof(double), hipMemcpyDeviceToDevice, s));
+        tail.x = x_dev;
+        tail.x_copy = fn->x_hess.p;
         fn->x_hess_valid = true;
     }
-    tm.begin("energy_sum", s);
-    TAD_HIP(launch_sum(fn->elem_f.p, fn->n_elem_total, 1, fn->n_elem_total, fn->partials.p, fn->results.p, s));
-    if (fn->n_seg > 0)
-        TAD_HIP(launch_segment_sum(fn->elem_f.p, fn->seg_ranges.p, (int)fn->terms.size(), fn->n_seg, fn->seg_f.p, s));
-    tm.end("energy_sum", s);
+    if (!pipe)
+    {
+        tail.gslot_ptr = fn->gslot_ptr.p;
+        tail.G = fn->gc_buf.p;
+        tail.g = g_dev;
+    }
+    tail.elem_f = fn->elem_f.p;
+    tail.n_elem = fn->n_elem_total;
+    tail.partials = fn->partials.p;
+    tail.seg_ranges = fn->seg_ranges.p;
+    tail.n_terms = (int)fn->terms.size();
+    tail.n_seg = fn->n_seg;
+    tail.seg_f = fn->seg_f.p;
     double* pin = fn->ctx->pinned;
-    TAD_HIP(hipMemcpyAsync(pin, fn->results.p, sizeof(double), hipMemcpyDeviceToHost, s));
-    TAD_HIP(hipMemcpyAsync(pin + 1, fn->err.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    tm.begin("assemble", s);
+    TAD_HIP(launch_eval_tail(fn->d, fn->precision, tail, fn->err.p, pin, reinterpret_cast<int*>(pin + 1), s));
+    tm.end("assemble", s);
     TAD_HIP(hipStreamSynchronize(s));
+    fn->err_clear = true;
     int errv = 0;
     std::memcpy(&errv, pin + 1, sizeof(int));
     *f = pin[0];
@@ -1372,12 +1439,11 @@ tad_status eval_energy_batch(tad_fn fn, const double* x_dev, const double* dir_d
         TAD_HIP(launch_energy(t, fn->d, x_dev, dir_dev, fn->steps.p, nc, dst, ne, s));
     tm.end("energy", s);
     tm.begin("energy_sum", s);
-    TAD_HIP(launch_sum(dst, ne, nc, ne, fn->partials.p, fn->results.p, s));
+    double* pin = fn->ctx->pinned;
+    TAD_HIP(launch_sum(dst, ne, nc, ne, fn->partials.p, pin + 32, s));
     if (!dir_dev && fn->n_seg > 0)
         TAD_HIP(launch_segment_sum(fn->elem_f.p, fn->seg_ranges.p, (int)fn->terms.size(), fn->n_seg, fn->seg_f.p, s));
     tm.end("energy_sum", s);
-    double* pin = fn->ctx->pinned;
-    TAD_HIP(hipMemcpyAsync(pin + 32, fn->results.p, nc * sizeof(double), hipMemcpyDeviceToHost, s));
     TAD_HIP(hipStreamSynchronize(s));
     for (int c = 0; c < nc; ++c) f_out[c] = pin[32 + c];
     return TAD_OK;
@@ -1386,9 +1452,8 @@ tad_status eval_energy_batch(tad_fn fn, const double* x_dev, const double* dir_d
 tad_status dot_dev(tad_fn fn, const double* a, const double* b, double* out)
 {
     hipStream_t s = fn->s();
-    TAD_HIP(launch_dot(a, b, fn->n_vars, fn->partials.p, fn->results.p + 8, s));
     double* pin = fn->ctx->pinned;
-    TAD_HIP(hipMemcpyAsync(pin + 48, fn->results.p + 8, sizeof(double), hipMemcpyDeviceToHost, s));
+    TAD_HIP(launch_dot(a, b, fn->n_vars, fn->partials.p, pin + 48, s));
     TAD_HIP(hipStreamSynchronize(s));
     *out = pin[48];
     return TAD_OK;
@@ -1399,10 +1464,9 @@ tad_status dot2_dev(tad_fn fn, const double* a1, const double* b1, const double*
                     double* out2)
 {
     hipStream_t s = fn->s();
-    TAD_HIP(launch_dot(a1, b1, fn->n_vars, fn->partials.p, fn->results.p + 8, s));
-    TAD_HIP(launch_dot(a2, b2, fn->n_vars, fn->partials.p, fn->results.p + 9, s));
     double* pin = fn->ctx->pinned;
-    TAD_HIP(hipMemcpyAsync(pin + 48, fn->results.p + 8, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+    TAD_HIP(launch_dot(a1, b1, fn->n_vars, fn->partials.p, pin + 48, s));
+    TAD_HIP(launch_dot(a2, b2, fn->n_vars, fn->partials.p, pin + 49, s));
     TAD_HIP(hipStreamSynchronize(s));
     *out1 = pin[48];
     *out2 = pin[49];
@@ -1840,7 +1904,7 @@ tad_status tad_fn_destroy(tad_fn fn)
     }
     free_pattern(fn);
     fn->gc_buf.release(); fn->hc_buf.release(); fn->elem_f.release(); fn->x_buf.release(); fn->g_buf.release(); fn->H_buf.release();
-    fn->partials.release(); fn->results.release(); fn->steps.release(); fn->err.release();
+    fn->partials.release(); fn->steps.release(); fn->err.release();
     fn->ls_f.release(); fn->x_tmp.release();
     fn->Dinv.release(); fn->r.release(); fn->z.release(); fn->p.release(); fn->q.release(); fn->sol.release();
     fn->scal.release(); fn->pcg_parts.release(); fn->seg_ranges.release(); fn->seg_f.release();
@@ -2457,9 +2521,8 @@ static tad_status dots_n(tad_fn fn, int64_t n, int count, const double* const* a
 {
     hipStream_t s = fn->s();
     for (int i = 0; i < count; ++i)
-        TAD_HIP(launch_dot(a[i], b[i], n, fn->partials.p, fn->results.p + 10 + i, s));
+        TAD_HIP(launch_dot(a[i], b[i], n, fn->partials.p, fn->ctx->pinned + 50 + i, s));
     double* pin = fn->ctx->pinned;
-    TAD_HIP(hipMemcpyAsync(pin + 50, fn->results.p + 10, count * sizeof(double), hipMemcpyDeviceToHost, s));
     TAD_HIP(hipStreamSynchronize(s));
     for (int i = 0; i < count; ++i) out[i] = pin[50 + i];
     return TAD_OK;
@@ -2570,6 +2633,7 @@ tad_status tad_fn_solve_basis(tad_fn fn, const double* H_values, int64_t m, cons
     const double* btv = fn->bas_tv.p;
     // r = B^T rhs, the Jacobi preconditioner of B^T H B + w I, y = 0
     TAD_HIP(launch_csr_spmv(m, btp, btc, btv, bd, 0.0, nullptr, r, s));
+    fn->err_clear = false;
     TAD_HIP(hipMemsetAsync(fn->err.p, 0, sizeof(int), s));
     TAD_HIP(launch_basis_diag(m, btp, btc, btv, fn->row_ptr.p, fn->col_idx.p, Hd, o.w_identity, dinv, fn->err.p, s));
     TAD_HIP(launch_fill(y, m, 0.0, s));
@@ -2971,6 +3035,7 @@ tad_status tad_fn_autotune(tad_fn fn, const double* x, tad_mem mem, double eps, 
         *out = best;
         return TAD_OK;
     };
+    fn->err_clear = false;  // element launches below may raise the flag
     struct Cand { int block, grid, map; double ms; };
     std::vector<std::vector<Cand>> shortlist(fn->terms.size());
     for (size_t ti = 0; ti < fn->terms.size(); ++ti)
@@ -3043,7 +3108,16 @@ tad_status tad_fn_autotune(tad_fn fn, const double* x, tad_mem mem, double eps, 
             for (int rep_i = 0; rep_i < 4; ++rep_i)
             {
                 TAD_HIP(hipEventRecord(e0, s));
-                TAD_HIP(launch_assemble_hessian(fn->d, fn->precision, shape, pat, fn->hc_buf.p, fn->H_buf.p, s));
+                if (shape == 0)
+                {
+                    EvalTail tail;
+                    tail.n_handles = fn->n_handles;
+                    set_tiles(fn, tail, fn->H_buf.p);
+                    tail.partials = fn->partials.p;
+                    TAD_HIP(launch_eval_tail(fn->d, fn->precision, tail, nullptr, fn->ctx->pinned, nullptr, s));
+                }
+                else
+                    TAD_HIP(launch_assemble_hessian(fn->d, fn->precision, shape, pat, fn->hc_buf.p, fn->H_buf.p, s));
                 TAD_HIP(hipEventRecord(e1, s));
                 TAD_HIP(hipEventSynchronize(e1));
                 float ms = 0.f;
@@ -3058,9 +3132,9 @@ tad_status tad_fn_autotune(tad_fn fn, const double* x, tad_mem mem, double eps, 
         fn->asm_shape = bs;
         char line[256];
         std::snprintf(line, sizeof(line),
-                      "Hessian assembly: %d lanes per block %.4f ms, one thread per block %.4f ms, "
+                      "Hessian assembly: tiles of rows %.4f ms, one thread per block %.4f ms, "
                       "%d lanes per upper block %.4f ms, one thread per upper block %.4f ms\n",
-                      fn->d * fn->d, ms_shape[0], ms_shape[1], fn->d * fn->d, ms_shape[2], ms_shape[3]);
+                      ms_shape[0], ms_shape[1], fn->d * fn->d, ms_shape[2], ms_shape[3]);
         rep += line;
         // element launch shape by whole evaluations among the finalists
         fn->pipe_chunks = 1;

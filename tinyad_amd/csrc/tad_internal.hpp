@@ -110,7 +110,7 @@ hipError_t launch_sum(const double* in, int64_t n, int ncand, int64_t stride, do
                       hipStream_t s);
 
 // Device pattern of the Hessian assembly.
-//   Per CSR block b (shapes 0, 1): its row block_row[b], the run
+//   Per CSR block b (shape 1): its row block_row[b], the run
 //   [hslot_ptr[m], hslot_ptr[m+1]) of m = mirror[b] (b itself for column >=
 //   row, else the upper block (col, row), read transposed).
 //   Per upper block i (shapes 2, 3; upper blocks in CSR order): its run
@@ -137,16 +137,51 @@ struct HessAsm
 constexpr int kAsmShapes = 4;
 
 // CSR values of H from the Hessian contributions Hc; gradient of handle u =
-// sum of slots [gslot_ptr[u], ..) of G.  shape 0: d*d lanes per block, 1: one
-// thread per block, 2: d*d lanes per upper block writing it and its mirror,
-// 3: one thread per upper block writing both.  Every shape sums each run in
-// slot order (identical results).
+// sum of slots [gslot_ptr[u], ..) of G.  shape 0: tiles of whole rows through
+// LDS (launch_eval_tail; here, for rows [r0, r1), as shape 1), 1: one thread
+// per block, 2: d*d lanes per upper block writing it and its mirror, 3: one
+// thread per upper block writing both.  Every shape sums each run in slot
+// order (identical results).
 // r0 >= 0: only the block rows (handles) [r0, r1).
 hipError_t launch_assemble_hessian(int d, int precision, int shape, const HessAsm& a, const void* Hc, double* H,
                                    hipStream_t s, int64_t r0 = -1, int64_t r1 = -1);
 
 hipError_t launch_assemble_gradient(int d, int precision, int64_t n_handles, const int64_t* gslot_ptr,
                                     const void* G, double* g, hipStream_t s, int64_t v0 = -1, int64_t v1 = -1);
+
+// The part of an evaluation after its element kernels: H's CSR values (null:
+// none, or assembled by another shape), the gradient, the copy of x, energy
+// sums.  Tile i of the assembly is the CSR blocks [tile_ptr[i],
+// tile_ptr[i + 1]), whole block rows; per CSR block its run of contributions
+// (arun: first slot, top bit: read transposed; alen: contributions) and its
+// place among its tile's values (apos: offset of entry (0, 0), row stride
+// << 16; unused for a row of more than kAsmTileBlocks blocks).
+constexpr int kAsmTileBlocks = 256;
+struct EvalTail
+{
+    int64_t n_tiles = 0;
+    const int32_t* tile_ptr = nullptr;
+    const uint32_t *arun = nullptr, *alen = nullptr, *apos = nullptr;
+    const void* Hc = nullptr;
+    double* H = nullptr;
+    int64_t n_handles = 0;
+    const int64_t* gslot_ptr = nullptr;
+    const void* G = nullptr;
+    double* g = nullptr;
+    const double* x = nullptr;
+    double* x_copy = nullptr;
+    const double* elem_f = nullptr;
+    int64_t n_elem = 0;
+    double* partials = nullptr;  // kReduceBlocks
+    const int64_t* seg_ranges = nullptr;
+    int n_terms = 0;
+    int64_t n_seg = 0;
+    double* seg_f = nullptr;
+    int64_t tile_blocks = 0, grad_blocks = 0, copy_blocks = 0;  // set by the launcher
+};
+// ... then the energy sum into f_out and the element kernels' error flag into
+// err_out (both may be pinned host memory); the flag is cleared.
+hipError_t launch_eval_tail(int d, int precision, EvalTail a, int* err, double* f_out, int* err_out, hipStream_t s);
 
 hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s);
 

@@ -54,36 +54,52 @@ __device__ __forceinline__ double strided_sum(const double* __restrict__ v, int6
     return acc;
 }
 
+// the b-th of kReduceBlocks chunks of in[0 .. n), summed by one block
+__device__ __forceinline__ double sum_chunk(const double* __restrict__ in, int64_t n, int64_t b, double* sh)
+{
+    const int64_t chunk = (n + kReduceBlocks - 1) / kReduceBlocks;
+    const int64_t lo = b * chunk;
+    const int64_t hi = lo + chunk < n ? lo + chunk : n;
+    return block_sum(strided_sum<kBlock>(in, lo + threadIdx.x, hi), sh);
+}
+
 // block b of row c sums the contiguous chunk [b*chunk, (b+1)*chunk)
 __global__ __launch_bounds__(kBlock) void k_sum_stage1(const double* __restrict__ in, int64_t n, int64_t stride,
                                                        double* __restrict__ partials)
 {
     __shared__ double sh[kBlock];
     const int c = blockIdx.y;
-    const int64_t chunk = (n + kReduceBlocks - 1) / kReduceBlocks;
-    const int64_t lo = (int64_t)blockIdx.x * chunk;
-    const int64_t hi = lo + chunk < n ? lo + chunk : n;
-    const double* row = in + c * stride;
-    const double acc = strided_sum<kBlock>(row, lo + threadIdx.x, hi);
-    const double s = block_sum(acc, sh);
+    const double s = sum_chunk(in + c * stride, n, blockIdx.x, sh);
     if (threadIdx.x == 0) partials[c * kReduceBlocks + blockIdx.x] = s;
 }
 
-__global__ __launch_bounds__(kBlock) void k_sum_stage2(const double* __restrict__ partials, double* __restrict__ out)
+// out[c] = the sum of row c's partials; err (optional): its value into
+// err_out and cleared for the next evaluation.  out and err_out may be pinned
+// host memory: a store instead of a copy per result.
+__global__ __launch_bounds__(kBlock) void k_sum_stage2(const double* __restrict__ partials, double* __restrict__ out,
+                                                       int* __restrict__ err, int* __restrict__ err_out)
 {
     __shared__ double sh[kBlock];
     const int c = blockIdx.x;
     double acc = 0.0;
     for (int i = threadIdx.x; i < kReduceBlocks; i += kBlock) acc += partials[c * kReduceBlocks + i];
     const double s = block_sum(acc, sh);
-    if (threadIdx.x == 0) out[c] = s;
+    if (threadIdx.x == 0)
+    {
+        out[c] = s;
+        if (err)
+        {
+            *err_out = *err;
+            *err = 0;
+        }
+    }
 }
 
 hipError_t launch_sum(const double* in, int64_t n, int ncand, int64_t stride, double* partials, double* out,
                       hipStream_t s)
 {
     k_sum_stage1<<<dim3(kReduceBlocks, ncand), kBlock, 0, s>>>(in, n, stride, partials);
-    k_sum_stage2<<<ncand, kBlock, 0, s>>>(partials, out);
+    k_sum_stage2<<<ncand, kBlock, 0, s>>>(partials, out, nullptr, nullptr);
     return hipGetLastError();
 }
 
@@ -103,7 +119,7 @@ __global__ __launch_bounds__(kBlock) void k_dot_stage1(const double* __restrict_
 hipError_t launch_dot(const double* a, const double* b, int64_t n, double* partials, double* out, hipStream_t s)
 {
     k_dot_stage1<<<kReduceBlocks, kBlock, 0, s>>>(a, b, n, partials);
-    k_sum_stage2<<<1, kBlock, 0, s>>>(partials, out);
+    k_sum_stage2<<<1, kBlock, 0, s>>>(partials, out, nullptr, nullptr);
     return hipGetLastError();
 }
 
@@ -141,11 +157,10 @@ hipError_t launch_axpy_point(const double* x0, const double* dir, const double* 
 // The element kernels scatter every d x d block (and every per-vertex gradient
 // part) to its slot; the slots of one destination are contiguous and in
 // element order, so each output entry is a fixed-order sum over one run.
-// sum_{c in [c0, c1)} src[c * S] in index order, four loads in flight
+// acc + src[c * S] for c in [c0, c1), in order
 template <int S, class T>
-__device__ __forceinline__ double run_sum(const T* __restrict__ src, int64_t c0, int64_t c1)
+__device__ __forceinline__ double run_tail(double acc, const T* __restrict__ src, int64_t c0, int64_t c1)
 {
-    double acc = 0.0;
     int64_t c = c0;
     for (; c + 4 <= c1; c += 4)
     {
@@ -160,43 +175,18 @@ __device__ __forceinline__ double run_sum(const T* __restrict__ src, int64_t c0,
     return acc;
 }
 
-// Runs exist for the upper blocks; a lower block (u, v), u > v, sums the run
-// of (v, u) transposed.  D*D lanes share one block (lane m sums entry m over
-// the run), so every contribution is read as one contiguous D*D-value segment
-// by consecutive lanes; a 64-lane wave serves floor(64 / D^2) blocks.
-template <class T, int D>
-__global__ __launch_bounds__(kBlock) void k_assemble_hessian(int64_t b_begin, int64_t nb, const int32_t* __restrict__ block_row,
-                                                             const int32_t* __restrict__ brow_ptr,
-                                                             const int64_t* __restrict__ hslot_ptr,
-                                                             const int32_t* __restrict__ mirror,
-                                                             const T* __restrict__ Hc,
-                                                             const int32_t* __restrict__ row_ptr,
-                                                             double* __restrict__ H)
+// sum_{c in [c0, c1)} src[c * S] in index order, four loads in flight
+template <int S, class T>
+__device__ __forceinline__ double run_sum(const T* __restrict__ src, int64_t c0, int64_t c1)
 {
-    constexpr int DD = D * D;
-    constexpr int BPW = 64 / DD;  // blocks per wave
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (lane >= BPW * DD) return;
-    const int64_t b = b_begin + wave * BPW + lane / DD;
-    if (b >= nb) return;
-    const int m = lane % DD;
-    const int u = block_row[b];
-    const int b0 = brow_ptr[u];
-    const int k = (int)(b - b0);
-    const int nbu = brow_ptr[u + 1] - b0;
-    const int i = m / D, j = m % D;
-    const int64_t mb = mirror[b];
-    const int src = (mb == b) ? m : j * D + i;
-    const int64_t c1 = hslot_ptr[mb + 1];
-    const double acc = run_sum<DD>(Hc + src, hslot_ptr[mb], c1);
-    H[(int64_t)row_ptr[D * u] + (int64_t)i * D * nbu + D * k + j] = acc;
+    return run_tail<S>(0.0, src, c0, c1);
 }
 
-// The same sums with one thread per block (all D*D entries of a contribution
-// per thread, two contributions in flight); identical bits.  Which shape is
-// faster depends on d, the precision and the run lengths (the autotuner times
-// both).
+// Runs exist for the upper blocks; a lower block (u, v), u > v, sums the run
+// of (v, u) transposed.
+// One thread per block (all D*D entries of a contribution per thread, two
+// contributions in flight).  Which shape is faster depends on d, the precision
+// and the run lengths (the autotuner times them).
 template <class T, int D>
 __global__ __launch_bounds__(kBlock) void k_assemble_hessian_tpb(int64_t b_begin, int64_t nb,
                                                                  const int32_t* __restrict__ block_row,
@@ -326,20 +316,183 @@ __global__ __launch_bounds__(kBlock) void k_assemble_hessian_upper_tpb(int64_t b
     }
 }
 
-// D lanes per handle, floor(64 / D) handles per wave.
+// D lanes per handle, floor(64 / D) handles per wave; wave index `wave`.
 template <class T, int D>
-__global__ __launch_bounds__(kBlock) void k_assemble_gradient(int64_t v_begin, int64_t nh,
-                                                              const int64_t* __restrict__ gslot_ptr,
-                                                              const T* __restrict__ G, double* __restrict__ g)
+__device__ __forceinline__ void gradient_rows(int64_t wave, int64_t v_begin, int64_t nh,
+                                              const int64_t* __restrict__ gslot_ptr, const T* __restrict__ G,
+                                              double* __restrict__ g)
 {
     constexpr int HPW = 64 / D;
     const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (lane >= HPW * D) return;
     const int64_t v = v_begin + wave * HPW + lane / D;
     if (v >= nh) return;
     const int i = lane % D;
     g[v * D + i] = run_sum<D>(G + i, gslot_ptr[v], gslot_ptr[v + 1]);
+}
+
+template <class T, int D>
+__global__ __launch_bounds__(kBlock) void k_assemble_gradient(int64_t v_begin, int64_t nh,
+                                                              const int64_t* __restrict__ gslot_ptr,
+                                                              const T* __restrict__ G, double* __restrict__ g)
+{
+    gradient_rows<T, D>(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6, v_begin, nh, gslot_ptr, G, g);
+}
+
+// A segment's energy: terms in order, fixed thread stride within each range,
+// fixed block tree.
+__device__ __forceinline__ double segment_total(const double* __restrict__ elem_f, const int64_t* __restrict__ ranges,
+                                                int n_terms, int64_t n_seg, int64_t sgm, double* sh)
+{
+    double acc = 0.0;
+    for (int t = 0; t < n_terms; ++t)
+    {
+        const int64_t a = ranges[(t * n_seg + sgm) * 2], b = ranges[(t * n_seg + sgm) * 2 + 1];
+        int64_t i = a + threadIdx.x;
+        for (; i + 3 * kBlock < b; i += 4 * kBlock)  // four loads in flight, same order
+        {
+            const double v0 = elem_f[i], v1 = elem_f[i + kBlock], v2 = elem_f[i + 2 * kBlock],
+                         v3 = elem_f[i + 3 * kBlock];
+            acc += v0;
+            acc += v1;
+            acc += v2;
+            acc += v3;
+        }
+        for (; i < b; i += kBlock) acc += elem_f[i];
+    }
+    return block_sum(acc, sh);
+}
+
+// Everything an evaluation does after its element kernels, in one launch: the
+// work is independent, and at small sizes each launch of its own is 2 .. 4 us
+// of mostly idle chip.  Blocks, in this order:
+//   tile_blocks   CSR values of H, one tile each: whole block rows holding at
+//                 most kAsmTileBlocks blocks.  One thread sums one block's
+//                 run (two contributions in flight), the values pass through
+//                 LDS and leave as one contiguous run.  The blocks of one XCD
+//                 (blockIdx % 8) take a contiguous eighth of the tiles, so a
+//                 run's second read, for the mirrored block, can hit in that
+//                 XCD's L2.  A row with more blocks is a tile of its own,
+//                 written directly.
+//   grad_blocks   gradient of kBlock / 64 waves of handles
+//   copy_blocks   x kept for the coarse space's lever arms
+//   kReduceBlocks first-stage sums of the element energies
+//   n_seg         segment energies
+// 25 x 25 grid: gradient, H, x copy and two sum launches, two result copies and
+// a clear, 13 us of kernels and 75 us per evaluation -> 3.3 + 2.5 us and 45 us.
+// 256 disks, mixed (430 MB of values written, 190 MB of runs read): 396 us with
+// D*D lanes per block, unstaged -> 180 us (3.4 TB/s).
+template <class T, int D>
+__global__ __launch_bounds__(kBlock) void k_assemble_all(EvalTail a)
+{
+    constexpr int DD = D * D;
+    __shared__ double sm[kAsmTileBlocks * DD < kBlock ? kBlock : kAsmTileBlocks * DD];
+    const int t = threadIdx.x;
+    int64_t blk = blockIdx.x;
+    if (blk < a.tile_blocks)
+    {
+        const int64_t per = a.tile_blocks >> 3;
+        const int64_t tile = (blk & 7) * per + (blk >> 3);
+        if (tile >= a.n_tiles) return;
+        const T* __restrict__ Hc = (const T*)a.Hc;
+        const int64_t b0 = a.tile_ptr[tile], b1 = a.tile_ptr[tile + 1];
+        const int nb = (int)(b1 - b0);
+        double* __restrict__ out = a.H + b0 * DD;
+        const bool direct = nb > kAsmTileBlocks;
+        for (int b = t; b < nb; b += kBlock)
+        {
+            const uint32_t run = a.arun[b0 + b], len = a.alen[b0 + b], pos = a.apos[b0 + b];
+            const T* __restrict__ src = Hc + (int64_t)(run & 0x7fffffffu) * DD;
+            double acc[DD];
+#pragma unroll
+            for (int m = 0; m < DD; ++m) acc[m] = 0.0;
+            uint32_t c = 0;
+            for (; c + 2 <= len; c += 2)
+            {
+                T v0[DD], v1[DD];
+#pragma unroll
+                for (int m = 0; m < DD; ++m)
+                {
+                    v0[m] = src[c * DD + m];
+                    v1[m] = src[(c + 1) * DD + m];
+                }
+#pragma unroll
+                for (int m = 0; m < DD; ++m)
+                {
+                    acc[m] += (double)v0[m];
+                    acc[m] += (double)v1[m];
+                }
+            }
+            if (c < len)
+            {
+#pragma unroll
+                for (int m = 0; m < DD; ++m) acc[m] += (double)src[c * DD + m];
+            }
+            const bool tr = run >> 31;  // the mirror's run, transposed
+            const int base = direct ? D * b : (int)(pos & 0xffffu), stride = direct ? D * nb : (int)(pos >> 16);
+#pragma unroll
+            for (int i = 0; i < D; ++i)
+#pragma unroll
+                for (int j = 0; j < D; ++j)
+                {
+                    const double e = tr ? acc[j * D + i] : acc[i * D + j];
+                    if (direct) out[base + (int64_t)i * stride + j] = e;
+                    else sm[base + i * stride + j] = e;
+                }
+        }
+        if (direct) return;
+        __syncthreads();
+        for (int i = t; i < nb * DD; i += kBlock) out[i] = sm[i];
+        return;
+    }
+    blk -= a.tile_blocks;
+    if (blk < a.grad_blocks)
+    {
+        gradient_rows<T, D>((blk * kBlock + t) >> 6, 0, a.n_handles, a.gslot_ptr, (const T*)a.G, a.g);
+        return;
+    }
+    blk -= a.grad_blocks;
+    if (blk < a.copy_blocks)
+    {
+        const int64_t i0 = blk * (4 * kBlock) + t;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + q * kBlock < a.n_handles * D) a.x_copy[i0 + q * kBlock] = a.x[i0 + q * kBlock];
+        return;
+    }
+    blk -= a.copy_blocks;
+    if (blk < kReduceBlocks)
+    {
+        const double s = sum_chunk(a.elem_f, a.n_elem, blk, sm);
+        if (t == 0) a.partials[blk] = s;
+        return;
+    }
+    blk -= kReduceBlocks;
+    const double s = segment_total(a.elem_f, a.seg_ranges, a.n_terms, a.n_seg, blk, sm);
+    if (t == 0) a.seg_f[blk] = s;
+}
+
+hipError_t launch_eval_tail(int d, int precision, EvalTail a, int* err, double* f_out, int* err_out, hipStream_t s)
+{
+    a.tile_blocks = a.H ? (a.n_tiles + 7) / 8 * 8 : 0;
+    const int64_t waves = a.g ? (a.n_handles + 64 / d - 1) / (64 / d) : 0;
+    a.grad_blocks = (waves * 64 + kBlock - 1) / kBlock;
+    a.copy_blocks = a.x_copy ? (a.n_handles * d + 4 * kBlock - 1) / (4 * kBlock) : 0;
+    const int64_t grid = a.tile_blocks + a.grad_blocks + a.copy_blocks + kReduceBlocks + a.n_seg;
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+#define TAD_TAIL(T, D) k_assemble_all<T, D><<<(unsigned)grid, kBlock, 0, s>>>(a)
+    if (precision == 0)
+    {
+        if (d == 1) TAD_TAIL(double, 1);
+        else if (d == 2) TAD_TAIL(double, 2);
+        else TAD_TAIL(double, 3);
+    }
+    else if (d == 1) TAD_TAIL(float, 1);
+    else if (d == 2) TAD_TAIL(float, 2);
+    else TAD_TAIL(float, 3);
+#undef TAD_TAIL
+    k_sum_stage2<<<1, kBlock, 0, s>>>(a.partials, f_out, err, err_out);
+    return hipGetLastError();
 }
 
 // Blocks [b0, b1) of the shape's index space: CSR blocks (shapes 0, 1) or
@@ -353,10 +506,7 @@ static void launch_assemble_hessian_td(int shape, const HessAsm& a, int64_t b0, 
     if (n <= 0) return;
     const unsigned gt = (unsigned)((n + kBlock - 1) / kBlock);
     const unsigned gl = (unsigned)((((n + bpw - 1) / bpw) * 64 + kBlock - 1) / kBlock);
-    if (shape == 0)
-        k_assemble_hessian<T, D><<<gl, kBlock, 0, s>>>(b0, b1, a.block_row, a.brow_ptr, a.hslot_ptr, a.mirror, Hc,
-                                                       a.row_ptr, H);
-    else if (shape == 1)
+    if (shape <= 1)  // (a range of rows has no whole tiles: shape 1 for shape 0)
         k_assemble_hessian_tpb<T, D><<<gt, kBlock, 0, s>>>(b0, b1, a.block_row, a.brow_ptr, a.hslot_ptr, a.mirror,
                                                            Hc, a.row_ptr, H);
     else if (shape == 2)
@@ -1575,33 +1725,15 @@ hipError_t launch_pcg_advance(PcgScalars* sc, hipStream_t s)
 }
 
 // ---------------------------------------------------------------------------
-// Per-segment energy sums (fixed order: terms in order, fixed thread stride
-// within each range, fixed block tree)
+// Per-segment energy sums
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_segment_sum(const double* __restrict__ elem_f,
                                                         const int64_t* __restrict__ ranges, int n_terms,
                                                         int64_t n_seg, double* __restrict__ out)
 {
     __shared__ double sh[kBlock];
-    const int64_t sgm = blockIdx.x;
-    double acc = 0.0;
-    for (int t = 0; t < n_terms; ++t)
-    {
-        const int64_t a = ranges[(t * n_seg + sgm) * 2], b = ranges[(t * n_seg + sgm) * 2 + 1];
-        int64_t i = a + threadIdx.x;
-        for (; i + 3 * kBlock < b; i += 4 * kBlock)  // four loads in flight, same order
-        {
-            const double v0 = elem_f[i], v1 = elem_f[i + kBlock], v2 = elem_f[i + 2 * kBlock],
-                         v3 = elem_f[i + 3 * kBlock];
-            acc += v0;
-            acc += v1;
-            acc += v2;
-            acc += v3;
-        }
-        for (; i < b; i += kBlock) acc += elem_f[i];
-    }
-    const double s = block_sum(acc, sh);
-    if (threadIdx.x == 0) out[sgm] = s;
+    const double s = segment_total(elem_f, ranges, n_terms, n_seg, blockIdx.x, sh);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 hipError_t launch_segment_sum(const double* elem_f, const int64_t* ranges, int n_terms, int64_t n_seg, double* out,
