@@ -425,7 +425,7 @@ typedef struct tad_solve_opts
     double w_identity;  /* regularization w in (w I + H) d = rhs (NewtonDirection.hh:32)  */
     double tol;         /* relative residual ||r|| <= tol ||rhs||                        */
     int max_iters;
-    int check_every;    /* host polls convergence every this many iterations             */
+    int check_every;    /* no longer used: the device reports its progress to the host   */
     int coarse_aggregate; /* two-level preconditioner: handles per aggregate of the      */
                         /* coarse space; 0: block-Jacobi only; < 0 (default): automatic, */
                         /* by mesh size (in 3D about 700 coarse unknowns up to 30K       */

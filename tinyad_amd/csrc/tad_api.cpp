@@ -18,6 +18,7 @@
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -293,6 +294,8 @@ struct tad_fn_s
     bool err_clear = false;  // the flag in err is 0 (the last kernel of an evaluation clears it)
     // line search
     DevBuf<double> ls_f, x_tmp;
+    double steps_host[kMaxTrials] = {};  // what steps holds (steps_valid)
+    bool steps_valid = false;
     // solver
     DevBuf<double> Dinv, xs, r, z, p, q, sol;  // xs: the iterate in solver order
     DevBuf<unsigned char> free_s;              // free-variable mask in solver order
@@ -318,8 +321,7 @@ struct tad_fn_s
         DevBuf<int64_t> gchunk_ptr;
         DevBuf<double> dvec, dvec_h, Ac, rpart, cparts, gpart, inv_work, rowsum;
         DevBuf<float> Ainv32;  // the inverse in FP32 with a diagonal shift, read by every CG iteration
-        bool use32 = false;    // Ainv32 belongs to the current factor
-        DevBuf<int> info;
+        DevBuf<int> info;      // the inversion's flag, then the iterations' mode (launch_coarse_mode)
         // the inverse coarse matrix in Ac and the lever arms in dvec belong
         // together and stay usable by a later solve that asks for reuse when
         // it needs the same aggregates, kc and w and neither solve is reduced
@@ -353,8 +355,6 @@ struct tad_fn_s
     DevBuf<int32_t> bas_rp, bas_ci, bas_tp, bas_tc;
     DevBuf<double> bas_v, bas_tv, bas_vec;
     bool x_hess_valid = false;
-    int last_solve_iters = 0;  // iterations of the previous solve (first poll of the next one)
-    int last_dense_iters = 1;  // the same with the dense preconditioner
     // CG iterations recorded as a HIP graph (tad_fn_set_solve_graphs): the
     // executable graph and the operands it was recorded with
     int solve_graphs = 0;      // 1 on, 0 off
@@ -1077,6 +1077,13 @@ constexpr double kCoarse32Change = 0.1;
 // *use = false when the coarse space is off or A_c is not numerically
 // positive definite (block-Jacobi alone then).  With o.coarse_reuse the
 // inverse and lever arms of the previous compatible solve are kept (*reused).
+// Regions of the context's pinned buffer (256 doubles): 0 .. 1 energy and error
+// flag of an evaluation, 16 .. 23 step sizes, 32 .. 51 energies and products,
+// and these.
+PcgReport* pcg_report(tad_fn fn) { return reinterpret_cast<PcgReport*>(fn->ctx->pinned + 56); }
+LineSearchHost* ls_host(tad_fn fn) { return reinterpret_cast<LineSearchHost*>(fn->ctx->pinned + 72); }
+int* mode_host(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 96); }
+
 tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o, const unsigned char* free_dev,
                         PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused, bool lagged)
 {
@@ -1127,7 +1134,9 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     cd->agg_ptr = c.agg_ptr.p;
     cd->dvec = c.dvec.p;
     cd->Ainv = c.Ac.p;
-    cd->Ainv32 = c.use32 ? c.Ainv32.p : nullptr;
+    TAD_HIP(c.Ainv32.ensure((size_t)(nc * nc)));
+    cd->Ainv32 = c.Ainv32.p;
+    cd->coarse_mode = c.info.p + 1;
     cd->rpart = c.rpart.p;
     cd->cparts = c.cparts.p;
     if (o.coarse_reuse && c.factor_valid && !free_dev && c.f_kc == kc && c.f_w == o.w_identity)
@@ -1137,8 +1146,6 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
         return TAD_OK;
     }
     c.factor_valid = false;
-    c.use32 = false;
-    cd->Ainv32 = nullptr;
     tm.begin("coarse_setup", s);
     tm.begin("coarse_galerkin", s);
     if (rot)
@@ -1159,36 +1166,11 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     tm.begin("coarse_inverse", s);
     TAD_HIP(launch_spd_inverse(nc, c.Ac.p, c.inv_work.p, c.info.p, s));
     tm.end("coarse_inverse", s);
-    TAD_HIP(launch_abs_rowmax(nc, c.Ac.p, c.rowsum.p, c.rowsum.p + nc + 1, s));
-    int* info = reinterpret_cast<int*>(fn->ctx->pinned + 96);  // past the solver scalars at 56..
-    double* norms = reinterpret_cast<double*>(fn->ctx->pinned + 104);
-    TAD_HIP(hipMemcpyAsync(info, c.info.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    TAD_HIP(hipMemcpyAsync(norms, c.rowsum.p + nc, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-    TAD_HIP(hipStreamSynchronize(s));
-    if (info[0] != 0)
-    {
-        tm.end("coarse_setup", s);
-        return TAD_OK;  // not positive definite at working precision: block-Jacobi alone
-    }
-    // The CG iterations read an FP32 copy with the diagonal shift
-    // delta = 2^-23 ||A_c^-1||_inf that keeps it positive definite
-    // (launch_coarse_to32) when the shift is small against the smallest
-    // eigenvalue of A_c^-1, 1 / lambda_max(A_c) >= 1 / ||A_c||_inf:
-    // 2^-22 kappa_inf <= 0.1 bounds the relative change of the coarse
-    // correction by 10 %.  Otherwise (e.g. a Hessian that is singular up to
-    // the projection's eps along rigid motions) they read the FP64 inverse.
-    const double kappa = norms[0] * norms[1];
-    if (std::isfinite(kappa) && std::ldexp(kappa, -22) <= kCoarse32Change)
-    {
-        TAD_HIP(c.Ainv32.ensure((size_t)(nc * nc)));
-        TAD_HIP(launch_coarse_to32(nc, c.Ac.p, std::ldexp(norms[1], -23), c.Ainv32.p, s));
-        c.use32 = true;
-        cd->Ainv32 = c.Ainv32.p;
-    }
+    TAD_HIP(launch_coarse_mode(nc, c.Ac.p, c.rowsum.p, c.rowsum.p + nc, c.info.p, kCoarse32Change, c.info.p + 1,
+                               mode_host(fn), c.Ainv32.p, s));
     tm.end("coarse_setup", s);
     *use = true;
-    c.factor_valid = !free_dev;
-    c.f_kc = kc;
+    c.f_kc = kc;  // usable by a later solve once the mode is known (solve_once)
     c.f_w = o.w_identity;
     return TAD_OK;
 }
@@ -1207,7 +1189,7 @@ tad_status ensure_ready(tad_fn fn)
     TAD_HIP(fn->x_buf.ensure((size_t)fn->n_vars));
     TAD_HIP(fn->g_buf.ensure((size_t)fn->n_vars));
     TAD_HIP(fn->H_buf.ensure((size_t)fn->nnz));
-    TAD_HIP(fn->partials.ensure(8 * kReduceBlocks + 4096));
+    TAD_HIP(fn->partials.ensure((kMaxTrials + 2) * kReduceBlocks + 4096));
     TAD_HIP(fn->steps.ensure(16));
     TAD_HIP(fn->err.ensure(1));
     return TAD_OK;
@@ -1316,6 +1298,19 @@ void set_tiles(tad_fn fn, EvalTail& tail, double* H_dev)
     tail.H = H_dev;
 }
 
+// f null: the results are left in flight (eval_result collects them after the
+// stream has been waited for).
+tad_status eval_result(tad_fn fn, double* f)
+{
+    fn->err_clear = true;
+    const double* pin = fn->ctx->pinned;
+    int errv = 0;
+    std::memcpy(&errv, pin + 1, sizeof(int));
+    *f = pin[0];
+    if (errv) return fail(TAD_ERR_NONFINITE, "non-finite element gradient or Hessian");
+    return TAD_OK;
+}
+
 tad_status eval_core(tad_fn fn, const double* x_dev, int mode, double eps, double* g_dev, double* H_dev, double* f)
 {
     hipStream_t s = fn->s();
@@ -1410,42 +1405,29 @@ tad_status eval_core(tad_fn fn, const double* x_dev, int mode, double eps, doubl
     tm.begin("assemble", s);
     TAD_HIP(launch_eval_tail(fn->d, fn->precision, tail, fn->err.p, pin, reinterpret_cast<int*>(pin + 1), s));
     tm.end("assemble", s);
+    if (!f) return TAD_OK;
     TAD_HIP(hipStreamSynchronize(s));
-    fn->err_clear = true;
-    int errv = 0;
-    std::memcpy(&errv, pin + 1, sizeof(int));
-    *f = pin[0];
-    if (errv) return fail(TAD_ERR_NONFINITE, "non-finite element gradient or Hessian");
-    return TAD_OK;
+    return eval_result(fn, f);
 }
 
-tad_status eval_energy_batch(tad_fn fn, const double* x_dev, const double* dir_dev, const double* steps_host, int ncand,
-                             double* f_out)
+// The passive energy at x (synchronizes).
+tad_status eval_energy(tad_fn fn, const double* x_dev, double* f_out)
 {
     hipStream_t s = fn->s();
     KernelTimer& tm = fn->ctx->timer;
     const int64_t ne = fn->n_elem_total;
-    if (dir_dev)
-    {
-        TAD_HIP(fn->ls_f.ensure((size_t)ne * 8));
-        double* pin = fn->ctx->pinned;
-        std::memcpy(pin + 16, steps_host, ncand * sizeof(double));
-        TAD_HIP(hipMemcpyAsync(fn->steps.p, pin + 16, ncand * sizeof(double), hipMemcpyHostToDevice, s));
-    }
-    double* dst = dir_dev ? fn->ls_f.p : fn->elem_f.p;
-    const int nc = dir_dev ? ncand : 1;
     tm.begin("energy", s);
     for (const TermDev& t : fn->terms)
-        TAD_HIP(launch_energy(t, fn->d, x_dev, dir_dev, fn->steps.p, nc, dst, ne, s));
+        TAD_HIP(launch_energy(t, fn->d, x_dev, nullptr, fn->steps.p, 1, fn->elem_f.p, ne, s));
     tm.end("energy", s);
-    tm.begin("energy_sum", s);
     double* pin = fn->ctx->pinned;
-    TAD_HIP(launch_sum(dst, ne, nc, ne, fn->partials.p, pin + 32, s));
-    if (!dir_dev && fn->n_seg > 0)
+    tm.begin("energy_sum", s);
+    TAD_HIP(launch_sum(fn->elem_f.p, ne, 1, ne, fn->partials.p, pin + 32, s));
+    if (fn->n_seg > 0)
         TAD_HIP(launch_segment_sum(fn->elem_f.p, fn->seg_ranges.p, (int)fn->terms.size(), fn->n_seg, fn->seg_f.p, s));
     tm.end("energy_sum", s);
     TAD_HIP(hipStreamSynchronize(s));
-    for (int c = 0; c < nc; ++c) f_out[c] = pin[32 + c];
+    *f_out = pin[32];
     return TAD_OK;
 }
 
@@ -1475,6 +1457,8 @@ tad_status dot2_dev(tad_fn fn, const double* a1, const double* b1, const double*
 
 // Recorded CG launches: iterations per graph.
 constexpr int kGraphIters = 8;
+// CG iterations launched beyond the last one the device has reported.
+constexpr int kAhead = 3;
 
 // Every operand the recorded CG launches hold: the graph is recorded again
 // when any of them changes.
@@ -1486,9 +1470,9 @@ std::vector<uint64_t> pcg_graph_key(int d, const PcgSystem& a, hipStream_t s)
     std::memcpy(&tbits, &a.tol2, sizeof(a.tol2));
     return { (uint64_t)d, (uint64_t)a.nh, u(a.perm), u(a.brow_ptr), u(a.bcol), u(a.sym_ptr), u(a.usrc), u(a.diag), u(a.Hs),
              u(a.part_ptr), (uint64_t)a.Gs, (uint64_t)a.Gv, wbits, tbits, (uint64_t)a.max_iters, u(a.b), u(a.sol),
-             u(a.Dinv), u(a.x), u(a.r), u(a.z), u(a.p), u(a.q), u(a.s), u(a.parts), u(a.sc), u(a.free_h), u(a.free_s),
+             u(a.Dinv), u(a.x), u(a.r), u(a.z), u(a.p), u(a.q), u(a.s), u(a.parts), u(a.sc), u(a.host), u(a.free_h), u(a.free_s),
              (uint64_t)a.kc, (uint64_t)a.dense, (uint64_t)a.ppa, (uint64_t)a.n_agg, (uint64_t)a.nc, u(a.agg_ptr), u(a.dvec), u(a.Ainv),
-             u(a.Ainv32), u(a.rpart), u(a.cparts), u(s) };
+             u(a.Ainv32), u(a.coarse_mode), u(a.rpart), u(a.cparts), u(s) };
 }
 
 // Systems of at most this many variables are solved with the dense inverse of
@@ -1597,22 +1581,14 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
             tm.end("coarse_setup", s);
         }
     }
+    PcgReport* rep = pcg_report(fn);
+    volatile int* state = &rep->state;
+    *state = 0;  // no kernel of an earlier solve writes it any more
+    sys.host = rep;
     tm.begin("pcg_init", s);
     TAD_HIP(launch_pcg_init(d, sys, s));
     tm.end("pcg_init", s);
-    PcgScalars hs;
-    PcgScalars* pin = (PcgScalars*)(fn->ctx->pinned + 56);
-    const int every = std::max(1, o.check_every);
     Timer* timer = fn->ctx->timer.enabled ? &fn->ctx->timer : nullptr;
-    // iterations are launched in chunks; every kernel returns at once after
-    // the device has recorded termination, so overshooting a chunk is cheap.
-    // Iteration k = max_iters launches only the SpMV, whose termination test
-    // then always fires.
-    // The first poll waits for 3/4 of the previous solve's iteration count
-    // (Newton steps need similar counts), later ones come every `every`:
-    // each poll stalls the device for a host round trip.
-    int k = 0;
-    int chunk = dense ? fn->last_dense_iters + 1 : std::max(every, fn->last_solve_iters * 3 / 4);
     // recorded launches: kGraphIters iterations, each followed by the
     // device-side iteration counter's advance, replayed until termination
     // (every kernel returns at once after it, and iteration max_iters stops
@@ -1662,52 +1638,58 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
             }
         }
     }
+    // The host launches at most kAhead iterations beyond the last one the
+    // device has reported, so that the stream never runs dry, it never stops
+    // for a copy, and only a few launches find the solve terminated (each
+    // kernel returns at once then).  Iteration k = max_iters launches only the
+    // SpMV, whose termination test then always fires.
+    const int step = gexec ? kGraphIters : 1;
+    int k = 0;
     while (k <= sys.max_iters)
     {
-        if (gexec)
-        {
-            for (int c = 0; c < chunk && k <= sys.max_iters; c += kGraphIters, k += kGraphIters)
-                TAD_HIP(hipGraphLaunch(gexec, s));
-        }
-        else
-        {
-            for (int c = 0; c < chunk && k <= sys.max_iters; ++c, ++k)
-                TAD_HIP(launch_pcg_iteration(d, sys, k, k < sys.max_iters, s, timer));
-        }
-        int* info = reinterpret_cast<int*>(fn->ctx->pinned + 96);
-        info[0] = 0;
-        if (dense && !coarse_reused) TAD_HIP(hipMemcpyAsync(info, fn->co.info.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        TAD_HIP(hipMemcpyAsync(pin, fn->scal.p, sizeof(hs), hipMemcpyDeviceToHost, s));
-        TAD_HIP(hipStreamSynchronize(s));
-        if (info[0] != 0)  // a pivot was not positive: not the preconditioner for this matrix
-        {
-            *again = true;
-            return TAD_OK;
-        }
-        if (pin->done) break;
-        chunk = dense ? 2 : every;
+        int seen = *state;
+        for (int64_t spins = 0; seen >= 0 && k - seen >= kAhead; seen = *state)
+            if (++spins % 4096 == 0)
+            {
+                // an error, or everything has run without reaching the end
+                const hipError_t e = hipStreamQuery(s);
+                if (e == hipSuccess && *state >= 0 && k - *state >= kAhead)
+                    return fail(TAD_ERR_SOLVE, "PCG did not report progress");
+                if (e != hipSuccess && e != hipErrorNotReady) TAD_HIP(e);
+            }
+        if (seen < 0) break;
+        if (gexec) TAD_HIP(hipGraphLaunch(gexec, s));
+        else TAD_HIP(launch_pcg_iteration(d, sys, k, k < sys.max_iters, s, timer));
+        k += step;
     }
-    if (!pin->done) return fail(TAD_ERR_SOLVE, "PCG did not report termination");
-    std::memcpy(&hs, pin, sizeof(hs));
-    if (dense && sys.max_iters < o.max_iters && !(hs.rr <= sys.tol2 * hs.bb))
+    while (*state >= 0)
+    {
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipSuccess && *state >= 0) return fail(TAD_ERR_SOLVE, "PCG did not report termination");
+        if (e != hipSuccess && e != hipErrorNotReady) TAD_HIP(e);
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    const PcgReport hs = *rep;
+    if (dense && (hs.breakdown || (sys.max_iters < o.max_iters && !(hs.rr <= sys.tol2 * hs.bb))))
     {
         *again = true;
         return TAD_OK;
     }
+    if (!dense && use_coarse && !coarse_reused)
+    {
+        use_coarse = *mode_host(fn) != 0;  // 0: A_c not positive definite at working precision
+        fn->co.factor_valid = use_coarse && !free_dev;
+    }
     if (dense)
     {
-        fn->co.dense_valid = !free_dev && !hs.breakdown;
+        fn->co.dense_valid = !free_dev;
         fn->co.dense_w = o.w_identity;
-        fn->last_dense_iters = hs.iters;
     }
-    else
-        fn->last_solve_iters = hs.iters;
     fn->solves_since_rebuild = coarse_reused ? fn->solves_since_rebuild + 1 : 0;
     const double rel = hs.bb > 0 ? std::sqrt(hs.rr / hs.bb) : 0.0;
     if (hs.breakdown)  // no product wrote the solution: the last iterate
     {
         TAD_HIP(launch_pcg_solution(d, sys, s));
-        TAD_HIP(hipStreamSynchronize(s));
     }
     if (st)
     {
@@ -1739,50 +1721,80 @@ tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
 
 // Armijo backtracking on device data (LineSearch.hh:26-65).  The direction is
 // dir_scale * dir (dir_scale = -1 lets the Newton step pass the solution of
-// H d' = g without negating it).  Writes the accepted point to x_out.
+// H d' = g without negating it).  Writes the accepted point to x_out.  The
+// products dir . g and (dot2 set) g . g are formed with the first batch of
+// trials, so that one wait serves them, the energies, the decision and x_out.
 tad_status line_search_core(tad_fn fn, const double* x0, const double* dir, double dir_scale, double f,
-                            double dir_dot_g, double* x_out, const tad_newton_opts& o, double* f_out, double* s_out,
-                            int* trials, bool* failed)
+                            const double* g, double* x_out, const tad_newton_opts& o, double* f_out, double* s_out,
+                            int* trials, bool* failed, double* dir_dot, double* dot2)
 {
     if (!(o.ls_s_max > 0.0)) return fail(TAD_ERR_INVALID, "Max step size not positive.");
     const bool try_one = o.ls_s_max > 1.0;
-    const int batch = std::min(8, std::max(1, o.ls_batch));
-    double s = o.ls_s_max;
+    const int batch = std::min(kMaxTrials, std::max(1, o.ls_batch));
+    hipStream_t s = fn->s();
+    KernelTimer& tm = fn->ctx->timer;
+    const int64_t ne = fn->n_elem_total;
+    TAD_HIP(fn->ls_f.ensure((size_t)ne * kMaxTrials));
+    LineSearchHost* host = ls_host(fn);
+    double sv = o.ls_s_max;
     int it = 0;
     *failed = false;
-    while (it < o.ls_max_iters)
+    if (o.ls_max_iters <= 0) TAD_TRY(dot2_dev(fn, dir, g, g, g, dir_dot, dot2));
+    for (bool first = true; it < o.ls_max_iters; first = false)
     {
-        const int nc = std::min(batch, o.ls_max_iters - it);
-        double svals[8], steps[8], fv[8];
-        for (int c = 0; c < nc; ++c)
+        LineSearchBatch b;
+        b.ncand = std::min(batch, o.ls_max_iters - it);
+        for (int c = 0; c < b.ncand; ++c)
         {
-            svals[c] = s;
-            steps[c] = dir_scale * s;
-            if (try_one && s > 1.0 && s * o.ls_shrink < 1.0) s = 1.0;
-            else s *= o.ls_shrink;
+            b.sval[c] = sv;
+            b.step[c] = dir_scale * sv;
+            if (try_one && sv > 1.0 && sv * o.ls_shrink < 1.0) sv = 1.0;
+            else sv *= o.ls_shrink;
         }
-        TAD_TRY(eval_energy_batch(fn, x0, dir, steps, nc, fv));
-        for (int c = 0; c < nc; ++c)
+        // the step sizes on the device: most searches try the same ones
+        if (!fn->steps_valid || std::memcmp(fn->steps_host, b.step, sizeof(b.step)) != 0)
         {
-            ++it;
-            if (fv[c] != fv[c]) return fail(TAD_ERR_NAN_ENERGY, "energy is NaN in line search");
-            if (fv[c] <= f + o.ls_armijo * svals[c] * dir_dot_g)
-            {
-                double* pin = fn->ctx->pinned;
-                pin[24] = steps[c];
-                TAD_HIP(hipMemcpyAsync(fn->steps.p + 8, pin + 24, sizeof(double), hipMemcpyHostToDevice, fn->s()));
-                TAD_HIP(launch_axpy_point(x0, dir, fn->steps.p + 8, fn->n_vars, x_out, fn->s()));
-                TAD_HIP(hipStreamSynchronize(fn->s()));
-                *f_out = fv[c];
-                *s_out = svals[c];
-                *trials = it;
-                return TAD_OK;
-            }
+            fn->steps_valid = false;
+            double* pin = fn->ctx->pinned;
+            std::memcpy(pin + 16, b.step, sizeof(b.step));
+            TAD_HIP(hipMemcpyAsync(fn->steps.p, pin + 16, sizeof(b.step), hipMemcpyHostToDevice, s));
+            std::memcpy(fn->steps_host, b.step, sizeof(b.step));
+            fn->steps_valid = true;
         }
+        tm.begin("energy", s);
+        for (const TermDev& t : fn->terms)
+            TAD_HIP(launch_energy(t, fn->d, x0, dir, fn->steps.p, b.ncand, fn->ls_f.p, ne, s));
+        tm.end("energy", s);
+        b.f = f;
+        b.armijo = o.ls_armijo;
+        b.dir_scale = dir_scale;
+        b.use_dots = first;
+        b.dir_dot_g = first ? 0.0 : dir_scale * *dir_dot;
+        b.step_out = fn->steps.p + kMaxTrials;
+        b.accepted_out = reinterpret_cast<int*>(fn->steps.p + kMaxTrials + 1);
+        b.host = host;
+        tm.begin("line_search", s);
+        TAD_HIP(launch_ls_finish(b, fn->ls_f.p, ne, ne, fn->partials.p, dir, g, g, g, fn->n_vars, x0, dir, x_out, s));
+        tm.end("line_search", s);
+        TAD_HIP(hipStreamSynchronize(s));
+        if (first)
+        {
+            *dir_dot = host->dir_dot;
+            *dot2 = host->dot2;
+        }
+        if (host->accepted == -2) return fail(TAD_ERR_NAN_ENERGY, "energy is NaN in line search");
+        if (host->accepted >= 0)
+        {
+            *f_out = host->f[host->accepted];
+            *s_out = b.sval[host->accepted];
+            *trials = it + host->accepted + 1;
+            return TAD_OK;
+        }
+        it += b.ncand;
     }
     if (x_out != x0)
-        TAD_HIP(hipMemcpyAsync(x_out, x0, fn->n_vars * sizeof(double), hipMemcpyDeviceToDevice, fn->s()));
-    TAD_HIP(hipStreamSynchronize(fn->s()));
+        TAD_HIP(hipMemcpyAsync(x_out, x0, fn->n_vars * sizeof(double), hipMemcpyDeviceToDevice, s));
+    TAD_HIP(hipStreamSynchronize(s));
     *f_out = f;
     *s_out = 0.0;
     *trials = it;
@@ -2267,7 +2279,7 @@ tad_status tad_fn_eval(tad_fn fn, const double* x, tad_mem mem, double* f)
     const double* xd = stage_x(fn, x, mem);
     if (!xd) return fail(TAD_ERR_HIP, "copy of x to the device failed");
     double fv = 0.0;
-    TAD_TRY(eval_energy_batch(fn, xd, nullptr, nullptr, 1, &fv));
+    TAD_TRY(eval_energy(fn, xd, &fv));
     *f = fv;
     return TAD_OK;
 }
@@ -2493,11 +2505,8 @@ static tad_status solve_entry(tad_fn fn, const double* H_values, const double* r
         xd = fn->sol.p;
     }
     tad_status st = solve_core(fn, Hd, bd, xd, o, stats, fd);
-    if (mem == TAD_MEM_HOST)
-    {
-        TAD_HIP(hipMemcpyAsync(sol, xd, n * sizeof(double), hipMemcpyDeviceToHost, s));
-        TAD_HIP(hipStreamSynchronize(s));
-    }
+    if (mem == TAD_MEM_HOST) TAD_HIP(hipMemcpyAsync(sol, xd, n * sizeof(double), hipMemcpyDeviceToHost, s));
+    TAD_HIP(hipStreamSynchronize(s));  // the launch that found the end writes the solution
     return st;
 }
 
@@ -2732,12 +2741,10 @@ tad_status tad_line_search(tad_fn fn, const double* x0, const double* dir, doubl
     tad_newton_opts o;
     tad_newton_default_opts(&o);
     if (opts) o = *opts;
-    double dg = 0.0;
-    TAD_TRY(dot_dev(fn, dir, g, &dg));
-    double fo = 0, so = 0;
+    double dg = 0.0, gg = 0.0, fo = 0, so = 0;
     int tr = 0;
     bool failed = false;
-    TAD_TRY(line_search_core(fn, x0, dir, 1.0, f, dg, x_out, o, &fo, &so, &tr, &failed));
+    TAD_TRY(line_search_core(fn, x0, dir, 1.0, f, g, x_out, o, &fo, &so, &tr, &failed, &dg, &gg));
     if (f_out) *f_out = fo;
     if (step_out) *step_out = so;
     if (trials_out) *trials_out = failed ? -tr : tr;
@@ -2793,29 +2800,40 @@ tad_status tad_newton_step(tad_fn fn, double* x, tad_mem mem, const tad_newton_o
     // a NaN eps selects the unprojected Hessian, as eval_with_derivatives
     // passes eps = NAN to the shared evaluation (ScalarFunctionImpl.hh:333)
     const int mode = std::isnan(o.projection_eps) ? MODE_HESS : MODE_HESS_PROJ;
-    TAD_TRY(eval_core(fn, xd, mode, o.projection_eps, fn->g_buf.p, fn->H_buf.p, &f));
-    fn->h_valid = true;
-    st.f = f;
+    // the evaluation's energy and error flag are collected after the solve
+    // (queued behind it): one wait less per step
+    TAD_TRY(eval_core(fn, xd, mode, o.projection_eps, fn->g_buf.p, fn->H_buf.p, nullptr));
     // solve (wI + H) d' = g; the Newton direction is d = -d'
     TAD_HIP(fn->sol.ensure(n));
     tad_solve_stats ss;
     std::memset(&ss, 0, sizeof(ss));
     tad_solve_opts sopt = o.solve;
     if (o.coarse_refresh > 1 && fn->solves_since_rebuild + 1 < o.coarse_refresh) sopt.coarse_reuse = 1;
-    TAD_TRY(solve_core(fn, fn->H_buf.p, fn->g_buf.p, fn->sol.p, sopt, &ss, nullptr, o.coarse_refresh > 1));
+    const tad_status solved =
+        solve_core(fn, fn->H_buf.p, fn->g_buf.p, fn->sol.p, sopt, &ss, nullptr, o.coarse_refresh > 1);
+    if (solved != TAD_OK)
+    {
+        const std::string why = g_last_error;
+        TAD_HIP(hipStreamSynchronize(s));
+        TAD_TRY(eval_result(fn, &f));
+        fn->h_valid = true;
+        return fail(solved, why);
+    }
+    TAD_TRY(eval_result(fn, &f));
+    fn->h_valid = true;
+    st.f = f;
     st.cg_iters = ss.iters;
     st.solve_converged = ss.converged;
     st.coarse_unknowns = ss.coarse_unknowns;
     st.coarse_reused = ss.coarse_reused;
     double dpg = 0.0, gg = 0.0;
-    TAD_TRY(dot2_dev(fn, fn->sol.p, fn->g_buf.p, fn->g_buf.p, fn->g_buf.p, &dpg, &gg));
-    const double dg = -dpg;  // d^T g
-    st.grad_norm = std::sqrt(gg);
-    st.newton_decrement = -0.5 * dg;
     double fo = 0, so = 0;
     int tr = 0;
     bool failed = false;
-    TAD_TRY(line_search_core(fn, xd, fn->sol.p, -1.0, f, dg, xd, o, &fo, &so, &tr, &failed));
+    TAD_TRY(line_search_core(fn, xd, fn->sol.p, -1.0, f, fn->g_buf.p, xd, o, &fo, &so, &tr, &failed, &dpg, &gg));
+    const double dg = -dpg;  // d^T g
+    st.grad_norm = std::sqrt(gg);
+    st.newton_decrement = -0.5 * dg;
     st.f_new = fo;
     st.step = so;
     st.ls_trials = tr;

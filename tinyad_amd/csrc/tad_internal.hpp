@@ -61,11 +61,42 @@ constexpr int kGroupMaxBlocks = 224;  // 4 waves x 224 x 9 doubles < 64 KiB of L
 // Solver bookkeeping written by block 0 of the PCG kernels (see tad_linalg.hip).
 struct PcgScalars
 {
-    double bb, rr;
+    double bb;
     double rho_hist[2], alpha_hist[2];  // rho_k and alpha_k, slot k & 1
-    int iters, breakdown;
     int done;  // 0; k + 1 when iteration k's product found the end; -1 after a breakdown
     int k;  // iteration index for launches that read it from here (graph replays)
+};
+
+// What the host sees of a solve (pinned memory).  state: 0 before the first
+// product, k + 1 once iteration k's product has found that the solve goes on,
+// -1 at the end, with the other members set.
+struct PcgReport
+{
+    double rr, bb;
+    int iters, breakdown;
+    int state;
+};
+
+// One batch of line-search trials at x0 + step[c] dir, step[c] = dir_scale *
+// sval[c]; results in `host` (pinned), the accepted step also on the device.
+constexpr int kMaxTrials = 8;
+struct LineSearchHost
+{
+    double f[kMaxTrials];
+    double dir_dot, dot2;  // use_dots: dir . g, and a second product
+    int accepted;          // candidate, -1 none, -2 NaN energy
+};
+struct LineSearchBatch
+{
+    int ncand = 0;
+    double f = 0.0, armijo = 0.0, dir_scale = 1.0;
+    bool use_dots = false;    // (dir_scale * dir) . g from this batch's dot products
+    double dir_dot_g = 0.0;   // otherwise
+    double sval[kMaxTrials] = {}, step[kMaxTrials] = {};
+    double* step_out = nullptr;    // device
+    int* accepted_out = nullptr;   // device
+    LineSearchHost* host = nullptr;
+    const double *partials = nullptr, *dot_partials = nullptr;  // set by the launcher
 };
 
 // Kernel timing hook (set by the host library when timing is enabled).
@@ -185,9 +216,14 @@ hipError_t launch_eval_tail(int d, int precision, EvalTail a, int* err, double* 
 
 hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s);
 
-// x_out = x0 + step * dir  (same rounding as the line-search energy kernel)
-hipError_t launch_axpy_point(const double* x0, const double* dir, const double* step, int64_t n, double* x_out,
-                             hipStream_t s);
+// The rest of a batch after its energy kernels (ls_f: ncand rows of n_elem
+// values): energy sums, the products a1.b1 and a2.b2 (use_dots), the Armijo
+// decision and, when a candidate is accepted, x_out = x0 + step dir (same
+// rounding as the line-search energy kernel).  partials: (kMaxTrials + 2) *
+// kReduceBlocks doubles.
+hipError_t launch_ls_finish(const LineSearchBatch& b, const double* ls_f, int64_t n_elem, int64_t stride,
+                            double* partials, const double* a1, const double* b1, const double* a2, const double* b2,
+                            int64_t n, const double* x0, const double* dir, double* x_out, hipStream_t s);
 
 // dot(a, b) -> out (deterministic)
 hipError_t launch_dot(const double* a, const double* b, int64_t n, double* partials, double* out, hipStream_t s);
@@ -220,6 +256,7 @@ struct PcgSystem
     double *Dinv = nullptr, *x = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *s = nullptr;
     double* parts = nullptr;            // pcg_parts_size(Gs, Gv) partial sums
     PcgScalars* sc = nullptr;
+    PcgReport* host = nullptr;          // pinned
     // reduced basis (CG on the free variables only, the reduced basis of
     // newton_direction_reduced_basis, NewtonDirection.hh:76-105, for a basis B
     // that selects variables): mask in handle order (null: every variable
@@ -233,7 +270,8 @@ struct PcgSystem
     const int32_t* agg_ptr = nullptr;   // [n_agg + 1] entries of each aggregate
     const double* dvec = nullptr;       // [nh * d]
     const double* Ainv = nullptr;       // [nc * nc] inverse Galerkin matrix (symmetric, both triangles)
-    const float* Ainv32 = nullptr;      // [nc * nc] its FP32 copy for the CG iterations (launch_coarse_to32), or null
+    const float* Ainv32 = nullptr;      // [nc * nc] its FP32 copy
+    const int* coarse_mode = nullptr;   // device: which of them the iterations read (launch_coarse_mode)
     double* rpart = nullptr;            // [ppa * nc] restricted residual, one row per part of an aggregate
     double* cparts = nullptr;           // [2 * n_agg] partials of r_c . A_c^-1 r_c, slot k & 1
     // small systems: z = A^-1 r with A = w I + H inverted densely (Ainv, handle
@@ -275,11 +313,15 @@ hipError_t launch_shift_diagonal(int64_t n, double* A, double rel, hipStream_t s
 // *out = ||A||_inf = max_i sum_j |A_ij| of the n x n matrix A (rowsum: n
 // doubles of work space); fixed-order sums.
 hipError_t launch_abs_rowmax(int64_t n, const double* A, double* rowsum, double* out, hipStream_t s);
-// A32 = fl32(A + delta I).  With delta = 2^-23 ||A||_inf the rounding error E
-// has ||E||_2 <= ||E||_inf <= 2^-24 (||A||_inf + delta) < delta, so for a
-// symmetric positive definite A the difference A32 - A = delta I + E is
-// positive definite and so is A32.
-hipError_t launch_coarse_to32(int64_t n, const double* A, double delta, float* A32, hipStream_t s);
+// After the inversion: norms[1] = ||A^-1||_inf, and from norms[0] = ||A||_inf
+// and info the correction the CG iterations apply, in mode (device) and
+// mode_host (pinned): 0 none, 1 the FP64 inverse, 2 the FP32 copy A32 =
+// fl32(A^-1 + delta I) (written then), when 2^-22 ||A|| ||A^-1|| <= change.
+// With delta = 2^-23 ||A^-1||_inf the rounding error E has ||E||_2 <= ||E||_inf
+// <= 2^-24 (||A^-1||_inf + delta) < delta, so delta I + E is positive definite
+// and so is A32.
+hipError_t launch_coarse_mode(int64_t n, const double* Ainv, double* rowsum, double* norms, const int* info,
+                              double change, int* mode, int* mode_host, float* A32, hipStream_t s);
 
 // The solver's copy of H: the n_sym blocks of its lower triangle in solver
 // order (diagonal included), d*d contiguous row-major values each; place: two

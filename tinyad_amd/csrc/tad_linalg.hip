@@ -136,18 +136,93 @@ hipError_t launch_fill(double* p, int64_t n, double v, hipStream_t s)
     return hipGetLastError();
 }
 
+// xo = x0 + step[0] * dir where a step was accepted (accepted[0] >= 0)
 __global__ void k_axpy_point(const double* __restrict__ x0, const double* __restrict__ dir,
-                             const double* __restrict__ step, int64_t n, double* __restrict__ xo)
+                             const double* __restrict__ step, const int* __restrict__ accepted, int64_t n,
+                             double* __restrict__ xo)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (accepted[0] < 0) return;
     if (i < n) xo[i] = fma(step[0], dir[i], x0[i]);
 }
 
-hipError_t launch_axpy_point(const double* x0, const double* dir, const double* step, int64_t n, double* x_out,
-                             hipStream_t s)
+// first-stage sums of two dot products (row blockIdx.y), as k_dot_stage1
+__global__ __launch_bounds__(kBlock) void k_dot2_stage1(const double* __restrict__ a1, const double* __restrict__ b1,
+                                                        const double* __restrict__ a2, const double* __restrict__ b2,
+                                                        int64_t n, double* __restrict__ partials)
 {
-    if (n == 0) return hipSuccess;
-    k_axpy_point<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(x0, dir, step, n, x_out);
+    __shared__ double sh[kBlock];
+    const double* __restrict__ a = blockIdx.y ? a2 : a1;
+    const double* __restrict__ b = blockIdx.y ? b2 : b1;
+    const int64_t chunk = (n + kReduceBlocks - 1) / kReduceBlocks;
+    const int64_t lo = (int64_t)blockIdx.x * chunk;
+    const int64_t hi = lo + chunk < n ? lo + chunk : n;
+    double acc = 0.0;
+    for (int64_t i = lo + threadIdx.x; i < hi; i += kBlock) acc += a[i] * b[i];
+    const double s = block_sum(acc, sh);
+    if (threadIdx.x == 0) partials[blockIdx.y * kReduceBlocks + blockIdx.x] = s;
+}
+
+// The end of one batch of line-search trials, one block: the candidates'
+// energies and (use_dots) the two dot products from their partials, one wave
+// per row with the sums of k_sum_stage2 bit for bit, then the first candidate
+// in order that satisfies the Armijo condition (LineSearch.hh:49-58), or -1,
+// or -2 at a NaN energy before one is accepted.  Its step goes to the device
+// for k_axpy_point, everything to pinned memory for the host.
+__global__ __launch_bounds__(kBlock) void k_ls_finish(LineSearchBatch a)
+{
+    static_assert(kReduceBlocks == kBlock && kBlock == 256, "four partials per lane");
+    __shared__ double tot[kMaxTrials + 2];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int rows = a.ncand + (a.use_dots ? 2 : 0);
+    for (int r = wv; r < rows; r += kBlock / 64)
+    {
+        const double* __restrict__ p = r < a.ncand ? a.partials + r * kReduceBlocks
+                                                   : a.dot_partials + (r - a.ncand) * kReduceBlocks;
+        double v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = 0.0 + p[lane + 64 * q];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] += __shfl_xor(v[q], off, 64);
+        if (lane == 0) tot[r] = ((v[0] + v[1]) + v[2]) + v[3];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const double dg = a.use_dots ? a.dir_scale * tot[a.ncand] : a.dir_dot_g;
+    int acc = -1;
+    for (int c = 0; c < a.ncand && acc == -1; ++c)
+    {
+        if (tot[c] != tot[c]) acc = -2;
+        else if (tot[c] <= a.f + a.armijo * a.sval[c] * dg) acc = c;
+    }
+    a.step_out[0] = acc >= 0 ? a.step[acc] : 0.0;
+    a.accepted_out[0] = acc;
+    for (int c = 0; c < a.ncand; ++c) a.host->f[c] = tot[c];
+    if (a.use_dots)
+    {
+        a.host->dir_dot = tot[a.ncand];
+        a.host->dot2 = tot[a.ncand + 1];
+    }
+    a.host->accepted = acc;
+}
+
+hipError_t launch_ls_finish(const LineSearchBatch& b, const double* ls_f, int64_t n_elem, int64_t stride,
+                            double* partials, const double* a1, const double* b1, const double* a2, const double* b2,
+                            int64_t n, const double* x0, const double* dir, double* x_out, hipStream_t s)
+{
+    LineSearchBatch a = b;
+    a.partials = partials;
+    a.dot_partials = partials + kMaxTrials * kReduceBlocks;
+    k_sum_stage1<<<dim3(kReduceBlocks, a.ncand), kBlock, 0, s>>>(ls_f, n_elem, stride, partials);
+    if (a.use_dots)
+        k_dot2_stage1<<<dim3(kReduceBlocks, 2), kBlock, 0, s>>>(a1, b1, a2, b2, n,
+                                                                partials + kMaxTrials * kReduceBlocks);
+    k_ls_finish<<<1, kBlock, 0, s>>>(a);
+    if (n > 0)
+        k_axpy_point<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(x0, dir, a.step_out, a.accepted_out, n,
+                                                                              x_out);
     return hipGetLastError();
 }
 
@@ -666,6 +741,23 @@ __global__ __launch_bounds__(kBlock) void k_sym_pack(int64_t n_sym, const int2* 
     Hs[id] = H[(int64_t)pl.x + (int64_t)i * (pl.y >> 2) + j];
 }
 
+// Progress and result of a solve in pinned host memory: the host launches only
+// a few iterations ahead of it and never waits for the stream.  Plain
+// system-scope stores, the state after the others have been acknowledged: a
+// release would write back the XCD's L2 in every iteration.
+__device__ __forceinline__ void report(PcgReport* h, double rr, double bb, int k, int breakdown, bool end)
+{
+    if (end)
+    {
+        __hip_atomic_store(&h->rr, rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&h->bb, bb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&h->iters, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&h->breakdown, breakdown, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __hip_atomic_store(&h->state, end ? -1 : k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // sol = x in handle order (solver entry i belongs to handle perm[i])
 template <int D>
 __device__ __forceinline__ void unpermute(int64_t nh, const int32_t* __restrict__ perm, const double* __restrict__ x,
@@ -786,13 +878,12 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sym(PcgSystem a, int Gs, int Gv
     if (flag != 0 && flag != k + 1) return;
     const double rr = racc[0];
     const double bb = k == 0 ? rr : sc->bb;
-    const bool stop = rr <= a.tol2 * bb || k >= a.max_iters;
+    const bool stop = !(rr > a.tol2 * bb) || k >= a.max_iters;  // (a NaN residual stops too)
     if (blockIdx.x == 0 && threadIdx.x == 0)
     {
         if (k == 0) sc->bb = bb;
-        sc->rr = rr;
-        sc->iters = k;
         if (stop) sc->done = k + 1;
+        report(a.host, rr, bb, k, 0, stop);
     }
     if (stop)
     {
@@ -955,9 +1046,7 @@ __global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(PcgSystem a, int G
         if (lo < hi) load(lo);
         if (blk == 0 && t == 0)
         {
-            sc->iters = 0;
             sc->done = 0;
-            sc->breakdown = 0;
             sc->k = 0;
         }
     }
@@ -1002,9 +1091,8 @@ __global__ __launch_bounds__(kUpdVerts * D) void k_pcg_update(PcgSystem a, int G
             // not positive definite along z: the same decision in every block
             if (blk == 0 && t == 0)
             {
-                sc->breakdown = 1;
                 sc->done = -1;
-                sc->iters = k;
+                report(a.host, 0.0, 0.0, k, 1, true);
             }
             return;
         }
@@ -1301,8 +1389,11 @@ __global__ __launch_bounds__(kBlock) void k_shift_diagonal(int64_t n, double* __
 // aggregates, per CG iteration: 512 and 256 lanes alike, 1,024 2 us slower.
 constexpr int kCoarseBlock = 512;
 
-template <int D, int KC, class TA>
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem a, const TA* __restrict__ Ainv, int k,
+//
+// a.coarse_mode: 2 reads the FP32 copy, 1 the FP64 inverse, 0 no correction (z
+// stays D^-1 r and r_c . y_c is 0); only the inverse's loads wait for it.
+template <int D, int KC>
+__global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem a, int k,
                                                                        const int* __restrict__ kdev)
 {
     constexpr int NW = kCoarseBlock / 64;
@@ -1311,9 +1402,9 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
     __shared__ int flag;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int done_v = t == 0 ? a.sc->done : 0;
+    const int mode = a.coarse_mode[0];
     const int slot = (kdev ? *kdev : k) & 1;
     const int64_t ag = blockIdx.x, nc = a.nc;
-    const TA* __restrict__ col = Ainv + ag * KC * nc;
     const double* __restrict__ rpart = a.rpart;
     const int ppa = a.ppa;
     auto rc = [&](int64_t j) {
@@ -1324,17 +1415,6 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
         for (int p = 4; p < ppa; ++p) e += rpart[p * nc + j];
         return e;
     };
-    double acc[KC];
-#pragma unroll
-    for (int c = 0; c < KC; ++c) acc[c] = 0.0;
-    int64_t j = t;
-    if (j < nc)
-    {
-        const double rj = rc(j);
-#pragma unroll
-        for (int c = 0; c < KC; ++c) acc[c] = (double)col[c * nc + j] * rj;
-    }
-    const double rown = t < KC ? rc(ag * KC + t) : 0.0;
     // this thread's first member
     const int64_t m0 = a.agg_ptr[ag], m1 = a.agg_ptr[ag + 1];
     double zv[D], dv[D];
@@ -1346,16 +1426,35 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
             dv[i] = KC > D ? a.dvec[v * D + i] : 0.0;
         }
     };
+    const double r0 = t < nc ? rc(t) : 0.0;
+    const double rown = t < KC ? rc(ag * KC + t) : 0.0;
     if (m0 + t < m1) member(m0 + t);
+    double acc[KC];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) acc[c] = 0.0;
+    auto column = [&](const auto* __restrict__ col, int64_t j, double rj) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) acc[c] += (double)col[c * nc + j] * rj;
+    };
+    const float* __restrict__ col32 = a.Ainv32 + ag * KC * nc;
+    const double* __restrict__ col64 = a.Ainv + ag * KC * nc;
+    if (t < nc)
+    {
+        if (mode == 2) column(col32, t, r0);
+        else column(col64, t, r0);
+    }
     if (t == 0) flag = done_v;
     __syncthreads();
     if (flag) return;
-    for (j += kCoarseBlock; j < nc; j += kCoarseBlock)
+    if (mode == 0)
     {
-        const double rj = rc(j);
-#pragma unroll
-        for (int c = 0; c < KC; ++c) acc[c] += (double)col[c * nc + j] * rj;
+        if (t == 0) a.cparts[slot * a.n_agg + ag] = 0.0;
+        return;
     }
+    if (mode == 2)
+        for (int64_t j = t + kCoarseBlock; j < nc; j += kCoarseBlock) column(col32, j, rc(j));
+    else
+        for (int64_t j = t + kCoarseBlock; j < nc; j += kCoarseBlock) column(col64, j, rc(j));
     wave_sum<KC>(acc);
     if (lane == 0)
     {
@@ -1397,168 +1496,6 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
             a.z[v * D + i] = e;
         }
     }
-}
-
-hipError_t launch_coarse_dvec(int d, int64_t nh, const double* x, const int32_t* agg_of, const int32_t* agg_ptr,
-                              const int32_t* perm, double* dvec_h, double* dvec, hipStream_t s)
-{
-    if (nh == 0) return hipSuccess;
-    const unsigned g = (unsigned)((nh + kBlock - 1) / kBlock);
-    if (d == 1) k_coarse_dvec<1><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
-    else if (d == 2) k_coarse_dvec<2><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
-    else k_coarse_dvec<3><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
-    return hipGetLastError();
-}
-
-template <int D, int KC>
-static void galerkin_t(int64_t n_pairs, int64_t n_gchunks, const int64_t* gchunk_ptr, const int32_t* pair_chunk,
-                       const int32_t* pair_blocks, const int32_t* pair_ab, const int32_t* block_row,
-                       const int32_t* brow_ptr, const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
-                       const double* dvec_h, const unsigned char* free_vars, int64_t nc, double* gpart, double* Ac,
-                       hipStream_t s)
-{
-    const unsigned g1 = (unsigned)((n_gchunks * 64 + kBlock - 1) / kBlock);
-    k_coarse_galerkin_chunk<D, KC><<<g1, kBlock, 0, s>>>(n_gchunks, gchunk_ptr, pair_blocks, block_row, brow_ptr,
-                                                          bcol, row_ptr, H, w, dvec_h, free_vars, gpart);
-    const unsigned g2 = (unsigned)((n_pairs * KC * KC + kBlock - 1) / kBlock);
-    k_coarse_galerkin_pairs<KC><<<g2, kBlock, 0, s>>>(n_pairs, pair_chunk, pair_ab, gpart, nc, Ac);
-}
-
-hipError_t launch_coarse_galerkin(int d, int kc, int64_t nc, int64_t n_pairs, int64_t n_gchunks,
-                                  const int64_t* gchunk_ptr, const int32_t* pair_chunk, const int32_t* pair_blocks,
-                                  const int32_t* pair_ab, const int32_t* block_row, const int32_t* brow_ptr,
-                                  const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
-                                  const double* dvec_h, const unsigned char* free_vars, double* gpart, double* Ac,
-                                  hipStream_t s)
-{
-    if (n_pairs == 0) return hipSuccess;
-#define TAD_GALERKIN(DD, KK) galerkin_t<DD, KK>(n_pairs, n_gchunks, gchunk_ptr, pair_chunk, pair_blocks, pair_ab, \
-                                                 block_row, brow_ptr, bcol, row_ptr, H, w, dvec_h, free_vars, nc, \
-                                                 gpart, Ac, s)
-    if (d == 3 && kc == 6) TAD_GALERKIN(3, 6);
-    else if (d == 3 && kc == 3) TAD_GALERKIN(3, 3);
-    else if (d == 2 && kc == 3) TAD_GALERKIN(2, 3);
-    else if (d == 2 && kc == 2) TAD_GALERKIN(2, 2);
-    else if (d == 1 && kc == 1) TAD_GALERKIN(1, 1);
-    else return hipErrorInvalidValue;
-#undef TAD_GALERKIN
-    return hipGetLastError();
-}
-
-hipError_t launch_shift_diagonal(int64_t n, double* A, double rel, hipStream_t s)
-{
-    if (n == 0) return hipSuccess;
-    k_shift_diagonal<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, A, rel);
-    return hipGetLastError();
-}
-
-// |A| row sums, one wave per row: lane-strided partial sums, then a fixed
-// wave tree; k_rowmax then takes their maximum (||A||_inf).
-__global__ __launch_bounds__(kBlock) void k_abs_rowsum(int64_t n, const double* __restrict__ A,
-                                                       double* __restrict__ rowsum)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (i >= n) return;
-    double t = 0.0;
-    for (int64_t j = lane; j < n; j += 64) t += fabs(A[i * n + j]);
-    wave_sum<1>(&t);
-    if (lane == 0) rowsum[i] = t;
-}
-
-__global__ __launch_bounds__(kBlock) void k_rowmax(int64_t n, const double* __restrict__ rowsum,
-                                                   double* __restrict__ out)
-{
-    __shared__ double sh[kBlock];
-    double m = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += kBlock) m = fmax(m, rowsum[i]);
-    sh[threadIdx.x] = m;
-    __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1)
-    {
-        if ((int)threadIdx.x < off) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + off]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = sh[0];
-}
-
-__global__ __launch_bounds__(kBlock) void k_coarse_to32(int64_t n, const double* __restrict__ A, double delta,
-                                                        float* __restrict__ A32)
-{
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n * n) return;
-    const int64_t i = id / n, j = id - i * n;
-    A32[id] = (float)(A[id] + (i == j ? delta : 0.0));
-}
-
-hipError_t launch_abs_rowmax(int64_t n, const double* A, double* rowsum, double* out, hipStream_t s)
-{
-    if (n == 0) return hipSuccess;
-    k_abs_rowsum<<<(unsigned)((n * 64 + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, A, rowsum);
-    k_rowmax<<<1, kBlock, 0, s>>>(n, rowsum, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_coarse_to32(int64_t n, const double* A, double delta, float* A32, hipStream_t s)
-{
-    if (n == 0) return hipSuccess;
-    k_coarse_to32<<<(unsigned)((n * n + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, A, delta, A32);
-    return hipGetLastError();
-}
-
-constexpr int kSpmvLanes = 8;
-
-int pcg_spmv_groups(int64_t nh)
-{
-    // SpMV: kSpmvLanes lanes per block row, at most 1,024 workgroups (60^3
-    // tet cube, 227K block rows: 8 lanes and 1,024 workgroups 40.7 us per
-    // product against 42.1 with 768, 49.4 with 512, 43.1 with 1,536 and 44.8
-    // with 2,048; 16 lanes with 2,048 workgroups 47.3, 4 lanes with 1,536
-    // 50.1), a multiple of 8 (the XCDs) from 8 on
-    const int64_t rows_per_block = kBlock / kSpmvLanes;
-    const int64_t gs = std::max<int64_t>(1, std::min<int64_t>((nh + rows_per_block - 1) / rows_per_block, 1024));
-    return (int)(gs < 8 ? gs : (gs + 7) / 8 * 8);
-}
-
-int64_t pcg_parts_size(int64_t Gs, int64_t Gv) { return Gs + 4 * Gv; }
-
-hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* place, const double* H, double* sym_H, hipStream_t s)
-{
-    if (n_sym == 0) return hipSuccess;
-    const unsigned grid = (unsigned)((n_sym * d * d + kBlock - 1) / kBlock);
-    const int2* pl = reinterpret_cast<const int2*>(place);
-    if (d == 1) k_sym_pack<1><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
-    else if (d == 2) k_sym_pack<2><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
-    else k_sym_pack<3><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
-    return hipGetLastError();
-}
-
-template <int D>
-static void spmv_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
-{
-    if (a.Gs % 8 == 0) k_spmv_sym<D, kSpmvLanes, true><<<a.Gs, kBlock, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
-    else k_spmv_sym<D, kSpmvLanes, false><<<a.Gs, kBlock, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
-}
-
-template <int D, int KC>
-static void update_t(const PcgSystem& a, int k, const int* kdev, bool init, hipStream_t s)
-{
-    if (init) k_pcg_update<D, KC, true><<<a.Gv, kUpdVerts * D, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
-    else k_pcg_update<D, KC, false><<<a.Gv, kUpdVerts * D, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
-}
-
-static hipError_t update_any(int d, const PcgSystem& a, int k, const int* kdev, bool init, hipStream_t s)
-{
-    if (d == 3 && a.kc == 6) update_t<3, 6>(a, k, kdev, init, s);
-    else if (d == 3 && a.kc == 3) update_t<3, 3>(a, k, kdev, init, s);
-    else if (d == 3 && a.kc == 0) update_t<3, 0>(a, k, kdev, init, s);
-    else if (d == 2 && a.kc == 3) update_t<2, 3>(a, k, kdev, init, s);
-    else if (d == 2 && a.kc == 2) update_t<2, 2>(a, k, kdev, init, s);
-    else if (d == 2 && a.kc == 0) update_t<2, 0>(a, k, kdev, init, s);
-    else if (d == 1 && a.kc == 1) update_t<1, 1>(a, k, kdev, init, s);
-    else if (d == 1 && a.kc == 0) update_t<1, 0>(a, k, kdev, init, s);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
 }
 
 // A small system's dense preconditioner: A = w I + H in FP64 (column-major
@@ -1658,10 +1595,7 @@ int64_t dense_apply_groups(int64_t n) { return (n + kBlock / 64 - 1) / (kBlock /
 template <int D, int KC>
 static void coarse_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
 {
-    if (a.Ainv32)
-        k_coarse_apply_prolong<D, KC, float><<<(unsigned)a.n_agg, kCoarseBlock, 0, s>>>(a, a.Ainv32, k, kdev);
-    else
-        k_coarse_apply_prolong<D, KC, double><<<(unsigned)a.n_agg, kCoarseBlock, 0, s>>>(a, a.Ainv, k, kdev);
+    k_coarse_apply_prolong<D, KC><<<(unsigned)a.n_agg, kCoarseBlock, 0, s>>>(a, k, kdev);
 }
 
 // z += P A_c^-1 P^T r with the restricted residual's parts of the last update,
