@@ -1389,22 +1389,16 @@ __global__ __launch_bounds__(kBlock) void k_shift_diagonal(int64_t n, double* __
 // aggregates, per CG iteration: 512 and 256 lanes alike, 1,024 2 us slower.
 constexpr int kCoarseBlock = 512;
 
-//
-// a.coarse_mode: 2 reads the FP32 copy, 1 the FP64 inverse, 0 no correction (z
-// stays D^-1 r and r_c . y_c is 0); only the inverse's loads wait for it.
-template <int D, int KC>
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem a, int k,
-                                                                       const int* __restrict__ kdev)
+template <int D, int KC, class TA>
+__device__ __forceinline__ void coarse_apply(const PcgSystem& a, const TA* __restrict__ Ainv, int slot, int done_v)
 {
     constexpr int NW = kCoarseBlock / 64;
     __shared__ double wpart[NW][KC];
     __shared__ double y[KC], ry[KC];
     __shared__ int flag;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int done_v = t == 0 ? a.sc->done : 0;
-    const int mode = a.coarse_mode[0];
-    const int slot = (kdev ? *kdev : k) & 1;
     const int64_t ag = blockIdx.x, nc = a.nc;
+    const TA* __restrict__ col = Ainv + ag * KC * nc;
     const double* __restrict__ rpart = a.rpart;
     const int ppa = a.ppa;
     auto rc = [&](int64_t j) {
@@ -1415,6 +1409,17 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
         for (int p = 4; p < ppa; ++p) e += rpart[p * nc + j];
         return e;
     };
+    double acc[KC];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) acc[c] = 0.0;
+    int64_t j = t;
+    if (j < nc)
+    {
+        const double rj = rc(j);
+#pragma unroll
+        for (int c = 0; c < KC; ++c) acc[c] = (double)col[c * nc + j] * rj;
+    }
+    const double rown = t < KC ? rc(ag * KC + t) : 0.0;
     // this thread's first member
     const int64_t m0 = a.agg_ptr[ag], m1 = a.agg_ptr[ag + 1];
     double zv[D], dv[D];
@@ -1426,35 +1431,16 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
             dv[i] = KC > D ? a.dvec[v * D + i] : 0.0;
         }
     };
-    const double r0 = t < nc ? rc(t) : 0.0;
-    const double rown = t < KC ? rc(ag * KC + t) : 0.0;
     if (m0 + t < m1) member(m0 + t);
-    double acc[KC];
-#pragma unroll
-    for (int c = 0; c < KC; ++c) acc[c] = 0.0;
-    auto column = [&](const auto* __restrict__ col, int64_t j, double rj) {
-#pragma unroll
-        for (int c = 0; c < KC; ++c) acc[c] += (double)col[c * nc + j] * rj;
-    };
-    const float* __restrict__ col32 = a.Ainv32 + ag * KC * nc;
-    const double* __restrict__ col64 = a.Ainv + ag * KC * nc;
-    if (t < nc)
-    {
-        if (mode == 2) column(col32, t, r0);
-        else column(col64, t, r0);
-    }
     if (t == 0) flag = done_v;
     __syncthreads();
     if (flag) return;
-    if (mode == 0)
+    for (j += kCoarseBlock; j < nc; j += kCoarseBlock)
     {
-        if (t == 0) a.cparts[slot * a.n_agg + ag] = 0.0;
-        return;
+        const double rj = rc(j);
+#pragma unroll
+        for (int c = 0; c < KC; ++c) acc[c] += (double)col[c * nc + j] * rj;
     }
-    if (mode == 2)
-        for (int64_t j = t + kCoarseBlock; j < nc; j += kCoarseBlock) column(col32, j, rc(j));
-    else
-        for (int64_t j = t + kCoarseBlock; j < nc; j += kCoarseBlock) column(col64, j, rc(j));
     wave_sum<KC>(acc);
     if (lane == 0)
     {
@@ -1496,6 +1482,204 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem
             a.z[v * D + i] = e;
         }
     }
+}
+
+hipError_t launch_coarse_dvec(int d, int64_t nh, const double* x, const int32_t* agg_of, const int32_t* agg_ptr,
+                              const int32_t* perm, double* dvec_h, double* dvec, hipStream_t s)
+{
+    if (nh == 0) return hipSuccess;
+    const unsigned g = (unsigned)((nh + kBlock - 1) / kBlock);
+    if (d == 1) k_coarse_dvec<1><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
+    else if (d == 2) k_coarse_dvec<2><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
+    else k_coarse_dvec<3><<<g, kBlock, 0, s>>>(nh, x, agg_of, agg_ptr, perm, dvec_h, dvec);
+    return hipGetLastError();
+}
+
+template <int D, int KC>
+static void galerkin_t(int64_t n_pairs, int64_t n_gchunks, const int64_t* gchunk_ptr, const int32_t* pair_chunk,
+                       const int32_t* pair_blocks, const int32_t* pair_ab, const int32_t* block_row,
+                       const int32_t* brow_ptr, const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
+                       const double* dvec_h, const unsigned char* free_vars, int64_t nc, double* gpart, double* Ac,
+                       hipStream_t s)
+{
+    const unsigned g1 = (unsigned)((n_gchunks * 64 + kBlock - 1) / kBlock);
+    k_coarse_galerkin_chunk<D, KC><<<g1, kBlock, 0, s>>>(n_gchunks, gchunk_ptr, pair_blocks, block_row, brow_ptr,
+                                                          bcol, row_ptr, H, w, dvec_h, free_vars, gpart);
+    const unsigned g2 = (unsigned)((n_pairs * KC * KC + kBlock - 1) / kBlock);
+    k_coarse_galerkin_pairs<KC><<<g2, kBlock, 0, s>>>(n_pairs, pair_chunk, pair_ab, gpart, nc, Ac);
+}
+
+hipError_t launch_coarse_galerkin(int d, int kc, int64_t nc, int64_t n_pairs, int64_t n_gchunks,
+                                  const int64_t* gchunk_ptr, const int32_t* pair_chunk, const int32_t* pair_blocks,
+                                  const int32_t* pair_ab, const int32_t* block_row, const int32_t* brow_ptr,
+                                  const int32_t* bcol, const int32_t* row_ptr, const double* H, double w,
+                                  const double* dvec_h, const unsigned char* free_vars, double* gpart, double* Ac,
+                                  hipStream_t s)
+{
+    if (n_pairs == 0) return hipSuccess;
+#define TAD_GALERKIN(DD, KK) galerkin_t<DD, KK>(n_pairs, n_gchunks, gchunk_ptr, pair_chunk, pair_blocks, pair_ab, \
+                                                 block_row, brow_ptr, bcol, row_ptr, H, w, dvec_h, free_vars, nc, \
+                                                 gpart, Ac, s)
+    if (d == 3 && kc == 6) TAD_GALERKIN(3, 6);
+    else if (d == 3 && kc == 3) TAD_GALERKIN(3, 3);
+    else if (d == 2 && kc == 3) TAD_GALERKIN(2, 3);
+    else if (d == 2 && kc == 2) TAD_GALERKIN(2, 2);
+    else if (d == 1 && kc == 1) TAD_GALERKIN(1, 1);
+    else return hipErrorInvalidValue;
+#undef TAD_GALERKIN
+    return hipGetLastError();
+}
+
+hipError_t launch_shift_diagonal(int64_t n, double* A, double rel, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    k_shift_diagonal<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, A, rel);
+    return hipGetLastError();
+}
+
+// |A| row sums, one wave per row: lane-strided partial sums, then a fixed
+// wave tree; k_rowmax then takes their maximum (||A||_inf).
+__global__ __launch_bounds__(kBlock) void k_abs_rowsum(int64_t n, const double* __restrict__ A,
+                                                       double* __restrict__ rowsum)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (i >= n) return;
+    double t = 0.0;
+    for (int64_t j = lane; j < n; j += 64) t += fabs(A[i * n + j]);
+    wave_sum<1>(&t);
+    if (lane == 0) rowsum[i] = t;
+}
+
+// out[0] = max of the row sums.  With `mode` (the second norm, of A^-1): the
+// coarse correction the CG iterations apply, decided here so that the host
+// need not wait for it: 0 none (the sweeps met a pivot that was not positive:
+// A_c is not positive definite at working precision), 2 the FP32 copy, where
+// 2^-22 kappa_inf <= `change` bounds the relative change of the correction
+// by the copy's diagonal shift (2^-23 ||A^-1||_inf, small against the smallest
+// eigenvalue of A^-1, >= 1 / ||A||_inf), 1 the FP64 inverse otherwise.
+__global__ __launch_bounds__(kBlock) void k_rowmax(int64_t n, const double* __restrict__ rowsum,
+                                                   double* __restrict__ out, const double* __restrict__ norm_a,
+                                                   const int* __restrict__ info, double change, int* __restrict__ mode,
+                                                   int* __restrict__ mode_host)
+{
+    __shared__ double sh[kBlock];
+    double m = 0.0;
+    for (int64_t i = threadIdx.x; i < n; i += kBlock) m = fmax(m, rowsum[i]);
+    sh[threadIdx.x] = m;
+    __syncthreads();
+    for (int off = kBlock / 2; off > 0; off >>= 1)
+    {
+        if ((int)threadIdx.x < off) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + off]);
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    out[0] = sh[0];
+    if (!mode) return;
+    const double kappa = norm_a[0] * sh[0];
+    const int v = info[0] != 0 ? 0 : (kappa < 1.0 / 0.0 && ldexp(kappa, -22) <= change) ? 2 : 1;
+    mode[0] = v;
+    mode_host[0] = v;
+}
+
+// A32 = fl32(A + delta I), delta = 2^-23 norm[0], when the iterations read it
+__global__ __launch_bounds__(kBlock) void k_coarse_to32(int64_t n, const double* __restrict__ A,
+                                                        const double* __restrict__ norm, const int* __restrict__ mode,
+                                                        float* __restrict__ A32)
+{
+    if (mode[0] != 2) return;
+    const double delta = ldexp(norm[0], -23);
+    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= n * n) return;
+    const int64_t i = id / n, j = id - i * n;
+    A32[id] = (float)(A[id] + (i == j ? delta : 0.0));
+}
+
+hipError_t launch_abs_rowmax(int64_t n, const double* A, double* rowsum, double* out, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    k_abs_rowsum<<<(unsigned)((n * 64 + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, A, rowsum);
+    k_rowmax<<<1, kBlock, 0, s>>>(n, rowsum, out, nullptr, nullptr, 0.0, nullptr, nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_coarse_mode(int64_t n, const double* Ainv, double* rowsum, double* norms, const int* info,
+                              double change, int* mode, int* mode_host, float* A32, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    k_abs_rowsum<<<(unsigned)((n * 64 + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, Ainv, rowsum);
+    k_rowmax<<<1, kBlock, 0, s>>>(n, rowsum, norms + 1, norms, info, change, mode, mode_host);
+    k_coarse_to32<<<(unsigned)((n * n + kBlock - 1) / kBlock), kBlock, 0, s>>>(n, Ainv, norms + 1, mode, A32);
+    return hipGetLastError();
+}
+
+constexpr int kSpmvLanes = 8;
+
+int pcg_spmv_groups(int64_t nh)
+{
+    // SpMV: kSpmvLanes lanes per block row, at most 1,024 workgroups (60^3
+    // tet cube, 227K block rows: 8 lanes and 1,024 workgroups 40.7 us per
+    // product against 42.1 with 768, 49.4 with 512, 43.1 with 1,536 and 44.8
+    // with 2,048; 16 lanes with 2,048 workgroups 47.3, 4 lanes with 1,536
+    // 50.1), a multiple of 8 (the XCDs) from 8 on
+    const int64_t rows_per_block = kBlock / kSpmvLanes;
+    const int64_t gs = std::max<int64_t>(1, std::min<int64_t>((nh + rows_per_block - 1) / rows_per_block, 1024));
+    return (int)(gs < 8 ? gs : (gs + 7) / 8 * 8);
+}
+
+int64_t pcg_parts_size(int64_t Gs, int64_t Gv) { return Gs + 4 * Gv; }
+
+hipError_t launch_sym_pack(int d, int64_t n_sym, const int32_t* place, const double* H, double* sym_H, hipStream_t s)
+{
+    if (n_sym == 0) return hipSuccess;
+    const unsigned grid = (unsigned)((n_sym * d * d + kBlock - 1) / kBlock);
+    const int2* pl = reinterpret_cast<const int2*>(place);
+    if (d == 1) k_sym_pack<1><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
+    else if (d == 2) k_sym_pack<2><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
+    else k_sym_pack<3><<<grid, kBlock, 0, s>>>(n_sym, pl, H, sym_H);
+    return hipGetLastError();
+}
+
+template <int D>
+static void spmv_t(const PcgSystem& a, int k, const int* kdev, hipStream_t s)
+{
+    if (a.Gs % 8 == 0) k_spmv_sym<D, kSpmvLanes, true><<<a.Gs, kBlock, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+    else k_spmv_sym<D, kSpmvLanes, false><<<a.Gs, kBlock, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+}
+
+template <int D, int KC>
+static void update_t(const PcgSystem& a, int k, const int* kdev, bool init, hipStream_t s)
+{
+    if (init) k_pcg_update<D, KC, true><<<a.Gv, kUpdVerts * D, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+    else k_pcg_update<D, KC, false><<<a.Gv, kUpdVerts * D, 0, s>>>(a, a.Gs, a.Gv, k, kdev);
+}
+
+static hipError_t update_any(int d, const PcgSystem& a, int k, const int* kdev, bool init, hipStream_t s)
+{
+    if (d == 3 && a.kc == 6) update_t<3, 6>(a, k, kdev, init, s);
+    else if (d == 3 && a.kc == 3) update_t<3, 3>(a, k, kdev, init, s);
+    else if (d == 3 && a.kc == 0) update_t<3, 0>(a, k, kdev, init, s);
+    else if (d == 2 && a.kc == 3) update_t<2, 3>(a, k, kdev, init, s);
+    else if (d == 2 && a.kc == 2) update_t<2, 2>(a, k, kdev, init, s);
+    else if (d == 2 && a.kc == 0) update_t<2, 0>(a, k, kdev, init, s);
+    else if (d == 1 && a.kc == 1) update_t<1, 1>(a, k, kdev, init, s);
+    else if (d == 1 && a.kc == 0) update_t<1, 0>(a, k, kdev, init, s);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// a.coarse_mode: 2 the FP32 copy, 1 the FP64 inverse, 0 no correction (z stays
+// D^-1 r and r_c . y_c is 0).
+template <int D, int KC>
+__global__ __launch_bounds__(kCoarseBlock) void k_coarse_apply_prolong(PcgSystem a, int k,
+                                                                       const int* __restrict__ kdev)
+{
+    const int done_v = threadIdx.x == 0 ? a.sc->done : 0;
+    const int slot = (kdev ? *kdev : k) & 1;
+    const int mode = a.coarse_mode[0];
+    if (mode == 2) coarse_apply<D, KC, float>(a, a.Ainv32, slot, done_v);
+    else if (mode == 1) coarse_apply<D, KC, double>(a, a.Ainv, slot, done_v);
+    else if (threadIdx.x == 0) a.cparts[slot * a.n_agg + blockIdx.x] = 0.0;
 }
 
 // A small system's dense preconditioner: A = w I + H in FP64 (column-major
