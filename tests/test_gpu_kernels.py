@@ -167,3 +167,44 @@ def test_assembly_tiles(ctx, d, n, precision):
         np.add.at(ref, (idx[:, :, None], idx[:, None, :]), A)
     # FP64: sums of at most 2,000 terms; mixed: FP32 contributions, FP64 sums
     assert np.abs(out[0][2] - ref).max() <= (1e-12 if precision == "fp64" else 1e-6) * np.abs(ref).max()
+
+
+def tet_states(P, state):
+    rest = P.info["rest"].reshape(-1, 3)
+    rng = np.random.default_rng(5)
+    if state == "rest":            # three eigenvalues 0 to rounding
+        x = rest.copy()
+    elif state == "noise":         # three small ones of either sign, close together
+        x = rest + 1e-4 * P.info["h"] * rng.normal(size=rest.shape)
+    elif state == "compressed":    # three below 0
+        x = 0.9 * rest
+    elif state == "flattened":     # two below 0, one at 0 to rounding
+        x = rest * np.array([1.0, 1.0, 0.8])
+    elif state == "stretched":     # none to clamp
+        x = 1.2 * rest
+    else:                          # some elements inverted (zero Hessian)
+        x = rest + 0.1 * P.info["h"] * rng.normal(size=rest.shape)
+        x[::5] += 1.5 * P.info["h"]
+    return np.ascontiguousarray(x).reshape(-1)
+
+
+# 6, 48, 162 and 384 tets: one short group of 64, a full and a short one, ...
+@pytest.mark.parametrize("state", ["rest", "noise", "compressed", "flattened", "stretched", "inverted"])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_tet_projection_cases(ctx, m, state):
+    """FP64 tets projected through their clamped eigenvalues against the
+    oracle's full eigensolve, also with a level that clamps more than three of
+    them and with absolute values, plain and persistent launches.  Each side's
+    element error is below 30 eps |H_e| (7e-15), a block sums at most 24
+    elements: 24 * 2 * 7e-15 < 1e-12."""
+    import oracle
+    P = configs.twist_cube(m=m)
+    x = tet_states(P, state)
+    fg = tad.ScalarFunction.from_problem(P, ctx)
+    fo = oracle.Function.from_problem(P)
+    for eps in (1e-9, 0.05, -1.0, 0.0):
+        ref = fo.eval_with_hessian_proj(x, eps)[2]
+        for shape in [(0, 0, 0), (64, 8, 1), (256, 1, 0)]:
+            fg.set_launch_shape(0, *shape)
+            f, g, H = fg.eval_with_hessian_proj(x, eps)
+            assert nrel(H.toarray(), ref.toarray()) <= 1e-12, (eps, shape)

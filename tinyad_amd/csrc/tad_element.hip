@@ -49,7 +49,21 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int N, int Dm, class T>
+// The lane's index in its wave and the wave's in its workgroup.  The lane's is
+// formed where it is asked for (the empty statement keeps the compiler from
+// holding it in a register through an element's evaluation), so that nothing
+// of a lane is live from one tile of a persistent kernel to the next.
+__device__ __forceinline__ int wave_lane()
+{
+    unsigned zero = 0;
+    asm volatile("" : "+s"(zero));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64); }
+
+// Prefetch: begin() is called before an element's first block and loads its
+// codes and the group's pass counts at once; else each block loads its own.
+template <int N, int Dm, class T, bool Prefetch>
 struct GroupSink
 {
     T* __restrict__ G;
@@ -58,14 +72,39 @@ struct GroupSink
     const uint8_t* __restrict__ npass;  // this group's passes per block
     T* acc;                             // this wave's accumulators (LDS)
     int64_t e, n;
+    int count, lanes;                   // accumulated values, elements of the group
+    mutable uint32_t code[Prefetch ? n_blocks(N) : 1] = {};
+    mutable int np[Prefetch ? n_blocks(N) : 1] = {};
 
+    // The accumulators' LDS is the lanes' work area until begin<true>() clears
+    // them (the active lanes are the first `lanes` ones).
+    __device__ __forceinline__ T* area() const { return acc + wave_lane(); }
+    template <bool Clear>
+    __device__ __forceinline__ void begin() const
+    {
+        if constexpr (Prefetch)
+        {
+#pragma unroll
+            for (int bi = 0; bi < n_blocks(N); ++bi)
+            {
+                code[bi] = hcode[bi * n + e];
+                np[bi] = npass[bi];
+            }
+        }
+        if constexpr (Clear)
+        {
+            wave_sync();
+            for (int i = wave_lane(); i < count; i += lanes) acc[i] = T(0);
+            wave_sync();
+        }
+    }
     __device__ __forceinline__ void grad(int v, const T* g) const { store_run<Dm>(G + (int64_t)gpos[v * n + e] * Dm, g); }
     // block (v, u), v <= u: added to its group accumulator, transposed to
     // the orientation of the upper CSR block when the code says so
     __device__ __forceinline__ void block(int v, int u, const T* b) const
     {
         const int bi = block_index(N, v, u);
-        const uint32_t c = hcode[bi * n + e];
+        const uint32_t c = Prefetch ? code[bi] : hcode[bi * n + e];
         const int gs = (int)(c & 0xffffu);
         const int pass = (int)((c >> 16) & 0xffu);
         const bool tr = (c >> 31) != 0;
@@ -75,8 +114,8 @@ struct GroupSink
 #pragma unroll
             for (int j = 0; j < Dm; ++j) o[i * Dm + j] = tr ? b[j * Dm + i] : b[i * Dm + j];
         T* a = acc + gs * (Dm * Dm);
-        const int np = npass[bi];
-        for (int p = 0; p < np; ++p)
+        const int passes = Prefetch ? np[bi] : npass[bi];
+        for (int p = 0; p < passes; ++p)
         {
             if (p == pass)
             {
@@ -87,6 +126,32 @@ struct GroupSink
         }
     }
 };
+
+// Whether E's evaluation uses the work area, and the values of LDS a wave has.
+template <class E>
+struct SimplexDim
+{
+    static constexpr int value = 0;
+};
+template <int Dm>
+struct SimplexDim<SymdirElem<Dm>>
+{
+    static constexpr int value = Dm;
+};
+template <class E, class T>
+using GroupSinkOf = GroupSink<E::N, E::D, T, SimplexDim<E>::value != 0>;
+template <class E, class T, int MODE>
+__host__ __device__ constexpr bool group_area()
+{
+    return symdir_few<SimplexDim<E>::value, T, MODE, GroupSinkOf<E, T>>();
+}
+template <class E, class T, int MODE>
+__host__ __device__ constexpr int group_values(int group_max)
+{
+    const int sums = group_max * E::D * E::D;
+    const int area = group_area<E, T, MODE>() ? 64 * reflector_values(E::D * E::D) : 0;
+    return sums > area ? sums : area;
+}
 
 // One group: zero its accumulators, evaluate its elements (those below e1),
 // write its block sums.  Called by all 64 lanes of the wave; `first` is the
@@ -99,12 +164,15 @@ __device__ __forceinline__ void group_body(int64_t first, int64_t e1, int64_t n,
 {
     constexpr int DD = E::D * E::D;
     constexpr int NB = n_blocks(E::N);
-    const int lane = threadIdx.x & 63;
+    const int lane = wave_lane();
     const int64_t q = first / kElemGroup;
     const uint32_t g0 = go.gout_ptr[q];
     const int G = (int)(go.gout_ptr[q + 1] - g0);
-    for (int i = lane; i < G * DD; i += 64) acc[i] = T(0);
-    wave_sync();
+    if constexpr (!group_area<E, T, MODE>())
+    {
+        for (int i = lane; i < G * DD; i += 64) acc[i] = T(0);
+        wave_sync();
+    }
     const int64_t e = first + lane;
     if (e < e1)
     {
@@ -120,14 +188,32 @@ __device__ __forceinline__ void group_body(int64_t first, int64_t e1, int64_t n,
 #pragma unroll
         for (int k = 0; k < E::NP; ++k) p[k] = params[k * n + e];
         bool nf = false;
-        const GroupSink<E::N, E::D, T> out{ o.G, o.gpos, o.hpos, go.gpass + q * NB, acc, e, n };
+        const GroupSinkOf<E, T> out{ o.G, o.gpos, o.hpos, go.gpass + q * NB, acc, e, n,
+                                             G * DD, (int)(e1 - first < 64 ? e1 - first : 64) };
         elem_f[e] = E::template eval<T, MODE>(X, p, T(eps), out, nf);
         if (nf) *err = 1;
     }
     wave_sync();
     // value i of the group's sums: slot block i / DD, entry i % DD (a wave
-    // writes whole blocks with consecutive lanes)
-    for (int i = lane; i < G * DD; i += 64) o.Hc[(int64_t)go.gout[g0 + i / DD] * DD + i % DD] = acc[i];
+    // writes whole blocks with consecutive lanes); the slots of kOut rounds
+    // are fetched together, one wait for memory instead of one per round
+    constexpr int kOut = 8;
+    for (int i0 = wave_lane(); i0 < G * DD; i0 += 64 * kOut)
+    {
+        uint32_t slot[kOut];
+#pragma unroll
+        for (int r = 0; r < kOut; ++r)
+        {
+            const int i = i0 + 64 * r;
+            slot[r] = i < G * DD ? go.gout[g0 + i / DD] : 0u;
+        }
+#pragma unroll
+        for (int r = 0; r < kOut; ++r)
+        {
+            const int i = i0 + 64 * r;
+            if (i < G * DD) o.Hc[(int64_t)slot[r] * DD + i % DD] = acc[i];
+        }
+    }
     wave_sync();
 }
 
@@ -136,9 +222,15 @@ __device__ __forceinline__ void group_body(int64_t first, int64_t e1, int64_t n,
 extern __shared__ double tad_group_lds[];
 
 // Waves per SIMD the grouped kernels are compiled for: FP64 as the plain
-// kernels (2); FP32 3, which holds the pass loops of the grouped sums in 168
-// registers (unconstrained they take 191 and two waves: FP32 tets 0.73 ms
-// instead of 0.52 ms at the 60^3 cube).
+// kernels (2: tets take 252 registers, none spilled); FP32 3, which holds the
+// pass loops of the grouped sums in 168 registers (unconstrained they take 191
+// and two waves: FP32 tets 0.73 ms instead of 0.52 ms at the 60^3 cube).
+// FP64 tets (1,296,000 of the 60^3 cube, evaluation with assembly): with the
+// whole spectrum 1.21 ms, 19,100 vector instructions per wave and 61 % of the
+// issue slots; with the clamped eigenvalues only 9,500 and 0.97 ms, 46 % of
+// the wave's cycles waiting for memory, mostly for one slot or code at a time;
+// with both fetched together 0.84 ms.  (FP32, 45^3 cube: 0.34 -> 0.31 ms;
+// triangles of 256 disks: 0.55 -> 0.48 ms.)
 template <class T>
 struct GroupWaves
 {
@@ -151,8 +243,8 @@ __global__ __launch_bounds__(kBlock, GroupWaves<T>::value) void k_element_range_
     const double* __restrict__ x, double eps, double* __restrict__ elem_f, ElemOut<T> o, GroupOut go,
     int* __restrict__ err)
 {
-    T* acc = reinterpret_cast<T*>(tad_group_lds) + (threadIdx.x / 64) * (go.group_max * E::D * E::D);
-    const int64_t first = e0 + (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63);
+    T* acc = reinterpret_cast<T*>(tad_group_lds) + wave_index() * group_values<E, T, MODE>(go.group_max);
+    const int64_t first = e0 + (int64_t)blockIdx.x * blockDim.x + 64 * wave_index();
     if (first >= e1) return;  // whole wave past the end
     group_body<E, T, MODE>(first, e1, n, conn, params, x, eps, elem_f, o, go, acc, err);
 }
@@ -163,7 +255,7 @@ __global__ __launch_bounds__(BLOCK, GroupWaves<T>::value) void k_element_persist
     const double* __restrict__ x, double eps, double* __restrict__ elem_f, ElemOut<T> o, GroupOut go,
     int* __restrict__ err, int map_xcd)
 {
-    T* acc = reinterpret_cast<T*>(tad_group_lds) + (threadIdx.x / 64) * (go.group_max * E::D * E::D);
+    T* acc = reinterpret_cast<T*>(tad_group_lds) + wave_index() * group_values<E, T, MODE>(go.group_max);
     const int64_t n_tiles = (e1 - e0 + BLOCK - 1) / BLOCK;
     int64_t t1, stride, first_t;
     if (map_xcd)
@@ -183,7 +275,7 @@ __global__ __launch_bounds__(BLOCK, GroupWaves<T>::value) void k_element_persist
     }
     for (int64_t t = first_t; t < t1; t += stride)
     {
-        const int64_t first = e0 + t * BLOCK + (threadIdx.x & ~63);
+        const int64_t first = e0 + t * BLOCK + 64 * wave_index();
         if (first < e1) group_body<E, T, MODE>(first, e1, n, conn, params, x, eps, elem_f, o, go, acc, err);
     }
 }
@@ -261,7 +353,7 @@ static void launch_persistent_grouped(const TermDev& t, const double* x, double 
     const int64_t tiles = (e1 - e0 + BLOCK - 1) / BLOCK;
     int64_t grid = std::min<int64_t>(t.tune_grid, tiles);
     if (t.tune_map == 1) grid = (grid + 7) / 8 * 8;
-    const size_t lds = (size_t)(BLOCK / 64) * go.group_max * E::D * E::D * sizeof(T);
+    const size_t lds = (size_t)(BLOCK / 64) * group_values<E, T, MODE>(go.group_max) * sizeof(T);
     k_element_persistent_grouped<E, T, MODE, BLOCK><<<(unsigned)grid, BLOCK, lds, s>>>(
         e0, e1, t.n_elem, t.conn, t.params, x, eps, ef, o, go, err, t.tune_map);
 }
@@ -284,7 +376,7 @@ static hipError_t launch_grouped(const TermDev& t, const double* x, double eps, 
         }
     }
     const dim3 grid((unsigned)((e1 - e0 + kBlock - 1) / kBlock));
-    const size_t lds = (size_t)(kBlock / 64) * go.group_max * E::D * E::D * sizeof(T);
+    const size_t lds = (size_t)(kBlock / 64) * group_values<E, T, MODE>(go.group_max) * sizeof(T);
     k_element_range_grouped<E, T, MODE><<<grid, kBlock, lds, s>>>(e0, e1, t.n_elem, t.conn, t.params, x, eps, ef, o,
                                                                    go, err);
     return hipGetLastError();

@@ -352,6 +352,24 @@ __device__ __forceinline__ bool deflated_pdd(const T* Km, T eps)
     return ok;
 }
 
+// A sink that wants begin() before an element's first block, and has an LDS
+// work area until begin<true>() (Sink::area()): the lanes of a wave evaluate
+// together and write their blocks after the last of them is projected.
+template <class S, class = void>
+struct sink_area : std::false_type
+{
+};
+template <class S>
+struct sink_area<S, std::void_t<decltype(&S::area)>> : std::true_type
+{
+};
+
+// Tets in FP64 with such a sink are projected through the clamped eigenvalues
+// only; all lanes take one path, an inverted element with J = I in place of
+// its own and its results selected at the end.
+template <int Dm, class T, int MODE, class Sink>
+__host__ __device__ constexpr bool symdir_few() { return Dm == 3 && sizeof(T) == 8 && MODE == MODE_HESS_PROJ && sink_area<Sink>::value; }
+
 // Second-order evaluation of one symmetric-Dirichlet simplex.
 // X: element coordinates (FP64, AoS N x Dm); p: [Mr^-1, w] (FP64).
 // Writes the record (gradient + Hessian blocks) in type T; returns the FP64 energy.
@@ -361,9 +379,11 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
 {
     constexpr int N = Dm + 1;
     constexpr int KJ = Dm * Dm;
+    constexpr bool few = symdir_few<Dm, T, MODE, Sink>();
     const double f = energy_symdir<Dm>(X, p);
+    const bool inverted = !(f < tad_inf());
 
-    if (!(f < tad_inf()))
+    if (!few && inverted)
     {
         // inverted element: +inf energy, zero derivatives; the projection of
         // the zero Hessian is eps I (clamp mode) or 0 (absolute-value mode)
@@ -372,6 +392,7 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
         for (int v = 0; v < N; ++v) out.grad(v, zero);
         if constexpr (MODE >= MODE_HESS)
         {
+            if constexpr (sink_area<Sink>::value) out.template begin<few>();
             const T dg = (MODE == MODE_HESS_PROJ && eps > T(0)) ? eps : T(0);
 #pragma unroll
             for (int v = 0; v < N; ++v)
@@ -404,7 +425,7 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
             double s = 0.0;
 #pragma unroll
             for (int k = 0; k < Dm; ++k) s += Md[i][k] * p[k * Dm + j];
-            J[i * Dm + j] = T(s);
+            J[i * Dm + j] = few && inverted ? T(i == j) : T(s);
         }
     const T w = T(p[KJ]);
     // D (N x Dm): dJ_ij/dX_vi = D_vj
@@ -435,7 +456,7 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
             T s = T(0);
 #pragma unroll
             for (int j = 0; j < Dm; ++j) s += Dmat[v][j] * E.g[i * Dm + j];
-            gv[i] = w * s;
+            gv[i] = few && inverted ? T(0) : w * s;
             nonfinite = nonfinite || !finite_val(gv[i]);
         }
         out.grad(v, gv);
@@ -445,6 +466,7 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
 
     if constexpr (MODE == MODE_HESS)
     {
+        if constexpr (sink_area<Sink>::value) out.template begin<few>();
         symdir_write_hx<Dm, T>(E, Dmat, w, out, nonfinite);
         return f;
     }
@@ -502,7 +524,15 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
         // when the translations are in the kernel of H); it leaves H
         // unprojected.  Only evaluated for eps <= 0, see above.
         const bool pdd = (eps <= T(0)) && deflated_pdd<N, Dm, T>(Km, eps);
-        if (!pdd) project_psd<KJ, T, false>(Km, eps);
+        if constexpr (few)
+        {
+            if (!pdd && !inverted) project_psd_few<KJ>(Km, eps, out.area());
+        }
+        else if (!pdd)
+            project_psd<KJ, T, false>(Km, eps);
+        if constexpr (sink_area<Sink>::value) out.template begin<few>();
+        const T dg = eps > T(0) ? eps : T(0);
+        T nan_sum = T(0);  // stays 0 while all entries are finite
         // H[(v,i),(u,i')] = sum_{a,b} U_va U_ub P[(a,i),(b,i')] + max(eps,0)/N delta_ii'
         const T ct = eps > T(0) ? eps / T(N) : T(0);
         // one vertex row at a time: S1[i][(b,i')] = sum_a U_va P[(a,i),(b,i')]
@@ -543,12 +573,18 @@ __device__ __forceinline__ double symdir_element(const double* X, const double* 
                         for (int b = 0; b < Dm; ++b)
                             if (Helmert<N>::u(u, b) != 0.0)
                                 s += T(Helmert<N>::u(u, b)) * S1[i][b * Dm + ip];
+                        if (few && inverted) s = (v == u && i == ip) ? dg : T(0);
                         blk[i * Dm + ip] = s;
-                        nonfinite = nonfinite || !finite_val(s);
+                        if constexpr (few) nan_sum += s * T(0);
+                        else nonfinite = nonfinite || !finite_val(s);
                     }
+                // (one value to keep instead of the block's entries, which
+                // the compiler held for one test at the end)
+                if constexpr (few) asm volatile("" : "+v"(nan_sum));
                 out.block(v, u, blk);
             }
         }
+        if constexpr (few) nonfinite = nonfinite || !(nan_sum == T(0));
         return f;
     }
 }
