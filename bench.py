@@ -470,19 +470,19 @@ def main():
     if dom == "spmv":
         # s = (w I + H) z from the solver's packed lower triangle: its blocks
         # once (every vertex has its diagonal block here, so n_b + n_v blocks
-        # make both triangles), per CSR block its column and its stored-block
-        # index, block-row offsets, z read once, s written
+        # make both triangles), per CSR block its column, per upper block the
+        # block stored for it, block-row offsets, z read once, s written
         n_sym = (nb + P.n_handles) // 2
-        traffic_alg = 72 * n_sym + 8 * nb + 4 * (P.n_handles + 1) + 2 * 8 * n
+        traffic_alg = 72 * n_sym + 4 * nb + 4 * (nb - n_sym) + 8 * (P.n_handles + 1) + 2 * 8 * n
         roof = {"kernel": "k_spmv_sym<3,8,true>", "bound": "hbm", "achieved": traffic_alg / avg_s / 1e9,
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "bytes_per_launch": traffic_alg,
                 "pmc_name": "tad::k_spmv_sym<3, 8, true>"}
-    elif dom == "assemble_hessian":
+    elif dom == "assemble_hessian" or (dom == "assemble" and fn.assembly_shape == 0):
         tsz = 8 if args.precision == "fp64" else 4
         d = P.d
         nblk = sum(t.conn.shape[0] * t.valence * (t.valence + 1) // 2 for t in P.terms)
         per_launch = nblk * d * d * tsz + 8 * nnz
-        kbase = ["k_assemble_hessian", "k_assemble_hessian_tpb", "k_assemble_hessian_upper",
+        kbase = ["k_assemble_all", "k_assemble_hessian_tpb", "k_assemble_hessian_upper",
                  "k_assemble_hessian_upper_tpb"][fn.assembly_shape]
         tname = "double" if tsz == 8 else "float"
         roof = {"kernel": f"{kbase}<{tname},{d}>", "bound": "hbm", "achieved": per_launch / avg_s / 1e9,
