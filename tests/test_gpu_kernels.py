@@ -208,3 +208,25 @@ def test_tet_projection_cases(ctx, m, state):
             fg.set_launch_shape(0, *shape)
             f, g, H = fg.eval_with_hessian_proj(x, eps)
             assert nrel(H.toarray(), ref.toarray()) <= 1e-12, (eps, shape)
+
+
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 8])
+def test_line_search_batches(ctx, batch):
+    """The step accepted on the device does not depend on the batch size, and
+    a limit on the trials holds inside a batch: one trial fewer than needed
+    accepts nothing and returns x0."""
+    import torch
+    P = configs.twist_cube(m=3, seed=5)
+    fg = tad.ScalarFunction.from_problem(P, ctx)
+    f, g, H = fg.eval_with_hessian_proj(P.x0)
+    d, _ = fg.solve(g, w=1e-6)
+    x, dt, gt = (torch.tensor(a, device="cuda:0") for a in (P.x0, -200.0 * np.asarray(d), g))
+    ref, f_ref, s_ref, n_ref = fg.line_search(x, dt, f, gt, opts=tad.newton_default_opts(ls_batch=1))
+    assert n_ref > 8
+    out, f_new, s, n = fg.line_search(x, dt, f, gt, opts=tad.newton_default_opts(ls_batch=batch))
+    assert (f_new, s, n) == (f_ref, s_ref, n_ref) and torch.equal(out, ref)
+    out, f_new, s, n = fg.line_search(x, dt, f, gt, opts=tad.newton_default_opts(ls_batch=batch, ls_max_iters=n_ref))
+    assert (f_new, s, n) == (f_ref, s_ref, n_ref) and torch.equal(out, ref)
+    out, f_new, s, n = fg.line_search(x, dt, f, gt,
+                                      opts=tad.newton_default_opts(ls_batch=batch, ls_max_iters=n_ref - 1))
+    assert n < 0 and s == 0.0 and torch.equal(out, x)
