@@ -290,14 +290,19 @@ __device__ __forceinline__ bool ldl_pd(const double* A, double shift)
 // Most eigenvalues project_few clamps (three bounds what an
 // isotropic energy of a tet has below zero: one per pair of singular values).
 constexpr int kMaxClamped = 3;
-// On the scaled tridiagonal: where the search for the next root starts below
-// the last one; the Laguerre step at which a root is final; the distance from
-// the level below which a root counts as the level itself, and where the
-// count starts then; how far equal roots may be moved, the other roots' share
-// of the log-derivative they allow per step, and the shift off them for their
-// vectors; the residual at which a vector is final and the largest accepted.
-constexpr double kRootGap = 1e-5, kRootStep = 1e-7, kRootApart = 1e-13, kLevelShift = 1e-9,
-                 kWeakMove = 1e-7, kWeakShare = 1e4, kWeakShift = 1e-9, kResidual = 2e-15, kResidualMax = 1e-14;
+// On the scaled tridiagonal (norm 1): the rounding of a root; the shift off
+// roots that cannot be told apart for their vectors; the residual at which a
+// vector is final, the largest accepted, and the passes it gets.
+constexpr double kRootRounding = 1e-15, kSharedShift = 1e-13, kResidual = 2e-15, kResidualMax = 4e-15;
+constexpr int kVectorPasses = 5;
+// Distances from a known root at which the search for the next one sets out:
+// the largest with no root between.  (Closer than a thousandth of the distance
+// to the next root, the rounding of the known one would drown it.)
+constexpr int kRootGaps = 6;
+__device__ __forceinline__ double root_gap(int i)
+{
+    return ldexp(1.0, i == 0 ? -7 : i == 1 ? -17 : i == 2 ? -27 : i == 3 ? -37 : i == 4 ? -43 : -47);
+}
 
 // Number of eigenvalues of the tridiagonal (d, e2 = squared couplings) below
 // x (negative pivots of T - x I), and the logarithmic derivative of
@@ -319,7 +324,7 @@ __device__ __forceinline__ int tridiag_count(const double* d, const double* e2, 
             const int i = c == 0 ? s : n - 1 - s;
             if (c == 1 && i <= mid) continue;
             double q = (d[i] - x) - w[c];
-            q = fabs(q) < 1e-100 ? -1e-100 : q;
+            q = fabs(q) < 1e-17 ? -1e-17 : q;
             const double r = refined_rcp(q);
             count += q < 0.0 ? 1 : 0;
             const double q2 = w[c] * (u[c] - 2.0 * t[c] * t[c]);
@@ -330,7 +335,7 @@ __device__ __forceinline__ int tridiag_count(const double* d, const double* e2, 
             w[c] = e2[c == 0 ? i : i - 1] * r;
         }
     double q = ((d[mid] - x) - w[0]) - w[1];
-    q = fabs(q) < 1e-100 ? -1e-100 : q;
+    q = fabs(q) < 1e-17 ? -1e-17 : q;
     const double r = refined_rcp(q);
     count += q < 0.0 ? 1 : 0;
     const double q2 = w[0] * (u[0] - 2.0 * t[0] * t[0]) + w[1] * (u[1] - 2.0 * t[1] * t[1]);
@@ -338,6 +343,59 @@ __device__ __forceinline__ int tridiag_count(const double* d, const double* e2, 
     s1 = a1[0] + a1[1] + tm;
     s2 = a2[0] + a2[1] + (q2 * r - tm * tm);
     return count;
+}
+
+// y <- (T - shift I)^-1 y for the tridiagonal (d, e) by Givens rotations: no
+// element growth at any shift (a zero pivot counts as 1e-30).
+template <int n>
+__device__ __forceinline__ void tridiag_solve(const double* d, const double* e, double shift, double* y)
+{
+    double r0[n], r1[n], r2[n];  // rows of R: reciprocal diagonal, the two superdiagonals
+    double a = d[0] - shift, b = e[0];
+#pragma unroll
+    for (int i = 0; i + 1 < n; ++i)
+    {
+        const double x = e[i], an = d[i + 1] - shift, bn = i + 2 < n ? e[i + 1] : 0.0;
+        const double w = a * a + x * x;
+        const bool zero = !(w > 1e-60);
+        const double ih = ql_rsqrt(zero ? 1.0 : w);
+        const double c = zero ? 1.0 : a * ih, s = zero ? 0.0 : x * ih;
+        r0[i] = zero ? 1e30 : ih;
+        r1[i] = c * b + s * an;
+        r2[i] = s * bn;
+        a = c * an - s * b;
+        b = c * bn;
+        const double t = c * y[i] + s * y[i + 1];
+        y[i + 1] = c * y[i + 1] - s * y[i];
+        y[i] = t;
+    }
+    r0[n - 1] = refined_rcp(fabs(a) < 1e-30 ? 1e-30 : a);
+#pragma unroll
+    for (int i = n - 1; i >= 0; --i)
+    {
+        if (i + 1 < n) y[i] -= r1[i] * y[i + 1];
+        if (i + 2 < n) y[i] -= r2[i] * y[i + 2];
+        y[i] *= r0[i];
+    }
+}
+
+// v / |v|, without overflow for |v| up to 1e300
+template <int n>
+__device__ __forceinline__ void normalize(double* v)
+{
+    double top = 0.0, vv = 0.0;
+#pragma unroll
+    for (int i = 0; i < n; ++i) top = fmax(top, fabs(v[i]));
+    const double it = refined_rcp(top);
+#pragma unroll
+    for (int i = 0; i < n; ++i)
+    {
+        v[i] *= it;
+        vv += v[i] * v[i];
+    }
+    const double iv = ql_rsqrt(vv);
+#pragma unroll
+    for (int i = 0; i < n; ++i) v[i] *= iv;
 }
 
 // Place of reflector k (n - 1 - k values) among the stored ones, and their
@@ -350,27 +408,37 @@ __host__ __device__ constexpr int reflector_values(int n) { return reflector_at(
 // over the eigenvalues below the clamp level only, so no other eigenvector
 // and no full spectrum is computed.  Returns false, with A restored up to
 // rounding, when more than kMaxClamped eigenvalues are clamped or a vector
-// misses its residual or orthogonality bound; the caller then projects A by
-// the full eigensolve (none of 24,000 elements of the 16^3 twisted cube, 0.1 %
-// of those within 1e-4 of a rest state).
+// misses its residual; the caller then projects A by the full eigensolve.
 //   1. Householder reduction to the tridiagonal T, scaled by a power of two
 //      to norm 1, the reflectors going to `store` (in registers they do not
 //      fit beside the rest); the number m of clamped eigenvalues from the
-//      pivot signs.
+//      pivot signs.  Roots within rounding of the level are not clamped
+//      (they would move by rounding).
 //   2. Their values from right to left by Laguerre's iteration (cubic, and
 //      monotone towards the neighbouring root as all roots are real), each
-//      started below the previous root, which is divided out: 6.7 evaluations
-//      per matrix, 10.7 for the slowest lane of a wave, where the full QL
-//      iteration takes 27.5 sweeps of a wave.
-//   3. Their vectors from twisted factorizations of T - lam I (Fernando,
-//      SIAM J. Matrix Anal. Appl. 18 (1997) 1013-1034) at the index with the
-//      smallest twist pivot, which gives the residual; Rayleigh quotient
-//      steps until it is at rounding level; two Gram-Schmidt passes, so that
-//      close eigenvalues (whose vectors are determined as a set only) give
-//      orthonormal vectors of their common space.
+//      started next to the previous root, which is divided out.  k roots that
+//      look like one are approached as one k-fold root; roots within 1e-14 of
+//      each other share one value.
+//   3. Their vectors: a twisted factorization of T - lam I (Fernando, SIAM J.
+//      Matrix Anal. Appl. 18 (1997) 1013-1034) at the index with the smallest
+//      twist pivot, then inverse iteration until T z - rho z is at rounding
+//      level, with two Gram-Schmidt passes against the earlier vectors.  m
+//      orthonormal vectors with such residuals and m Rayleigh quotients below
+//      the level are all there is below it, however close the roots are:
+//      which vectors of close roots they are does not matter to P(A).
 //   4. T + sum c w w^T, then the reflectors from both sides.
-// Error against 80-bit arithmetic on those elements, relative to |A|: 7e-16
-// in the mean, 3e-15 at most (full eigensolve: 1.4e-15 and 5e-15).
+// On the CPU, 6,000 element matrices (10^3 cube) per state, eps 1e-9, 0 and
+// absolute values, against 80-bit arithmetic, relative to |A|: at rest, noise
+// of 1e-12 .. 0.1 mesh widths, smooth displacements, compressed and flattened
+// by 1e-9 .. 0.2, twisted by 0.01 .. 60 degrees 4.1e-15 at most (full
+// eigensolve 4.2e-15), at most 0.13 % of the elements given to the full
+// eigensolve.  Noise of 1e-13 and 1e-14 mesh widths, whose roots are hardly
+// above rounding: 0.3 %, and 3 and 23 % for eps <= 0, where the level lies
+// among them; error 1.5e-14 at most.  8 to 17 evaluations of step 2 per wave,
+// where the full QL iteration takes 27 sweeps.  Evaluation of 1,296,000 tets:
+// twisted by 30 and 54 degrees 0.85 and 0.84 ms, at rest 0.77, noise of 1e-9
+// and 1e-4 0.89 and 0.83, compressed by 1e-4 0.79 (with the full eigensolve,
+// and a tail of its own launches, 1.36, 1.35, 1.18, 1.14, 1.25, 1.12).
 template <int n>
 __device__ __forceinline__ bool project_few(double* A, double eps, double* store)
 {
@@ -378,8 +446,9 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
 #pragma unroll
     for (int q = 0; q < Sym<n>::n; ++q) amax = fmax(amax, fabs(A[q]));
     if (!(amax > 1e-100 && amax < 1e100)) return false;
-    double d[n], e[n], tau[n - 2];
-    // 1. as in tridiag_ql_eigen, with refined reciprocals
+    double d[n], e[n];
+    // 1. as in tridiag_ql_eigen, with refined reciprocals; a reflector that is
+    //    the identity is stored as 0
 #pragma unroll
     for (int k = 0; k + 2 < n; ++k)
     {
@@ -394,10 +463,9 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
         const double v0 = x0 > 0.0 ? x0 + mu : x0 - mu;
         const double tk = has ? 2.0 * refined_rcp(v0 * v0 + sigma) : 0.0;
         e[k] = has ? (x0 > 0.0 ? -mu : mu) : x0;
-        tau[k] = tk;
         A[Sym<n>::idx(k, k + 1)] = v0;
 #pragma unroll
-        for (int i = 0; i < L; ++i) store[(reflector_at(n, k) + i) * 64] = A[Sym<n>::idx(k, k + 1 + i)];
+        for (int i = 0; i < L; ++i) store[(reflector_at(n, k) + i) * 64] = has ? A[Sym<n>::idx(k, k + 1 + i)] : 0.0;
         double pv[n], vp = 0.0;
 #pragma unroll
         for (int i = 0; i < L; ++i)
@@ -439,16 +507,16 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
         e2[i] = e[i] * e[i];
     }
     const double level = ldexp(eps > 0.0 ? eps : 0.0, -ex);
-    // 2. roots r[0] >= r[1] >= ... below the level
+    // 2. roots r[0] >= r[1] >= ... below `start`
     double r[kMaxClamped] = {};
+    double start = level - kRootRounding;
     int m = 0, found = 0;
-    bool weak = false;     // roots that count as one value
-    double start = level;  // the roots below it are clamped
     {
-        double x = level;
-        bool fresh = false, run = true, first = true;
+        double x = start, from = start;  // from: the last root (or the level)
+        int gap = -1;                    // >= 0: x lies root_gap(gap) below `from`
+        bool first = true, run = true;
 #pragma unroll 1
-        for (int it = 0; run && it < 48; ++it)
+        for (int it = 0; run && it < 64; ++it)
         {
             double g, h;
             const int below = tridiag_count<n>(d, e2, x, g, h);
@@ -457,83 +525,103 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
             {
                 m = below;
                 if (m == 0 || m > kMaxClamped) break;
-                first = false;
             }
-            if (below < m - found)
-            {
-                // a root between x and the last one found: too close to tell
-                // apart from it; or x itself, passed by rounding
-                if (fresh) break;
-            }
-#pragma unroll
-            for (int j = 0; j + 1 < kMaxClamped; ++j)
-                if (j < found)
-                {
-                    const double q = refined_rcp(x - r[j]);
-                    g -= q;
-                    h -= q * q;
-                }
-            const double deg = (double)(n - found);
-            const double gg = g * g;
-            const double disc = (deg - 1.0) * (deg * h - gg);
-            const double sq = disc > 0.0 ? disc * ql_rsqrt(disc) : 0.0;
-            const double step = deg * refined_rcp(g + sq);
-            // next to k equal roots g = k / (x - root), h = k / (x - root)^2, up
-            // to the other roots' share (g < 0: the near ones lie above x)
+            const int inside = m - found - below;  // roots not found yet that are not below x
             int take = 0;
-            double share = 1.0;
-            if (g > 0.0 && step < kRootStep)
-#pragma unroll
-                for (int k = kMaxClamped; k >= 1; --k)
-                    if (k <= m - found && fabs(gg - k * h) < 0.01 * gg)
-                    {
-                        take = k;
-                        share = fabs(gg - k * h);
-                    }
-            if (take > 1)
+            double root = from;
+            if (gap >= 0 && inside > 0)
             {
-                // equal roots: only where the clamping moves them by next to
-                // nothing and the others are well apart
-                const double move = eps < 0.0 ? -2.0 * x : level - x;
-                if (!(move < kWeakMove && share < gg * fabs(step) * kWeakShare)) break;
-                weak = true;
+                // between the last root and x
+                if (gap + 1 < kRootGaps)
+                {
+                    x = from - root_gap(++gap);
+                    continue;
+                }
+                take = inside;  // cannot be told apart from it
             }
-            else if (below < m - found || (g > 0.0 && step < 2e-16))
-                take = 1;
-            const double root = x - (take > 1 ? take * refined_rcp(g) : step);
-            if (take > 0 && found == 0 && !(root < start - kRootApart))
+            else
             {
-                // the level itself is an eigenvalue up to rounding: count
-                // (and clamp, by nothing) it as one of those below
-                if (start != level) break;
-                start = level + kLevelShift;
-                x = start;
+#pragma unroll
+                for (int j = 0; j + 1 < kMaxClamped; ++j)
+                    if (j < found)
+                    {
+                        const double q = refined_rcp(x - r[j]);
+                        g -= q;
+                        h -= q * q;
+                    }
+                if (first && g < -1e3)
+                {
+                    // roots right above the level: set out away from them
+                    first = false;
+                    gap = 0;
+                    x = from - root_gap(gap);
+                    continue;
+                }
+                const double deg = (double)(n - found), gg = g * g;
+                const double spread = deg * h - gg;  // 0 for one deg-fold root
+                const double disc = (deg - 1.0) * spread;
+                const double sq = disc > 0.0 ? disc * ql_rsqrt(disc) : 0.0;
+                // k equal roots have g = k / (x - root), h = k / (x - root)^2
+                // (g < 0: the near ones lie above x)
+                int fold = 1;
+                double dev = fabs(gg - h);
+#pragma unroll
+                for (int k = 2; k <= kMaxClamped; ++k)
+                    if (k <= m - found && fabs(gg - k * h) < dev)
+                    {
+                        dev = fabs(gg - k * h);
+                        fold = k;
+                    }
+                const bool past = inside > 0;  // x is below the next root: towards it
+                const bool alike = (past ? g < 0.0 : g > 0.0) && dev < 0.01 * gg;
+                double step = deg * refined_rcp(past ? g - sq : g + sq);
+                if (alike && fold == 1)
+                    take = fabs(step) * dev * dev < 1e-16 * gg * gg ? 1 : 0;  // (the error: step (dev / gg)^2)
+                else if (alike)
+                {
+                    const double f = (deg - fold) / fold * spread;
+                    const double sf = f > 0.0 ? f * ql_rsqrt(f) : 0.0;
+                    step = deg * refined_rcp(past ? g - sf : g + sf);
+                    take = fabs(step) < 1e-13 ? fold : 0;
+                }
+                if (fabs(step) < 4e-16 && (past || g > 0.0)) take = max(take, 1);
+                root = x - step;
+                if (inside > 1)
+                {
+                    // beyond all but one of them, or they share a value
+                    take = fabs(step) < 1e-14 ? inside : 0;
+                    step *= 2.0;
+                }
+                else if (take == 0 && alike && fold > 1)
+                {
+                    // short of the first of them (their spread is about 2 sqrt(dev / gg) of the distance)
+                    const double q = fmax(dev * refined_rcp(gg), 1e-12);
+                    step *= 1.0 - 2.0 * q * ql_rsqrt(q);
+                }
+                if (take == 0) x -= step;
+            }
+            first = false;
+            gap = -1;
+            if (take == 0) continue;
+            if (found == 0 && !(root < start - 2.0 * kRootRounding))
+            {
+                // at the level up to rounding: those below it are clamped
+                if (!(root > level - 4.0 * kRootRounding)) break;
+                start = x = from = root - 2.0 * kRootRounding;
                 first = true;
                 continue;
             }
-            x -= step;
-            fresh = false;
-            if (take > 0)
-            {
 #pragma unroll
-                for (int j = 0; j < kMaxClamped; ++j)
-                    if (j >= found && j < found + take) r[j] = root;
-                found += take;
-                run = found < m;
-                x = root - kRootGap;
-                fresh = true;
-            }
+            for (int j = 0; j < kMaxClamped; ++j)
+                if (j >= found && j < found + take) r[j] = root;
+            found += take;
+            run = found < m;
+            from = root;
+            gap = 1;
+            x = from - root_gap(gap);
         }
     }
     ok = ok && m <= kMaxClamped && found == m;
-    // the lowest first: the vectors of equal roots next to the level (which
-    // need not be accurate, they move by next to nothing) are made orthogonal
-    // to the others, not the others to them
-    static_assert(kMaxClamped == 3, "the order of up to three roots is reversed");
-    const double top = r[0];
-    r[0] = m == 3 ? r[2] : (m == 2 ? r[1] : r[0]);
-    r[1] = m == 2 ? top : r[1];
-    r[2] = m == 3 ? top : r[2];
     // 3.
     double W[kMaxClamped][n], c[kMaxClamped];
 #pragma unroll
@@ -544,13 +632,11 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
         for (int i = 0; i < n; ++i) W[j][i] = 0.0;
         if (ok && j < m)
         {
-            double lam = r[j], res = 0.0, z[n];
+            double lam = r[j], z[n];
             bool shared = false;
 #pragma unroll
-            for (int q = 0; q < kMaxClamped; ++q) shared = shared || (weak && q != j && q < m && r[q] == r[j]);
-            if (shared) lam -= kWeakShift;
-#pragma unroll 1
-            for (int pass = 0; pass < 3; ++pass)
+            for (int q = 0; q < kMaxClamped; ++q) shared = shared || (q != j && q < m && r[q] == r[j]);
+            if (shared) lam -= kSharedShift;
             {
                 // pivots from the top (dp) and from the bottom (dm), side by side
                 double l[n], u[n], dp[n], dm[n];
@@ -567,23 +653,20 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
                     dp[i + 1] = (d[i + 1] - lam) - e[i] * l[i];
                     dm[b - 1] = (d[b - 1] - lam) - e[b - 1] * u[b - 1];
                 }
-                double gamma = 0.0, best = 1e300;
+                // the smallest twist pivot's vector (of roots close to an
+                // earlier one, not the earlier vector again)
+                double best = 1e300;
                 int k = n - 1;
 #pragma unroll
                 for (int i = n - 1; i >= 0; --i)
                 {
-                    const double gi = dp[i] + (dm[i] - (d[i] - lam));
+                    const double gi = fabs(dp[i] + (dm[i] - (d[i] - lam)));
                     double used = 0.0;
 #pragma unroll
                     for (int q = 0; q < j; ++q) used += W[q][i] * W[q][i];
-                    // the smallest pivot's vector; of equal roots the one with
-                    // the largest part (shift / pivot) outside the earlier ones
-                    const double rank = shared ? used - kWeakShift * refined_rcp(fmax(fabs(gi), 1e-30))
-                                               : (used < 0.5 ? fabs(gi) : 1e300);
-                    if (rank < best)
+                    if (used < 0.5 && gi < best)
                     {
-                        best = rank;
-                        gamma = gi;
+                        best = gi;
                         k = i;
                     }
                 }
@@ -599,42 +682,58 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
                 const double iz = ql_rsqrt(zz);
 #pragma unroll
                 for (int i = 0; i < n; ++i) z[i] *= iz;
-                res = shared ? 0.0 : fabs(gamma) * iz;
-                lam += gamma * iz * iz;
-                if (res < kResidual) break;
             }
-            double zz = 1.0;
-            if (j > 0)
+            double rho = 0.0, rr = 0.0;  // Rayleigh quotient, squared residual
+#pragma unroll 1
+            for (int pass = 0; pass < kVectorPasses; ++pass)
             {
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
+                if (pass > 0)
                 {
-#pragma unroll
-                    for (int q = 0; q < j; ++q)
-                    {
-                        double s = 0.0;
-#pragma unroll
-                        for (int i = 0; i < n; ++i) s += W[q][i] * z[i];
-#pragma unroll
-                        for (int i = 0; i < n; ++i) z[i] -= s * W[q][i];
-                    }
-                    zz = 0.0;
-#pragma unroll
-                    for (int i = 0; i < n; ++i) zz += z[i] * z[i];
-                    ok = ok && zz > 0.01;
-                    const double iz = ql_rsqrt(zz);
-#pragma unroll
-                    for (int i = 0; i < n; ++i) z[i] *= iz;
+                    tridiag_solve<n>(d, e, pass == 1 ? lam : rho, z);
+                    normalize<n>(z);
                 }
-            }
-                        double rho = 0.0;
+                double zz = 1.0;  // what the second orthogonalization kept
+                if (j > 0)
 #pragma unroll
-            for (int i = 0; i < n; ++i)
-            {
-                W[j][i] = z[i];
-                rho += z[i] * (d[i] * z[i] + (i + 1 < n ? 2.0 * e[i] * z[i + 1] : 0.0));
+                    for (int t = 0; t < 2; ++t)
+                    {
+#pragma unroll
+                        for (int q = 0; q < j; ++q)
+                        {
+                            double s = 0.0;
+#pragma unroll
+                            for (int i = 0; i < n; ++i) s += W[q][i] * z[i];
+#pragma unroll
+                            for (int i = 0; i < n; ++i) z[i] -= s * W[q][i];
+                        }
+                        zz = 0.0;
+#pragma unroll
+                        for (int i = 0; i < n; ++i) zz += z[i] * z[i];
+                        const double iz = ql_rsqrt(zz);
+#pragma unroll
+                        for (int i = 0; i < n; ++i) z[i] *= iz;
+                    }
+                double tz[n];
+                rho = 0.0;
+                rr = 0.0;
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                {
+                    tz[i] = d[i] * z[i] + (i + 1 < n ? e[i] * z[i + 1] : 0.0) + (i > 0 ? e[i - 1] * z[i - 1] : 0.0);
+                    rho += z[i] * tz[i];
+                }
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                {
+                    const double t = tz[i] - rho * z[i];
+                    rr += t * t;
+                }
+                if (!(zz > 0.5)) rr = 1.0;
+                if (rr < kResidual * kResidual) break;
             }
-            ok = ok && res < kResidualMax && rho < start + kResidualMax;
+#pragma unroll
+            for (int i = 0; i < n; ++i) W[j][i] = z[i];
+            ok = ok && rr < kResidualMax * kResidualMax && rho < start - kRootRounding;
             c[j] = fmax(eps < 0.0 ? -2.0 * rho : level - rho, 0.0);
         }
     }
@@ -655,16 +754,20 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
     for (int k = n - 3; k >= 0; --k)
     {
         const int L = n - k - 1;
-        double v[n];
+        double v[n], vv = 0.0;
 #pragma unroll
         for (int i = 0; i < L; ++i) v[i] = store[(reflector_at(n, k) + i) * 64];
+#pragma unroll
+        for (int i = 1; i < L; ++i) vv += v[i] * v[i];
+        vv += v[0] * v[0];
+        const double tau = vv > 0.0 ? 2.0 * refined_rcp(vv) : 0.0;
 #pragma unroll
         for (int row = 0; row <= k; ++row)
         {
             double s = 0.0;
 #pragma unroll
             for (int i = 0; i < L; ++i) s += P[Sym<n>::idx(row, k + 1 + i)] * v[i];
-            s *= tau[k];
+            s *= tau;
 #pragma unroll
             for (int i = 0; i < L; ++i) P[Sym<n>::idx(row, k + 1 + i)] -= s * v[i];
         }
@@ -675,10 +778,10 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
             double acc = 0.0;
 #pragma unroll
             for (int j = 0; j < L; ++j) acc += P[Sym<n>::at(k + 1 + i, k + 1 + j)] * v[j];
-            pv[i] = tau[k] * acc;
+            pv[i] = tau * acc;
             vp += v[i] * pv[i];
         }
-        const double K = 0.5 * tau[k] * vp;
+        const double K = 0.5 * tau * vp;
 #pragma unroll
         for (int i = 0; i < L; ++i) pv[i] -= K * v[i];
 #pragma unroll
