@@ -1,0 +1,68 @@
+"""Which preconditioner a solve takes and keeps, through the public entry points."""
+import numpy as np
+import pytest
+
+import tinyad_amd as tad
+from tinyad_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+
+def pinned_grid(n, seed=1):
+    """grid_param with its left and right columns pinned (a definite Hessian)."""
+    P = configs.grid_param(n, seed)
+    cols = np.concatenate([np.arange(n) * n, np.arange(n) * n + n - 1]).astype(np.int32)
+    pins = configs.Term(configs.E_PENALTY, cols[:, None].copy(),
+                        np.concatenate([P.x0.reshape(-1, 2)[cols], np.ones((cols.size, 1))], axis=1))
+    return configs.Problem(f"grid_pinned_{n}", 2, P.n_handles, [P.terms[0], pins], P.x0)
+
+
+def indefinite(ctx, n):
+    """(function, H, A, b): A = H - s I, of H's pattern, with one negative
+    eigenvalue, and right-hand sides b with b . A^-1 b of either sign."""
+    import scipy.sparse as sp
+    P = pinned_grid(n)
+    fn = tad.ScalarFunction.from_problem(P, ctx)
+    _, _, H = fn.eval_with_hessian_proj(P.x0)
+    lam, V = np.linalg.eigh(H.toarray())
+    A = (H - 0.5 * (lam[0] + lam[1]) * sp.identity(H.shape[0])).tocsr()
+    A.sort_indices()
+    assert np.array_equal(A.indices, H.indices)
+    mu = lam - 0.5 * (lam[0] + lam[1])
+    c = np.random.default_rng(5).standard_normal(lam.size)
+    rest = float(np.sum(c[1:] ** 2 / mu[1:]))
+    b = {}
+    for sign in (1.0, -1.0):
+        c[0] = np.sqrt(-mu[0] * rest * (0.25 if sign > 0 else 4.0))
+        b[sign] = V @ c
+        assert sign * (b[sign] @ np.linalg.solve(A.toarray(), b[sign])) > 0.0
+    return fn, H, A, b
+
+
+# the dense preconditioner of small systems, and the two-level one
+@pytest.mark.parametrize("n", [6, 16, 33])
+def test_indefinite_systems_are_refused(ctx, n):
+    """w I + H must be positive definite, whatever the right-hand side: also
+    where b . A^-1 b > 0, so that the curvature along A^-1 b is positive."""
+    fn, H, A, b = indefinite(ctx, n)
+    for sign in (1.0, -1.0):
+        with pytest.raises(tad.TadError):
+            _, st = fn.solve(b[sign], H=A.data, tol=1e-10)
+            if not st.converged:
+                raise tad.TadError(0, "not converged")
+        # the definite system of the same function still takes the dense inverse
+        x, st = fn.solve(b[sign], H=H.data, tol=1e-10)
+        assert st.converged and st.coarse_unknowns == (2 * n * n if 2 * n * n <= 2400 else st.coarse_unknowns)
+        assert np.linalg.norm(H @ x - b[sign]) <= 1e-9 * np.linalg.norm(b[sign])
+
+
+def test_inverse_of_an_indefinite_matrix_is_not_kept(ctx):
+    """A solve with b = 0 converges at once; the inverse it formed is kept for
+    a later solve only when its matrix was positive definite."""
+    fn, H, A, b = indefinite(ctx, 16)
+    x, st = fn.solve(np.zeros(H.shape[0]), H=A.data)
+    assert st.converged and not np.any(x)
+    x, st = fn.solve(b[1.0], H=H.data, tol=1e-10, coarse_reuse=1)
+    assert st.converged and st.coarse_reused == 0 and st.iters <= 2
+    _, st = fn.solve(b[1.0], H=H.data, tol=1e-10, coarse_reuse=1)
+    assert st.converged and st.coarse_reused == 1 and st.iters <= 2

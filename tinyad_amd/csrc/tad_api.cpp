@@ -1083,6 +1083,7 @@ constexpr double kCoarse32Change = 0.1;
 PcgReport* pcg_report(tad_fn fn) { return reinterpret_cast<PcgReport*>(fn->ctx->pinned + 56); }
 LineSearchHost* ls_host(tad_fn fn) { return reinterpret_cast<LineSearchHost*>(fn->ctx->pinned + 72); }
 int* mode_host(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 96); }
+int* dense_flag(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 97); }
 
 tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o, const unsigned char* free_dev,
                         PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused, bool lagged)
@@ -1489,9 +1490,9 @@ constexpr int64_t kDenseVars2 = 2400, kDenseVars3 = 1536;
 // useless), with a rebuilt and with a reused inverse.
 constexpr int kDenseIters = 32, kDenseReuseIters = 200;
 
-// One solve.  lagged: the coarse space serves several solves.  dense: with the dense preconditioner; *again = true when that
-// one is not usable or did not converge within its iterations (nothing is
-// returned then).
+// One solve.  lagged: the coarse space serves several solves.  dense: with the
+// dense preconditioner; *again = true when that one is not usable or did not
+// converge within its iterations (nothing is returned then).
 tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev, const tad_solve_opts& o,
                       tad_solve_stats* st, const unsigned char* free_dev, bool lagged, bool dense, bool* again)
 {
@@ -1576,7 +1577,7 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
             TAD_HIP(c.inv_work.ensure((size_t)spd_inverse_work(n)));
             TAD_HIP(launch_dense_fill(d, sys, c.dense_inv.p, s));
             tm.begin("coarse_inverse", s);
-            TAD_HIP(launch_spd_inverse(n, c.dense_inv.p, c.inv_work.p, c.info.p, s));
+            TAD_HIP(launch_spd_inverse(n, c.dense_inv.p, c.inv_work.p, c.info.p, s, dense_flag(fn)));
             tm.end("coarse_inverse", s);
             tm.end("coarse_setup", s);
         }
@@ -1670,7 +1671,11 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     }
     std::atomic_thread_fence(std::memory_order_acquire);
     const PcgReport hs = *rep;
-    if (dense && (hs.breakdown || (sys.max_iters < o.max_iters && !(hs.rr <= sys.tol2 * hs.bb))))
+    // (a matrix that is not positive definite has an inverse all the same, and
+    // with that one CG ends in one step for every right-hand side b with
+    // b . A^-1 b > 0: the two-level solve decides instead)
+    if (dense && ((!coarse_reused && *dense_flag(fn) != 0) || hs.breakdown ||
+                  (sys.max_iters < o.max_iters && !(hs.rr <= sys.tol2 * hs.bb))))
     {
         *again = true;
         return TAD_OK;

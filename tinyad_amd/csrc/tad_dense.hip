@@ -460,10 +460,13 @@ __global__ __launch_bounds__(256, 2) void k_sweep_step(int64_t nt, int64_t K, in
     }
 }
 
-// A = -S on the leading n x n part, both triangles (the sweeps leave -A^-1).
-__global__ __launch_bounds__(256) void k_sweep_store(int64_t n, const double* __restrict__ S, double* __restrict__ A)
+// A = -S on the leading n x n part, both triangles (the sweeps leave -A^-1);
+// the finished flag to info_host (optional, pinned).
+__global__ __launch_bounds__(256) void k_sweep_store(int64_t n, const double* __restrict__ S, double* __restrict__ A,
+                                                     const int* __restrict__ info, int* __restrict__ info_host)
 {
     __shared__ Tile P;
+    if (info_host && blockIdx.x == 0 && threadIdx.x == 0) *info_host = info[0];
     int64_t I = 0, J = blockIdx.x;
     while (J > I) J -= ++I;
     const double* __restrict__ in = S + tile_at(I, J);
@@ -497,7 +500,7 @@ int64_t spd_inverse_work(int64_t n)
     return 2 * (nt * (nt + 1) / 2) * kTT + 2 * kTT;
 }
 
-hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hipStream_t s)
+hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hipStream_t s, int* info_host)
 {
     if (n <= 0) return hipSuccess;
     const int64_t nt = (n + kTile - 1) / kTile;
@@ -514,7 +517,7 @@ hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hip
     for (int64_t K = 0; K < nt; ++K)
         k_sweep_step<<<(unsigned)(strips + (K + 1 < nt ? 1 : 0)), 256, 0, s>>>(nt, K, L, S[K & 1], Q[K & 1],
                                                                                S[(K + 1) & 1], Q[(K + 1) & 1], info);
-    k_sweep_store<<<(unsigned)tiles, 256, 0, s>>>(n, S[nt & 1], A);
+    k_sweep_store<<<(unsigned)tiles, 256, 0, s>>>(n, S[nt & 1], A, info, info_host);
     return hipGetLastError();
 }
 
