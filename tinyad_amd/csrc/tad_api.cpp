@@ -74,6 +74,10 @@ struct DevBuf
 {
     T* p = nullptr;
     size_t n = 0;
+    DevBuf() = default;
+    DevBuf(const DevBuf&) = delete;
+    DevBuf& operator=(const DevBuf&) = delete;
+    ~DevBuf() { release(); }  // (the owner's device is current when it is destroyed)
     hipError_t ensure(size_t count)
     {
         if (count <= n && p) return hipSuccess;
