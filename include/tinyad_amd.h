@@ -385,10 +385,11 @@ tad_status tad_fn_autotune(tad_fn fn, const double* x, tad_mem mem, double eps, 
  * symmetric-Dirichlet term): block 0 is the plain grid; otherwise a
  * persistent grid of `grid` workgroups (1 .. 2^20) of 64, 128 or 256 lanes,
  * map 0 strided or 1 per-XCD contiguous (grid a multiple of 8).  Hessian
- * assembly shape 0 .. 3 (automatic by size, tiles of whole rows or one of the
- * others; one thread per CSR block; d*d lanes or one thread per upper block
- * writing it and its mirror).  Every shape gives
- * bit-identical results.  No counterpart in the reference. */
+ * assembly shape 0 .. 3 (tiles of whole rows; one thread per CSR block; d*d
+ * lanes or one thread per upper block writing it and its mirror): the one in
+ * use, chosen by size until it is tuned or set (0 before the pattern is
+ * known).  Every shape gives bit-identical results.  No counterpart in the
+ * reference. */
 tad_status tad_fn_get_launch_shape(tad_fn fn, int term, int* block, int* grid, int* map);
 tad_status tad_fn_set_launch_shape(tad_fn fn, int term, int block, int grid, int map);
 tad_status tad_fn_get_assembly_shape(tad_fn fn, int* shape);

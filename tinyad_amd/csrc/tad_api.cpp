@@ -278,7 +278,7 @@ struct tad_fn_s
     // solves without a coarse space: handle order
     SolverOrder natural;
     DevBuf<double> sym_H;          // stored blocks of the order in use
-    int asm_shape = 0;             // Hessian assembly launch shape (tad_fn_autotune)
+    int asm_shape = -1;            // Hessian assembly shape as set or tuned; -1: by size (assembly_shape)
     std::vector<int32_t> h_brow_ptr, h_bcol;  // host copy of the block pattern (coarse aggregation)
     std::vector<int64_t> h_urow_ptr;          // first upper block of each block row (host)
     // pipelined second-order evaluation: the largest catalog term's elements
@@ -1277,7 +1277,7 @@ tad_status ensure_aux(tad_ctx ctx, int n_events)
     return TAD_OK;
 }
 
-// The assembly shape in use: as set or tuned; for 0 (the default) the tiles of
+// The assembly shape in use: as set or tuned; otherwise the tiles of
 // launch_eval_tail, except for large 3D patterns, where one launch of its own
 // is faster: whole evaluations in us by shape 0 tiles / 1 / 2 / 3, 60^3 cube
 // (3.3 M blocks) FP64 1,251 / 1,226 / 1,219 / 1,229, mixed 751 / 716 / 753 /
@@ -1287,7 +1287,8 @@ tad_status ensure_aux(tad_ctx ctx, int n_events)
 constexpr int64_t kTileBlocks3 = 200000;
 int assembly_shape(tad_fn fn)
 {
-    if (fn->asm_shape != 0 || fn->d < 3 || fn->n_blocks < kTileBlocks3) return fn->asm_shape;
+    if (fn->asm_shape >= 0) return fn->asm_shape;
+    if (fn->d < 3 || !fn->pattern_ready || fn->n_blocks < kTileBlocks3) return 0;
     return fn->precision == TAD_PREC_FP64 ? 2 : 1;
 }
 
@@ -1354,7 +1355,7 @@ tad_status eval_core(tad_fn fn, const double* x_dev, int mode, double eps, doubl
                 TAD_HIP(hipStreamWaitEvent(s2, ctx->events[k], 0));
                 // one timed span per chunk: gradient and Hessian rows of the chunk
                 tm.begin("assemble_hessian", s2);
-                TAD_HIP(launch_assemble_hessian(fn->d, fn->precision, fn->asm_shape, pat, fn->hc_buf.p, H_dev, s2, r0,
+                TAD_HIP(launch_assemble_hessian(fn->d, fn->precision, assembly_shape(fn), pat, fn->hc_buf.p, H_dev, s2, r0,
                                                 r1));
                 if (g_dev)
                     TAD_HIP(launch_assemble_gradient(fn->d, fn->precision, fn->n_handles, fn->gslot_ptr.p,
@@ -2952,7 +2953,7 @@ tad_status tad_fn_get_assembly_shape(tad_fn fn, int* shape)
 {
     TAD_TRY(check_fn(fn));
     if (!shape) return fail(TAD_ERR_INVALID, "null argument");
-    *shape = fn->asm_shape;
+    *shape = assembly_shape(fn);
     return TAD_OK;
 }
 
