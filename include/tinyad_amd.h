@@ -430,8 +430,10 @@ typedef struct tad_solve_opts
     int coarse_aggregate; /* two-level preconditioner: handles per aggregate of the      */
                         /* coarse space; 0: block-Jacobi only; < 0 (default): automatic, */
                         /* by mesh size (in 3D about 700 coarse unknowns up to 30K       */
-                        /* handles, at most 2,800; small systems, up to 2,400 variables  */
-                        /* or 1,536 in 3D, take the dense inverse of the whole matrix)   */
+                        /* handles, 1,400 once a solve of the function has asked for     */
+                        /* coarse_reuse, at most 2,800; small systems, up to 2,400       */
+                        /* variables or 1,536 in 3D, take the dense inverse of the whole */
+                        /* matrix)                                                       */
     int coarse_reuse;   /* 1: keep the coarse space and inverse coarse matrix of the     */
                         /* function's previous solve when it is compatible (same         */
                         /* aggregates, unknowns per aggregate and w, neither solve       */

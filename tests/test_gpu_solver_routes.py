@@ -97,3 +97,42 @@ def test_destroyed_functions_leave_no_device_memory(ctx):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     assert before - torch.cuda.mem_get_info()[0] <= 16 << 20
+
+
+def lagged_size(ctx, P):
+    """Coarse unknowns of a Newton loop that keeps its coarse space."""
+    fn = tad.ScalarFunction.from_problem(P, ctx)
+    return fn.newton_step(P.x0.copy(), tad.newton_default_opts(coarse_refresh=3))["coarse_unknowns"]
+
+
+def test_solves_between_lagged_newton_steps_share_the_coarse_space(ctx):
+    """Automatic solves between the steps neither replace the steps' aggregates
+    nor make the next step rebuild what it was going to keep."""
+    P = configs.twist_cube(m=16)
+    fn = tad.ScalarFunction.from_problem(P, ctx)
+    opts = tad.newton_default_opts(coarse_refresh=5)
+    x = P.x0.copy()
+    n = fn.newton_step(x, opts)["coarse_unknowns"]
+    g = np.random.default_rng(0).standard_normal(x.size)
+    for _ in range(2):
+        _, st = fn.solve(g, tol=1e-8, w_identity=0.0)
+        assert st.converged and st.coarse_unknowns == n
+        s = fn.newton_step(x, opts)
+        assert s["coarse_reused"] == 1 and s["coarse_unknowns"] == n
+
+
+def test_callers_own_reuse_schedule_gets_the_lagged_size(ctx):
+    """A caller that asks for reuse solve by solve gets, from the next rebuild
+    on, the size of a space that serves several solves; the solves that only
+    keep what is there keep it."""
+    P = configs.twist_cube(m=16)
+    big = lagged_size(ctx, P)
+    fn = tad.ScalarFunction.from_problem(P, ctx)
+    _, g, _ = fn.eval_with_hessian_proj(P.x0)
+    sizes = []
+    for reuse in (0, 1, 1, 0, 1, 0):
+        _, st = fn.solve(g, tol=1e-8, coarse_reuse=reuse)
+        assert st.converged and st.coarse_reused == reuse
+        sizes.append(st.coarse_unknowns)
+    assert sizes[0] == sizes[1] == sizes[2] < big
+    assert sizes[3] == sizes[4] == sizes[5] == big

@@ -318,6 +318,7 @@ struct tad_fn_s
     struct Coarse
     {
         int requested = 0;            // aggregate size asked for when the pattern was built (0: none)
+        bool automatic = false;       // the last solve left that size to the library
         int target = 0;               // aggregate size the pattern was built with
         int64_t n_agg = 0, n_pairs = 0, n_gchunks = 0;
         SolverOrder ord;              // aggregate after aggregate, members ascending
@@ -366,6 +367,7 @@ struct tad_fn_s
     std::vector<uint64_t> pcg_graph_key;
     bool pcg_graph_failed = false;  // recording failed once: launch directly
     int solves_since_rebuild = 0;  // solves that reused the coarse space since it was built
+    bool keeps_coarse = false;     // some solve asked to reuse a coarse space (its automatic size)
 
     hipStream_t s() const { return ctx->stream; }
     HessAsm hess_asm() const
@@ -1090,7 +1092,7 @@ int* mode_host(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 96);
 int* dense_flag(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 97); }
 
 tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o, const unsigned char* free_dev,
-                        PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused, bool lagged)
+                        PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused)
 {
     *use = false;
     *reused = false;
@@ -1099,6 +1101,14 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     if (o.coarse_aggregate == 0 || nh == 0 || fn->n_blocks == 0) return TAD_OK;
     const bool rot = fn->x_hess_valid && d >= 2;
     const int kc = rot ? (d == 3 ? 6 : 3) : d;
+    auto& c = fn->co;
+    const bool automatic = o.coarse_aggregate < 0;
+    const bool keep = o.coarse_reuse && c.factor_valid && !free_dev && c.f_kc == kc && c.f_w == o.w_identity;
+    // the size for a space that serves several solves as soon as any solve of
+    // this function has asked for that (the sizes do not take turns: each
+    // change of size orders the mesh anew on the host); a space that can be
+    // kept as asked is kept whichever size it was built for
+    const bool lagged = fn->keeps_coarse;
     const int64_t agg = o.coarse_aggregate > 0
                             ? o.coarse_aggregate
                             : std::max<int64_t>(lagged || d == 3 ? kAutoMinAggregate : kAutoMinAggregate2,
@@ -1106,8 +1116,10 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
                                                                    auto_coarse_unknowns(d, nh, lagged)));
     // keep the dense coarse matrix bounded: larger aggregates for large meshes
     // (grown further while breadth-first aggregates come out too small)
-    const int want = (int)std::max<int64_t>(agg, (nh * kc + kMaxCoarse - 1) / kMaxCoarse);
-    auto& c = fn->co;
+    const int want = automatic && keep && c.automatic
+                         ? c.requested
+                         : (int)std::max<int64_t>(agg, (nh * kc + kMaxCoarse - 1) / kMaxCoarse);
+    c.automatic = automatic;
     if (c.requested != want)
     {
         c.factor_valid = false;
@@ -1144,7 +1156,7 @@ tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o,
     cd->coarse_mode = c.info.p + 1;
     cd->rpart = c.rpart.p;
     cd->cparts = c.cparts.p;
-    if (o.coarse_reuse && c.factor_valid && !free_dev && c.f_kc == kc && c.f_w == o.w_identity)
+    if (keep && c.factor_valid)
     {
         *use = true;
         *reused = true;
@@ -1495,11 +1507,11 @@ constexpr int64_t kDenseVars2 = 2400, kDenseVars3 = 1536;
 // useless), with a rebuilt and with a reused inverse.
 constexpr int kDenseIters = 32, kDenseReuseIters = 200;
 
-// One solve.  lagged: the coarse space serves several solves.  dense: with the
-// dense preconditioner; *again = true when that one is not usable or did not
-// converge within its iterations (nothing is returned then).
+// One solve.  dense: with the dense preconditioner; *again = true when that one
+// is not usable or did not converge within its iterations (nothing is returned
+// then).
 tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev, const tad_solve_opts& o,
-                      tad_solve_stats* st, const unsigned char* free_dev, bool lagged, bool dense, bool* again)
+                      tad_solve_stats* st, const unsigned char* free_dev, bool dense, bool* again)
 {
     const int d = fn->d;
     const int64_t nh = fn->n_handles, n = fn->n_vars;
@@ -1515,7 +1527,7 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
     PcgSystem sys;
     const SolverOrder* od = &fn->natural;
     bool use_coarse = false, coarse_reused = false;
-    if (!dense) TAD_TRY(setup_coarse(fn, H_dev, o, free_dev, &sys, &od, &use_coarse, &coarse_reused, lagged));
+    if (!dense) TAD_TRY(setup_coarse(fn, H_dev, o, free_dev, &sys, &od, &use_coarse, &coarse_reused));
     if (od == &fn->natural && !od->ready)
     {
         std::vector<int32_t> id(nh);
@@ -1715,18 +1727,18 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
 }
 
 tad_status solve_core(tad_fn fn, const double* H_dev, const double* rhs_dev, double* sol_dev,
-                      const tad_solve_opts& o, tad_solve_stats* st, const unsigned char* free_dev = nullptr,
-                      bool lagged = false)
+                      const tad_solve_opts& o, tad_solve_stats* st, const unsigned char* free_dev = nullptr)
 {
     if (o.max_iters <= 0) return fail(TAD_ERR_INVALID, "max_iters must be positive");
+    if (o.coarse_reuse) fn->keeps_coarse = true;
     if (o.coarse_aggregate < 0 && fn->n_blocks > 0 && fn->n_vars <= (fn->d == 3 ? kDenseVars3 : kDenseVars2))
     {
         bool again = false;
-        const tad_status r = solve_once(fn, H_dev, rhs_dev, sol_dev, o, st, free_dev, lagged, true, &again);
+        const tad_status r = solve_once(fn, H_dev, rhs_dev, sol_dev, o, st, free_dev, true, &again);
         if (!again) return r;
         fn->co.dense_valid = false;
     }
-    return solve_once(fn, H_dev, rhs_dev, sol_dev, o, st, free_dev, lagged, false, nullptr);
+    return solve_once(fn, H_dev, rhs_dev, sol_dev, o, st, free_dev, false, nullptr);
 }
 
 // Armijo backtracking on device data (LineSearch.hh:26-65).  The direction is
@@ -2818,9 +2830,12 @@ tad_status tad_newton_step(tad_fn fn, double* x, tad_mem mem, const tad_newton_o
     tad_solve_stats ss;
     std::memset(&ss, 0, sizeof(ss));
     tad_solve_opts sopt = o.solve;
-    if (o.coarse_refresh > 1 && fn->solves_since_rebuild + 1 < o.coarse_refresh) sopt.coarse_reuse = 1;
-    const tad_status solved =
-        solve_core(fn, fn->H_buf.p, fn->g_buf.p, fn->sol.p, sopt, &ss, nullptr, o.coarse_refresh > 1);
+    if (o.coarse_refresh > 1)
+    {
+        fn->keeps_coarse = true;
+        if (fn->solves_since_rebuild + 1 < o.coarse_refresh) sopt.coarse_reuse = 1;
+    }
+    const tad_status solved = solve_core(fn, fn->H_buf.p, fn->g_buf.p, fn->sol.p, sopt, &ss);
     if (solved != TAD_OK)
     {
         const std::string why = g_last_error;
