@@ -194,8 +194,11 @@ __global__ __launch_bounds__(kBlock) void k_ls_finish(LineSearchBatch a)
     int acc = -1;
     for (int c = 0; c < a.ncand && acc == -1; ++c)
     {
+        // products and sum rounded one by one, as the host computes them
+#pragma clang fp contract(off)
+        const double bound = a.f + a.armijo * a.sval[c] * dg;
         if (tot[c] != tot[c]) acc = -2;
-        else if (tot[c] <= a.f + a.armijo * a.sval[c] * dg) acc = c;
+        else if (tot[c] <= bound) acc = c;
     }
     a.step_out[0] = acc >= 0 ? a.step[acc] : 0.0;
     a.accepted_out[0] = acc;
