@@ -1590,11 +1590,11 @@ tad_status solve_once(tad_fn fn, const double* H_dev, const double* rhs_dev, dou
         {
             c.dense_valid = false;
             tm.begin("coarse_setup", s);
-            TAD_HIP(c.info.ensure(2));
             TAD_HIP(c.inv_work.ensure((size_t)spd_inverse_work(n)));
+            *dense_flag(fn) = 0;  // (the last solve's launches before this one have run)
             TAD_HIP(launch_dense_fill(d, sys, c.dense_inv.p, s));
             tm.begin("coarse_inverse", s);
-            TAD_HIP(launch_spd_inverse(n, c.dense_inv.p, c.inv_work.p, c.info.p, s, dense_flag(fn)));
+            TAD_HIP(launch_spd_inverse(n, c.dense_inv.p, c.inv_work.p, dense_flag(fn), s, true));
             tm.end("coarse_inverse", s);
             tm.end("coarse_setup", s);
         }

@@ -243,8 +243,8 @@ __device__ __forceinline__ bool tile_inverse(Tile& P, Tile& T)
 }
 
 // Q (column-major tile in memory) = P^-1 for the pivot block in LDS; info[0]
-// = 1 when a pivot is not positive and finite (first: 0 otherwise).
-__device__ __forceinline__ void pivot_to(Tile& P, Tile& T, double* __restrict__ Q, int* __restrict__ info, bool first)
+// = 1 when a pivot is not positive and finite (clear: 0 otherwise).
+__device__ __forceinline__ void pivot_to(Tile& P, Tile& T, double* __restrict__ Q, int* __restrict__ info, bool clear)
 {
     const bool bad = tile_inverse(P, T);  // known to wave 0
 #pragma unroll
@@ -253,7 +253,7 @@ __device__ __forceinline__ void pivot_to(Tile& P, Tile& T, double* __restrict__ 
         const int e = threadIdx.x + 256 * p;
         Q[e] = -P[e / kTile][e % kTile];
     }
-    if (threadIdx.x == 0 && (bad || first)) info[0] = bad ? 1 : 0;
+    if (threadIdx.x == 0 && (bad || clear)) info[0] = bad ? 1 : 0;
 }
 
 __host__ __device__ __forceinline__ int64_t tile_at(int64_t I, int64_t J)  // lower tile (I >= J)
@@ -265,7 +265,7 @@ __host__ __device__ __forceinline__ int64_t tile_at(int64_t I, int64_t J)  // lo
 // the first pivot block's inverse; one workgroup per tile (I = row of the
 // grid's triangle).
 __global__ __launch_bounds__(256) void k_sweep_load(int64_t n, const double* __restrict__ A, double* __restrict__ S,
-                                                    double* __restrict__ Q, int* __restrict__ info)
+                                                    double* __restrict__ Q, int* __restrict__ info, bool clear)
 {
     __shared__ Tile P, T;
     int64_t I = 0, J = blockIdx.x;
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(256) void k_sweep_load(int64_t n, const double* __r
     }
     if (blockIdx.x != 0) return;
     __syncthreads();
-    pivot_to(P, T, Q, info, true);
+    pivot_to(P, T, Q, info, clear);
 }
 
 // acc[c] (16 x 16 block: rows 16 w .. 16 w + 15, columns 16 c ..) = sum over
@@ -460,13 +460,10 @@ __global__ __launch_bounds__(256, 2) void k_sweep_step(int64_t nt, int64_t K, in
     }
 }
 
-// A = -S on the leading n x n part, both triangles (the sweeps leave -A^-1);
-// the finished flag to info_host (optional, pinned).
-__global__ __launch_bounds__(256) void k_sweep_store(int64_t n, const double* __restrict__ S, double* __restrict__ A,
-                                                     const int* __restrict__ info, int* __restrict__ info_host)
+// A = -S on the leading n x n part, both triangles (the sweeps leave -A^-1).
+__global__ __launch_bounds__(256) void k_sweep_store(int64_t n, const double* __restrict__ S, double* __restrict__ A)
 {
     __shared__ Tile P;
-    if (info_host && blockIdx.x == 0 && threadIdx.x == 0) *info_host = info[0];
     int64_t I = 0, J = blockIdx.x;
     while (J > I) J -= ++I;
     const double* __restrict__ in = S + tile_at(I, J);
@@ -500,7 +497,7 @@ int64_t spd_inverse_work(int64_t n)
     return 2 * (nt * (nt + 1) / 2) * kTT + 2 * kTT;
 }
 
-hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hipStream_t s, int* info_host)
+hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hipStream_t s, bool cleared)
 {
     if (n <= 0) return hipSuccess;
     const int64_t nt = (n + kTile - 1) / kTile;
@@ -513,11 +510,11 @@ hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hip
     const int64_t L = std::min<int64_t>(4, std::max<int64_t>(1, tiles / 512 + 1));
     int64_t strips = 0;
     for (int64_t J = 0; J < nt; ++J) strips += strips_of(nt, J, L);
-    k_sweep_load<<<(unsigned)tiles, 256, 0, s>>>(n, A, S[0], Q[0], info);
+    k_sweep_load<<<(unsigned)tiles, 256, 0, s>>>(n, A, S[0], Q[0], info, !cleared);
     for (int64_t K = 0; K < nt; ++K)
         k_sweep_step<<<(unsigned)(strips + (K + 1 < nt ? 1 : 0)), 256, 0, s>>>(nt, K, L, S[K & 1], Q[K & 1],
                                                                                S[(K + 1) & 1], Q[(K + 1) & 1], info);
-    k_sweep_store<<<(unsigned)tiles, 256, 0, s>>>(n, S[nt & 1], A, info, info_host);
+    k_sweep_store<<<(unsigned)tiles, 256, 0, s>>>(n, S[nt & 1], A);
     return hipGetLastError();
 }
 

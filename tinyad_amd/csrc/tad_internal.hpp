@@ -305,10 +305,10 @@ hipError_t launch_coarse_galerkin(int d, int kc, int64_t nc, int64_t n_pairs, in
 // by blocked Gauss-Jordan sweeps with FP64 MFMA products.  work:
 // spd_inverse_work(n) doubles; info[0] = 1 when a pivot block is not
 // positive definite at working precision (A is then not to be used: garbage,
-// or the inverse of an indefinite matrix); info_host (optional, pinned): its
-// copy.
+// or the inverse of an indefinite matrix).  cleared: info[0] is 0 already (it
+// may be pinned memory then, which is written only to report such a block).
 int64_t spd_inverse_work(int64_t n);
-hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hipStream_t s, int* info_host = nullptr);
+hipError_t launch_spd_inverse(int64_t n, double* A, double* work, int* info, hipStream_t s, bool cleared = false);
 
 // A_jj <- A_jj (1 + rel), 1 where A_jj = 0 (column-major n x n).
 hipError_t launch_shift_diagonal(int64_t n, double* A, double rel, hipStream_t s);
