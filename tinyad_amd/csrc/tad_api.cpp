@@ -259,7 +259,7 @@ struct tad_fn_s
     // pattern (block rows = handles)
     bool pattern_ready = false;
     int64_t n_blocks = 0, nnz = 0;
-    DevBuf<int32_t> brow_ptr, bcol, block_row, diag_block, row_ptr, col_idx;
+    DevBuf<int32_t> brow_ptr, bcol, block_row, row_ptr, col_idx;
     // destination-sorted contribution slots: CSR block b owns Hessian slots
     // [hslot_ptr[b], hslot_ptr[b+1]), handle u gradient slots [gslot_ptr[u], ..)
     int64_t n_hslots = 0, n_gslots = 0;
@@ -398,7 +398,7 @@ tad_status check_fn(tad_fn fn)
 
 void free_pattern(tad_fn fn)
 {
-    fn->brow_ptr.release(); fn->bcol.release(); fn->block_row.release(); fn->diag_block.release();
+    fn->brow_ptr.release(); fn->bcol.release(); fn->block_row.release();
     fn->row_ptr.release(); fn->col_idx.release(); fn->hslot_ptr.release(); fn->gslot_ptr.release();
     fn->block_mirror.release(); fn->uslot_ptr.release(); fn->uplace.release();
     fn->tile_ptr.release(); fn->arun.release(); fn->alen.release(); fn->apos.release();
@@ -449,8 +449,8 @@ tad_status build_pattern(tad_fn fn)
                 }
     }
     // handles used by no element keep empty rows, as in the reference's
-    // triplet assembly; their diagonal block index is -1
-    std::vector<int32_t> brow_ptr(nh + 1, 0), bcol, diag(nh, -1);
+    // triplet assembly
+    std::vector<int32_t> brow_ptr(nh + 1, 0), bcol;
     bcol.reserve(adj.size() / 3 + nh);
     for (int64_t u = 0; u < nh; ++u)
     {
@@ -460,8 +460,6 @@ tad_status build_pattern(tad_fn fn)
         while (b != e && *b < 0) ++b;  // padding entries of dynamic-valence elements
         for (auto it = b; it != e; ++it) bcol.push_back(*it);
         brow_ptr[u + 1] = (int32_t)bcol.size();
-        for (int32_t k = brow_ptr[u]; k < brow_ptr[u + 1]; ++k)
-            if (bcol[k] == u) diag[u] = k - brow_ptr[u];
     }
     const int64_t nb = (int64_t)bcol.size();
     if ((double)nb * d * d >= 2147483647.0)
@@ -732,7 +730,6 @@ tad_status build_pattern(tad_fn fn)
     TAD_HIP(up(fn->brow_ptr, brow_ptr));
     TAD_HIP(up(fn->bcol, bcol));
     TAD_HIP(up(fn->block_row, block_row));
-    TAD_HIP(up(fn->diag_block, diag));
     TAD_HIP(up(fn->row_ptr, row_ptr));
     TAD_HIP(up(fn->col_idx, col_idx));
     TAD_HIP(up(fn->hslot_ptr, hptr));
@@ -1077,12 +1074,6 @@ double auto_coarse_unknowns(int d, int64_t nh, bool lagged)
 // Largest relative change of the coarse correction accepted from its FP32 copy.
 constexpr double kCoarse32Change = 0.1;
 
-// Per solve: coarse unknowns per aggregate, lever arms, A_c = P^T (w I + H) P,
-// its inverse (blocked Gauss-Jordan sweeps with FP64 MFMA, tad_dense.hip;
-// fixed-order sums, so the result is deterministic), symmetrized.
-// *use = false when the coarse space is off or A_c is not numerically
-// positive definite (block-Jacobi alone then).  With o.coarse_reuse the
-// inverse and lever arms of the previous compatible solve are kept (*reused).
 // Regions of the context's pinned buffer (256 doubles): 0 .. 1 energy and error
 // flag of an evaluation, 16 .. 23 step sizes, 32 .. 51 energies and products,
 // and these.
@@ -1091,6 +1082,12 @@ LineSearchHost* ls_host(tad_fn fn) { return reinterpret_cast<LineSearchHost*>(fn
 int* mode_host(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 96); }
 int* dense_flag(tad_fn fn) { return reinterpret_cast<int*>(fn->ctx->pinned + 97); }
 
+// Per solve: coarse unknowns per aggregate, lever arms, A_c = P^T (w I + H) P,
+// its inverse (blocked Gauss-Jordan sweeps with FP64 MFMA, tad_dense.hip;
+// fixed-order sums, so the result is deterministic), symmetrized.
+// *use = false when the coarse space is off or A_c is not numerically
+// positive definite (block-Jacobi alone then).  With o.coarse_reuse the
+// inverse and lever arms of the previous compatible solve are kept (*reused).
 tad_status setup_coarse(tad_fn fn, const double* H_dev, const tad_solve_opts& o, const unsigned char* free_dev,
                         PcgSystem* cd, const SolverOrder** order, bool* use, bool* reused)
 {
