@@ -254,6 +254,15 @@ __device__ __forceinline__ double refined_rcp(double x)
     return y;
 }
 
+// |x| < 2^K, from the exponent (false for NaN): its constant stands in the
+// instruction, where a double's would be held in registers through the
+// persistent kernels' loop.
+template <int K>
+__device__ __forceinline__ bool under(double x)
+{
+    return ((uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32) & 0x7fffffffu) < (uint32_t)(1023 + K) << 20;
+}
+
 // True when A - shift I is positive definite, from the pivots of its L D L^T
 // factorization (no square roots, one reciprocal per column).
 template <int n>
@@ -287,9 +296,10 @@ __device__ __forceinline__ bool ldl_pd(const double* A, double shift)
     return ok;
 }
 
-// Most eigenvalues project_few clamps (three bounds what an
-// isotropic energy of a tet has below zero: one per pair of singular values).
-constexpr int kMaxClamped = 3;
+// Eigenvectors project_few computes at most.  An isotropic energy of a tet has
+// up to three eigenvalues below zero, one per pair of singular values; four are
+// the smaller side of any level among the nine of a tet.
+constexpr int kMaxClamped = 4;
 // On the scaled tridiagonal (norm 1): the rounding of a root; the shift off
 // roots that cannot be told apart for their vectors; the residual at which a
 // vector is final, the largest accepted, and the passes it gets.
@@ -303,6 +313,10 @@ __device__ __forceinline__ double root_gap(int i)
 {
     return ldexp(1.0, i == 0 ? -7 : i == 1 ? -17 : i == 2 ? -27 : i == 3 ? -37 : i == 4 ? -43 : -47);
 }
+
+// A pivot, kept from zero by less than the rounding of a matrix of norm 1 (NaN
+// becomes a number).
+__device__ __forceinline__ double off_zero(double x) { return copysign(fmax(fabs(x), 0x1p-56), x); }
 
 // Number of eigenvalues of the tridiagonal (d, e2 = squared couplings) below
 // x (negative pivots of T - x I), and the logarithmic derivative of
@@ -324,7 +338,7 @@ __device__ __forceinline__ int tridiag_count(const double* d, const double* e2, 
             const int i = c == 0 ? s : n - 1 - s;
             if (c == 1 && i <= mid) continue;
             double q = (d[i] - x) - w[c];
-            q = fabs(q) < 1e-17 ? -1e-17 : q;
+            q = off_zero(q);
             const double r = refined_rcp(q);
             count += q < 0.0 ? 1 : 0;
             const double q2 = w[c] * (u[c] - 2.0 * t[c] * t[c]);
@@ -335,7 +349,7 @@ __device__ __forceinline__ int tridiag_count(const double* d, const double* e2, 
             w[c] = e2[c == 0 ? i : i - 1] * r;
         }
     double q = ((d[mid] - x) - w[0]) - w[1];
-    q = fabs(q) < 1e-17 ? -1e-17 : q;
+    q = off_zero(q);
     const double r = refined_rcp(q);
     count += q < 0.0 ? 1 : 0;
     const double q2 = w[0] * (u[0] - 2.0 * t[0] * t[0]) + w[1] * (u[1] - 2.0 * t[1] * t[1]);
@@ -357,7 +371,7 @@ __device__ __forceinline__ void tridiag_solve(const double* d, const double* e, 
     {
         const double x = e[i], an = d[i + 1] - shift, bn = i + 2 < n ? e[i + 1] : 0.0;
         const double w = a * a + x * x;
-        const bool zero = !(w > 1e-60);
+        const bool zero = under<-200>(w);
         const double ih = ql_rsqrt(zero ? 1.0 : w);
         const double c = zero ? 1.0 : a * ih, s = zero ? 0.0 : x * ih;
         r0[i] = zero ? 1e30 : ih;
@@ -369,7 +383,7 @@ __device__ __forceinline__ void tridiag_solve(const double* d, const double* e, 
         y[i + 1] = c * y[i + 1] - s * y[i];
         y[i] = t;
     }
-    r0[n - 1] = refined_rcp(fabs(a) < 1e-30 ? 1e-30 : a);
+    r0[n - 1] = refined_rcp(under<-100>(a) ? 1e-30 : a);
 #pragma unroll
     for (int i = n - 1; i >= 0; --i)
     {
@@ -403,17 +417,21 @@ __device__ __forceinline__ void normalize(double* v)
 __host__ __device__ constexpr int reflector_at(int n, int k) { return k * (n - 1) - k * (k - 1) / 2; }
 __host__ __device__ constexpr int reflector_values(int n) { return reflector_at(n, n - 2); }
 
-// Projects packed symmetric A in place when few eigenvalues are clamped:
+// Projects packed symmetric A in place from the eigenvectors on the smaller
+// side of the clamp level only:
 //   P(A) = A + sum_j (clamped_j - lam_j) v_j v_j^T
-// over the eigenvalues below the clamp level only, so no other eigenvector
-// and no full spectrum is computed.  Returns false, with A restored up to
-// rounding, when more than kMaxClamped eigenvalues are clamped or a vector
-// misses its residual; the caller then projects A by the full eigensolve.
+// over the eigenvalues below it or, if more than kMaxClamped are,
+//   P(A) = eps I + sum_j (lam_j - eps) v_j v_j^T    (absolute values:
+//   P(A) = -A + sum_j 2 lam_j v_j v_j^T)
+// over those above it, computed as the ones below it of -A.  Returns false,
+// with A restored up to rounding, when a vector misses its residual; the
+// caller then projects A by the full eigensolve.
 //   1. Householder reduction to the tridiagonal T, scaled by a power of two
 //      to norm 1, the reflectors going to `store` (in registers they do not
-//      fit beside the rest); the number m of clamped eigenvalues from the
-//      pivot signs.  Roots within rounding of the level are not clamped
-//      (they would move by rounding).
+//      fit beside the rest); the number m of eigenvalues below the level from
+//      the pivot signs (T and the level negated if those are the most).  Roots
+//      within rounding of the level are not clamped (they would move by
+//      rounding).
 //   2. Their values from right to left by Laguerre's iteration (cubic, and
 //      monotone towards the neighbouring root as all roots are real), each
 //      started next to the previous root, which is divided out.  k roots that
@@ -426,22 +444,27 @@ __host__ __device__ constexpr int reflector_values(int n) { return reflector_at(
 //      orthonormal vectors with such residuals and m Rayleigh quotients below
 //      the level are all there is below it, however close the roots are:
 //      which vectors of close roots they are does not matter to P(A).
-//   4. T + sum c w w^T, then the reflectors from both sides.
-// On the CPU, 6,000 element matrices (10^3 cube) per state, eps 1e-9, 0 and
-// absolute values, against 80-bit arithmetic, relative to |A|: at rest, noise
+//   4. T (or eps I, or -T) + sum c w w^T, then the reflectors from both sides.
+// On the CPU, 6,000 element matrices (10^3 cube) per state, eps 1e-9, 0.05, 0
+// and absolute values, against 80-bit arithmetic, relative to |A|: at rest, noise
 // of 1e-12 .. 0.1 mesh widths, smooth displacements, compressed and flattened
 // by 1e-9 .. 0.2, twisted by 0.01 .. 60 degrees 4.1e-15 at most (full
-// eigensolve 4.2e-15), at most 0.13 % of the elements given to the full
-// eigensolve.  Noise of 1e-13 and 1e-14 mesh widths, whose roots are hardly
-// above rounding: 0.3 %, and 3 and 23 % for eps <= 0, where the level lies
-// among them; error 1.5e-14 at most.  8 to 17 evaluations of step 2 per wave,
-// where the full QL iteration takes 27 sweeps.  Evaluation of 1,296,000 tets:
-// twisted by 30 and 54 degrees 0.85 and 0.84 ms, at rest 0.77, noise of 1e-9
-// and 1e-4 0.89 and 0.83, compressed by 1e-4 0.79 (with the full eigensolve,
-// and a tail of its own launches, 1.36, 1.35, 1.18, 1.14, 1.25, 1.12).
+// eigensolve 4.2e-15), at most 0.18 % of the elements given to the full
+// eigensolve (0.5 % for levels in the middle of the spectrum).  Noise of 1e-13
+// and 1e-14 mesh widths, whose roots are hardly above rounding: 0.4 %, and 3
+// and 23 % for eps <= 0, where the level lies among them; error 1.5e-14 at most.
+// 7 to 18 evaluations of step 2 per wave at eps 1e-9, where the full QL
+// iteration takes 27 sweeps, 31 with the level among the eigenvalues.
+// Evaluation of 1,296,000 tets: twisted by 30 and 54 degrees 0.82 and 0.81 ms,
+// at rest 0.74, noise of 1e-9 and 1e-4 mesh widths 0.88 and 0.81, compressed by
+// 1e-4 0.77 (with the full eigensolve, and a tail of its own launches, 1.35,
+// 1.36, 1.20, 1.16, 1.26, 1.15); eps 1e-4 .. 1e-2 0.79 .. 0.90, eps above every
+// eigenvalue 0.63 (full 1.19 .. 1.38; where only the side below the level is
+// computed and the rest left to the full eigensolve here, 6.7 .. 8.1).
 template <int n>
 __device__ __forceinline__ bool project_few(double* A, double eps, double* store)
 {
+    static_assert(n <= 2 * kMaxClamped + 1, "one side of the level has at most kMaxClamped eigenvalues");
     double amax = 0.0;
 #pragma unroll
     for (int q = 0; q < Sym<n>::n; ++q) amax = fmax(amax, fabs(A[q]));
@@ -495,6 +518,10 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
         d[i] = A[Sym<n>::idx(i, i)];
         norm = fmax(norm, fabs(d[i]) + fabs(e[i]) + (i > 0 ? fabs(e[i - 1]) : 0.0));
     }
+    double nan_sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < n; ++i) nan_sum += (d[i] + e[i]) * 0.0;
+    if (!(nan_sum == 0.0)) return false;
     int ex = 0;
     (void)frexp(norm, &ex);
     bool ok = true;
@@ -506,41 +533,69 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
         e[i] = ldexp(e[i], -ex);
         e2[i] = e[i] * e[i];
     }
-    const double level = ldexp(eps > 0.0 ? eps : 0.0, -ex);
+    double level = ldexp(eps > 0.0 ? eps : 0.0, -ex);
     // 2. roots r[0] >= r[1] >= ... below `start`
     double r[kMaxClamped] = {};
     double start = level - kRootRounding;
     int m = 0, found = 0;
+    bool flip = false;  // more eigenvalues clamped than not: the others, of -T
     {
-        double x = start, from = start;  // from: the last root (or the level)
-        int gap = -1;                    // >= 0: x lies root_gap(gap) below `from`
-        bool first = true, run = true;
+        double x = start, g, h;
+        int below = tridiag_count<n>(d, e2, x, g, h);
+        h = -h;
+        if (below > kMaxClamped)
+        {
+            flip = true;
+            below = n - below;
+            g = -g;
+            level = -level;
+            start = x = -start;
+#pragma unroll
+            for (int i = 0; i < n; ++i)
+            {
+                d[i] = -d[i];
+                e[i] = -e[i];
+            }
+        }
+        double from = x;  // the last root (or the level)
+        int gap = -1;     // >= 0: x lies root_gap(gap) below `from`
+        bool fresh = true, known = true;  // m to be taken from `below`; evaluated at x already
+        bool run = below > 0;
 #pragma unroll 1
         for (int it = 0; run && it < 64; ++it)
         {
-            double g, h;
-            const int below = tridiag_count<n>(d, e2, x, g, h);
-            h = -h;
-            if (first)
+            if (!known)
             {
+                below = tridiag_count<n>(d, e2, x, g, h);
+                h = -h;
+            }
+            known = false;
+            bool away = false;
+            if (fresh)
+            {
+                fresh = false;
                 m = below;
-                if (m == 0 || m > kMaxClamped) break;
+                run = m > 0;
+                // roots right above the level: set out away from them
+                away = g < 0.0 && !under<10>(g);
+                if (away)
+                {
+                    gap = 0;
+                    x = from - root_gap(0);
+                }
             }
             const int inside = m - found - below;  // roots not found yet that are not below x
             int take = 0;
             double root = from;
             if (gap >= 0 && inside > 0)
             {
-                // between the last root and x
-                if (gap + 1 < kRootGaps)
-                {
-                    x = from - root_gap(++gap);
-                    continue;
-                }
-                take = inside;  // cannot be told apart from it
+                // between the last root and x: closer to it, or not to be told apart from it
+                if (gap + 1 < kRootGaps) x = from - root_gap(++gap);
+                else take = inside;
             }
-            else
+            else if (!away)
             {
+                gap = -1;
 #pragma unroll
                 for (int j = 0; j + 1 < kMaxClamped; ++j)
                     if (j < found)
@@ -549,87 +604,77 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
                         g -= q;
                         h -= q * q;
                     }
-                if (first && g < -1e3)
-                {
-                    // roots right above the level: set out away from them
-                    first = false;
-                    gap = 0;
-                    x = from - root_gap(gap);
-                    continue;
-                }
                 const double deg = (double)(n - found), gg = g * g;
                 const double spread = deg * h - gg;  // 0 for one deg-fold root
                 const double disc = (deg - 1.0) * spread;
                 const double sq = disc > 0.0 ? disc * ql_rsqrt(disc) : 0.0;
                 // k equal roots have g = k / (x - root), h = k / (x - root)^2
                 // (g < 0: the near ones lie above x)
-                int fold = 1;
-                double dev = fabs(gg - h);
-#pragma unroll
-                for (int k = 2; k <= kMaxClamped; ++k)
-                    if (k <= m - found && fabs(gg - k * h) < dev)
-                    {
-                        dev = fabs(gg - k * h);
-                        fold = k;
-                    }
+                const double like = gg * __builtin_amdgcn_rcp(h);
+                const double fold = fmin(fmax(rint(like), 1.0), (double)(m - found));
+                const double dev = fabs(like - fold);
                 const bool past = inside > 0;  // x is below the next root: towards it
-                const bool alike = (past ? g < 0.0 : g > 0.0) && dev < 0.01 * gg;
+                const bool alike = (past ? g < 0.0 : g > 0.0) && dev < 0.01 * fold;
                 double step = deg * refined_rcp(past ? g - sq : g + sq);
-                if (alike && fold == 1)
-                    take = fabs(step) * dev * dev < 1e-16 * gg * gg ? 1 : 0;  // (the error: step (dev / gg)^2)
+                // (the wrong way: rounding of the roots divided out)
+                const bool lost = !(past ? step < 0.0 : step > 0.0);
+                if (lost) step = past ? 0.5 * (x - from) : fmax(from - x, root_gap(1));
+                else if (alike && fold == 1.0)
+                    take = under<-53>(step * dev * dev) ? 1 : 0;  // (the error of root: about step dev^2)
                 else if (alike)
                 {
-                    const double f = (deg - fold) / fold * spread;
+                    const double f = (deg * refined_rcp(fold) - 1.0) * spread;
                     const double sf = f > 0.0 ? f * ql_rsqrt(f) : 0.0;
                     step = deg * refined_rcp(past ? g - sf : g + sf);
-                    take = fabs(step) < 1e-13 ? fold : 0;
+                    take = under<-43>(step) ? (int)fold : 0;
                 }
-                if (fabs(step) < 4e-16 && (past || g > 0.0)) take = max(take, 1);
+                if (!lost && under<-51>(step) && (past || g > 0.0)) take = max(take, 1);
                 root = x - step;
                 if (inside > 1)
                 {
                     // beyond all but one of them, or they share a value
-                    take = fabs(step) < 1e-14 ? inside : 0;
+                    take = under<-47>(step) ? inside : 0;
                     step *= 2.0;
                 }
-                else if (take == 0 && alike && fold > 1)
+                else if (take == 0 && alike && fold > 1.0)
                 {
-                    // short of the first of them (their spread is about 2 sqrt(dev / gg) of the distance)
-                    const double q = fmax(dev * refined_rcp(gg), 1e-12);
+                    // short of the first of them (their spread is about 2 sqrt(dev / k) of the distance)
+                    const double q = fmax(dev, 1e-12);
                     step *= 1.0 - 2.0 * q * ql_rsqrt(q);
                 }
-                if (take == 0) x -= step;
+                x -= step;
             }
-            first = false;
-            gap = -1;
-            if (take == 0) continue;
-            if (found == 0 && !(root < start - 2.0 * kRootRounding))
+            if (take > 0)
             {
-                // at the level up to rounding: those below it are clamped
-                if (!(root > level - 4.0 * kRootRounding)) break;
-                start = x = from = root - 2.0 * kRootRounding;
-                first = true;
-                continue;
-            }
+                gap = 1;
+                from = root;
+                if (found == 0 && !(root < start - 2.0 * kRootRounding))
+                {
+                    // at the level up to rounding: those below it are clamped
+                    run = root > level - 4.0 * kRootRounding;
+                    start = from = root - 2.0 * kRootRounding;
+                    fresh = true;
+                    gap = -1;
+                    x = from;
+                }
+                else
+                {
 #pragma unroll
-            for (int j = 0; j < kMaxClamped; ++j)
-                if (j >= found && j < found + take) r[j] = root;
-            found += take;
-            run = found < m;
-            from = root;
-            gap = 1;
-            x = from - root_gap(gap);
+                    for (int j = 0; j < kMaxClamped; ++j)
+                        if (j >= found && j < found + take) r[j] = root;
+                    found += take;
+                    run = found < m;
+                    x = from - root_gap(1);
+                }
+            }
         }
     }
-    ok = ok && m <= kMaxClamped && found == m;
+    ok = ok && found == m;
     // 3.
     double W[kMaxClamped][n], c[kMaxClamped];
 #pragma unroll
     for (int j = 0; j < kMaxClamped; ++j)
     {
-        c[j] = 0.0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) W[j][i] = 0.0;
         if (ok && j < m)
         {
             double lam = r[j], z[n];
@@ -646,8 +691,8 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
                 for (int i = 0; i + 1 < n; ++i)
                 {
                     const int b = n - 1 - i;
-                    dp[i] = fabs(dp[i]) < 1e-100 ? -1e-100 : dp[i];
-                    dm[b] = fabs(dm[b]) < 1e-100 ? -1e-100 : dm[b];
+                    dp[i] = off_zero(dp[i]);
+                    dm[b] = off_zero(dm[b]);
                     l[i] = e[i] * refined_rcp(dp[i]);
                     u[b - 1] = e[b - 1] * refined_rcp(dm[b]);
                     dp[i + 1] = (d[i + 1] - lam) - e[i] * l[i];
@@ -740,15 +785,29 @@ __device__ __forceinline__ bool project_few(double* A, double eps, double* store
     // 4. (the reflectors are read, not kept: the compiler does not look past this)
     asm volatile("" ::: "memory");
     double P[Sym<n>::n];
+    {
+        const bool all = ok && flip && !(eps < 0.0);  // all at the level but for the others' vectors
+        const double sign = flip && !ok ? -1.0 : 1.0;   // (A as it was)
 #pragma unroll
-    for (int i = 0; i < n; ++i)
+        for (int i = 0; i < n; ++i)
 #pragma unroll
-        for (int j = i; j < n; ++j)
+            for (int j = i; j < n; ++j)
+                P[Sym<n>::idx(i, j)] = i == j       ? ldexp(all ? -level : sign * d[i], ex)
+                                       : j == i + 1 ? ldexp(all ? 0.0 : sign * e[i], ex)
+                                                    : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < kMaxClamped; ++q)
+        if (ok && q < m)
         {
-            double s = i == j ? d[i] : (j == i + 1 ? e[i] : 0.0);
+            const double cq = ldexp(c[q], ex);
 #pragma unroll
-            for (int q = 0; q < kMaxClamped; ++q) s += ok ? c[q] * W[q][i] * W[q][j] : 0.0;
-            P[Sym<n>::idx(i, j)] = ldexp(s, ex);
+            for (int i = 0; i < n; ++i)
+            {
+                const double ci = cq * W[q][i];
+#pragma unroll
+                for (int j = i; j < n; ++j) P[Sym<n>::idx(i, j)] += ci * W[q][j];
+            }
         }
 #pragma unroll
     for (int k = n - 3; k >= 0; --k)

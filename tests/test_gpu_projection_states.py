@@ -34,3 +34,29 @@ def test_tets_near_rest(ctx, state):
             fg.set_launch_shape(0, *shape)
             H = fg.eval_with_hessian_proj(x, eps)[2].toarray()
             assert np.abs(H - ref).max() <= 4e-13 * np.abs(ref).max(), (eps, shape)
+
+
+@pytest.mark.parametrize("eps", [0.02, 0.1, 0.3, 1.0, 30.0])
+@pytest.mark.parametrize("state", ["rest", "noise", "twisted"])
+def test_levels_that_clamp_most_eigenvalues(ctx, state, eps):
+    """Four to all nine of an element's eigenvalues below the level (they are
+    0.1 .. 3 here), against the oracle; the error bound of test_tets_near_rest,
+    relative to the level where that is larger."""
+    import oracle
+    P = configs.twist_cube(m=3)
+    rest = P.info["rest"].reshape(-1, 3)
+    x = rest.copy()
+    if state == "noise":
+        x = x + 0.02 * P.info["h"] * np.random.default_rng(3).standard_normal(rest.shape)
+    elif state == "twisted":
+        th = np.radians(50.0) * rest[:, 2]
+        px, py = rest[:, 0] - 0.5, rest[:, 1] - 0.5
+        x = np.stack([0.5 + np.cos(th) * px - np.sin(th) * py, 0.5 + np.sin(th) * px + np.cos(th) * py, rest[:, 2]], axis=1)
+    x = np.ascontiguousarray(x).reshape(-1)
+    fg = tad.ScalarFunction.from_problem(P, ctx)
+    fo = oracle.Function.from_problem(P)
+    ref = fo.eval_with_hessian_proj(x, eps)[2].toarray()
+    for shape in [(0, 0, 0), (256, 1, 0)]:
+        fg.set_launch_shape(0, *shape)
+        H = fg.eval_with_hessian_proj(x, eps)[2].toarray()
+        assert np.abs(H - ref).max() <= 4e-13 * max(np.abs(ref).max(), eps), shape

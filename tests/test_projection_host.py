@@ -22,7 +22,7 @@ STUB = """
 #define __device__
 #define __host__
 #define __forceinline__ inline
-using std::max; using std::fabs; using std::fma; using std::fmax; using std::frexp; using std::ldexp; using std::sqrt;
+using std::max; using std::copysign; using std::fabs; using std::fma; using std::fmax; using std::frexp; using std::ldexp; using std::rint; using std::sqrt;
 // (single precision accuracy, as the hardware's approximations have)
 inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x * (1 + 3e-8); }
 inline double __builtin_amdgcn_rsq(double x) { return 1.0 / std::sqrt(x) * (1 + 3e-8); }
@@ -85,7 +85,7 @@ def check(project, K, eps, fallback):
     and counts up to three times (once per clamped vector), twice for absolute
     values: 4e-15 + 7.2e-14 < 1e-13 (the largest entry for |A|)."""
     P, status = project(K, eps)
-    scale = np.abs(K).max(axis=(1, 2))
+    scale = np.maximum(np.abs(K).max(axis=(1, 2)), eps)
     few = status == 1
     err = np.abs(P - reference(K, eps)).max(axis=(1, 2)) / scale
     assert err[few].max(initial=0.0) <= 1e-13, eps
@@ -162,3 +162,26 @@ def test_close_roots(project, base, near, spread):
     K = 0.5 * (K + K.transpose(0, 2, 1))
     for eps in (1e-9, 0.0, -1.0):
         check(project, K, eps, 0.05 if base < 0.0 else 1.0)
+
+
+@pytest.mark.parametrize("state", [("noise", 0.0), ("noise", 1e-6), ("noise", 1e-2), ("compressed", 0.1), ("twisted", 54.0)],
+                         ids=lambda s: f"{s[0]}_{s[1]:g}")
+@pytest.mark.parametrize("eps", [0.02, 0.1, 0.2, 0.3, 0.5, 0.8, 5.0, 1e6])
+def test_large_clamp_levels(project, state, eps):
+    """Levels among and above the eigenvalues (0.1 .. 1 here): four to all nine
+    of them are clamped; still at most 1 % go to the full eigensolve."""
+    rest, h, conn, params = tets()
+    check(project, element_matrices(moved(rest, h, state), conn, params), eps, 0.01)
+
+
+def test_absolute_values_of_mostly_negative_matrices(project):
+    """Any number of negative eigenvalues, with and without close ones."""
+    rng = np.random.default_rng(4)
+    for negative in range(10):
+        Q = np.linalg.qr(rng.standard_normal((200, 9, 9)))[0]
+        lam = 0.05 + np.abs(rng.standard_normal((200, 9)))
+        lam[:, :negative] *= -1.0
+        lam[:100, 1] = lam[:100, 0] * (1.0 + 1e-9)
+        K = np.einsum("nik,nk,njk->nij", Q, lam, Q)
+        for eps in (-1.0, 0.0, 1e-9):
+            check(project, 0.5 * (K + K.transpose(0, 2, 1)), eps, 0.01)

@@ -230,8 +230,8 @@ extern __shared__ double tad_group_lds[];
 // issue slots; with the clamped eigenvalues only 9,500 and 0.97 ms, 46 % of
 // the wave's cycles waiting for memory, mostly for one slot or code at a time;
 // with both fetched together 0.84 ms; with no wave left that takes the full
-// eigensolve as well (close eigenvalues) 10,300 and 0.80 ms, 56 % of the issue
-// slots, 35 % waiting.  (FP32, 45^3 cube: 0.34 -> 0.31 ms; triangles of 256
+// eigensolve as well (close eigenvalues) 9,700 and 0.79 ms, 59 % of the issue
+// slots, 36 % waiting.  (FP32, 45^3 cube: 0.34 -> 0.31 ms; triangles of 256
 // disks: 0.55 -> 0.48 ms.)
 template <class T>
 struct GroupWaves
